@@ -356,7 +356,11 @@ void context_free(sbg_context ctx)
     ctx->workCounts.release();
     ctx->ccKeys.release();
     ctx->ccOwners.release();
+    ctx->ccValence.release();
+    ctx->ccMate.release();
     ctx->ccParent.release();
+    ctx->ccList.release();
+    ctx->ccListAlt.release();
     ctx->ccLabels.release();
     ctx->ccBlocked.release();
     ctx->rawA.release();
@@ -847,20 +851,24 @@ int sbg_components(sbg_mesh m, const uint8_t *blocked, uint32_t *labels)
     const size_t nt = m->nt;
     if (!nt)
         return SBG_OK;
-    const size_t slots = component_table_slots((uint32_t)nt);
-    TRY(c->ccKeys.ensure(slots));
-    TRY(c->ccOwners.ensure(slots + 1));
+    if (nt > 0x55555555u)  // half-edges are counted in 32 bits
+        return fail(SBG_ERR_INVALID, "too many triangles");
+    TRY(c->ccList.ensure(3 * nt));
+    TRY(c->ccListAlt.ensure(3 * nt));
+    TRY(c->hist.ensure(sort_hist_entries(3 * nt)));
+    TRY(c->ccValence.ensure(m->nv + 2));
+    TRY(c->ccMate.ensure(3 * nt));
     TRY(c->ccParent.ensure(nt));
     TRY(c->ccLabels.ensure(nt));
     if (blocked) {
         TRY(c->ccBlocked.ensure(nt));
         HIP_TRY(hipMemcpyAsync(c->ccBlocked.p, blocked, nt, hipMemcpyHostToDevice, c->stream));
     }
-    launch_components(m->T.p, (uint32_t)nt, blocked ? c->ccBlocked.p : nullptr, c->ccKeys.p, c->ccOwners.p,
-                      c->ccParent.p, c->ccLabels.p, c->stream);
+    launch_components(m->T.p, (uint32_t)nt, m->nv, blocked ? c->ccBlocked.p : nullptr, c->ccList.p, c->ccListAlt.p,
+                      c->hist.p, c->ccValence.p, c->ccMate.p, c->ccParent.p, c->ccLabels.p, c->stream);
     TRY(check_launch("components"));
     uint32_t *repeated = c->pinned + kComponentsPinned;
-    HIP_TRY(hipMemcpyAsync(repeated, c->ccOwners.p + slots, sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
+    HIP_TRY(hipMemcpyAsync(repeated, c->ccValence.p + m->nv + 1, sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipMemcpyAsync(labels, c->ccLabels.p, sizeof(uint32_t) * nt, hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
     if (*repeated)
@@ -881,7 +889,7 @@ int sbg_half_edges(sbg_context c, const uint32_t *tris, size_t ntris, const uint
             return fail(SBG_ERR_INVALID, "vertex index 0xffffffff");
     const size_t slots = component_table_slots((uint32_t)ntris);
     TRY(c->ccKeys.ensure(slots));
-    TRY(c->ccOwners.ensure(slots + 1));
+    TRY(c->ccOwners.ensure(slots));
     TRY(c->heTris.ensure(3 * ntris));
     TRY(c->heOpposite.ensure(3 * ntris));
     TRY(c->heQueries.ensure(nqueries));

@@ -149,8 +149,10 @@ struct sbg_context_s {
     DevBuf<uint32_t> ovf, rayList, ovf2, rayList2;
     PinnedBuf votesHost, votesHost2;  // vote readbacks of the two sets
     DevBuf<unsigned long long> workCounts;  // sbg_bench_rays
-    DevBuf<unsigned long long> ccKeys;      // sbg_components: half-edge table
-    DevBuf<uint32_t> ccOwners, ccParent, ccLabels;
+    DevBuf<unsigned long long> ccKeys;      // sbg_half_edges: half-edge table
+    DevBuf<uint32_t> ccOwners;
+    DevBuf<uint64_t> ccList, ccListAlt;     // sbg_components: half-edges listed by hash
+    DevBuf<uint32_t> ccValence, ccMate, ccParent, ccLabels;
     DevBuf<uint8_t> ccBlocked;
     DevBuf<uint32_t> heTris, heOpposite, heQueryOwner, heRepeat;  // sbg_half_edges
     DevBuf<unsigned long long> heQueries;

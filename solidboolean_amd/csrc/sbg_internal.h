@@ -204,8 +204,9 @@ void launch_vote(const uint8_t *axisBits, const uint8_t *skip, uint32_t n, uint8
 
 // k_components.hip: triangle components across opposite half-edges
 size_t component_table_slots(uint32_t nt);
-void launch_components(const uint32_t *T, uint32_t nt, const uint8_t *blocked, unsigned long long *keys,
-                       uint32_t *owners, uint32_t *parent, uint32_t *labels, hipStream_t s);
+void launch_components(const uint32_t *T, uint32_t nt, size_t nv, const uint8_t *blocked, uint64_t *list,
+                       uint64_t *listAlt, uint32_t *hist, uint32_t *valence, uint32_t *mate, uint32_t *parent,
+                       uint32_t *labels, hipStream_t s);
 void launch_half_edges(const uint32_t *T, uint32_t nt, const unsigned long long *queries, uint32_t nq,
                        unsigned long long *keys, uint32_t *owners, uint32_t *opposite, uint32_t *queryOwner,
                        uint32_t *firstRepeat, hipStream_t s);

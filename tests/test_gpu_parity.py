@@ -654,6 +654,50 @@ def test_components_vs_oracle(gpu):
     assert np.all(G.components() == 0)
 
 
+@pytest.mark.parametrize("nu,nv,order", [(32, 16, "ring"), (31, 16, "ring"), (33, 31, "ring"), (64, 40, "ring"),
+                                         (64, 40, "shuffled"), (33, 31, "blocks")])
+def test_components_across_tiles(gpu, nu, nv, order):
+    """sbg_components where its tiles of 1,024 triangles end: lists of just
+    under, exactly and over whole tiles, edges across tiles in ring order, in
+    shuffled order (hardly an edge inside a tile) and in interleaved blocks,
+    with and without blocked triangles."""
+    from oracle.oracle import face_groups
+
+    m = mg.torus(1.0, 0.3, nu, nv)
+    rng = np.random.default_rng(nu * nv)
+    perm = {"ring": np.arange(m.nt), "shuffled": rng.permutation(m.nt),
+            "blocks": np.concatenate([np.arange(k, m.nt, 3) for k in range(3)])}[order]
+    tris = m.triangles[perm]
+    G = gpu.mesh(m.vertices, tris, prepare=False)
+    for share in (None, 0.02, 0.4, 1.0):
+        blocked = None if share is None else rng.random(m.nt) < share
+        got = G.components(None if blocked is None else blocked.astype(np.uint8)).astype(np.int64)
+        got[got == 0xFFFFFFFF] = -1
+        assert np.array_equal(got, face_groups(tris, blocked))
+
+
+@pytest.mark.parametrize("copies", [[("same", 2000)], [("same", 3)], [("other", 2000), ("same", 2001)],
+                                    [("other", 2100), ("same", 2500)]])
+def test_components_repeats_across_tiles(gpu, copies):
+    """A directed edge held twice is refused wherever its triangles lie: twice
+    in one tile, in two tiles, and a second pair of opposite half-edges on an
+    edge that a tile had paired already (also pairwise in two other tiles);
+    blocking the extra triangles leaves the mesh's own groups."""
+    m = mg.torus(1.0, 0.3, 64, 40)
+    i, j = m.triangles[0][:2]
+    verts = np.concatenate([m.vertices, np.zeros((len(copies), 3))])
+    tris = m.triangles
+    for k, (way, at) in enumerate(copies):
+        extra = [i, j, m.nv + k] if way == "same" else [j, i, m.nv + k]
+        tris = np.insert(tris, at, extra, axis=0)
+    G = gpu.mesh(verts, tris, prepare=False)
+    with pytest.raises(N.SbgError, match="repeated half-edge"):
+        G.components()
+    blocked = (tris >= m.nv).any(1)
+    got = G.components(blocked.astype(np.uint8))
+    assert np.all(got[~blocked] == 0) and np.all(got[blocked] == 0xFFFFFFFF)
+
+
 def test_half_edges_vs_dict(gpu):
     """sbg_half_edges against a dictionary half-edge map built in index order
     (the reference's unordered_map keyed (from << 32) | to, first insert
