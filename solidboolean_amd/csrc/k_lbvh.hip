@@ -7,8 +7,8 @@
 //
 // Node i (0 <= i < n-1) is internal; node 0 is the root.  Leaves are referenced
 // as kLeafBit | triangle, so traversal never needs a leaf -> triangle lookup.
-// The refit stores each child's FP32 box inside its parent, so one 64-B node
-// load yields both child boxes.
+// Each child's FP32 box is stored inside its parent, so one 64-B node load
+// yields both child boxes.
 #include "sbg_internal.h"
 
 namespace sbg {
@@ -35,95 +35,11 @@ __device__ __forceinline__ int delta(const uint64_t *__restrict__ codes, int n, 
     return __clzll(a ^ b);
 }
 
-// Leaves are refit in tiles of kRefitTile sorted positions; a node whose leaf
-// range crosses a tile boundary is a "top" node, finished by k_refit_top.
-constexpr int kRefitTile = 1024;  // leaves per workgroup, one per lane
-
-// Scratch shared by the hierarchy and the refit (2n + 1 u32): the top-node
-// count, then per sorted leaf position two bytes saying whether a top node's
-// range starts there (its suffix union is needed) or ends there (its prefix
-// union is needed), then the top-node list.  Only the first two parts start
-// at zero.
-struct TopWork {
-    uint32_t *count;
-    uint8_t *need;  // [2 pos]: a range starts at pos, [2 pos + 1]: one ends at pos
-    uint32_t *list;
-};
-__host__ __device__ inline TopWork top_work(uint32_t *work, uint32_t n)
-{
-    return {work, reinterpret_cast<uint8_t *>(work + 1), work + n};
-}
-__host__ __device__ inline size_t top_work_zeroed(uint32_t n) { return 1 + ((size_t)n + 1) / 2; }
-
-template <typename K>
-__global__ __launch_bounds__(256) void k_hierarchy(const K *__restrict__ codes,
-                                                   const uint32_t *__restrict__ ids, int n,
-                                                   BNode *__restrict__ nodes, uint32_t *__restrict__ leafParent,
-                                                   TopWork top)
-{
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= n - 1)
-        return;
-    const int d = (delta(codes, n, i, i + 1) - delta(codes, n, i, i - 1)) >= 0 ? 1 : -1;
-    const int dmin = delta(codes, n, i, i - d);
-    int lmax = 2;
-    while (delta(codes, n, i, i + lmax * d) > dmin)
-        lmax <<= 1;
-    int l = 0;
-    for (int t = lmax >> 1; t >= 1; t >>= 1)
-        if (delta(codes, n, i, i + (l + t) * d) > dmin)
-            l += t;
-    const int j = i + l * d;
-    const int dnode = delta(codes, n, i, j);
-    int s = 0;
-    int t = l;
-    do {
-        t = (t + 1) >> 1;
-        if (delta(codes, n, i, i + (s + t) * d) > dnode)
-            s += t;
-    } while (t > 1);
-    const int gamma = i + s * d + (d < 0 ? d : 0);
-    const int lo = i < j ? i : j;
-    const int hi = i < j ? j : i;
-    int c0, c1;
-    if (lo == gamma) {
-        c0 = (int)(kLeafBit | ids[gamma]);
-        leafParent[gamma] = (uint32_t)i;
-    } else {
-        c0 = gamma;
-        nodes[gamma].d.z = i;
-    }
-    if (hi == gamma + 1) {
-        c1 = (int)(kLeafBit | ids[gamma + 1]);
-        leafParent[gamma + 1] = (uint32_t)i;
-    } else {
-        c1 = gamma + 1;
-        nodes[gamma + 1].d.z = i;
-    }
-    nodes[i].d.x = c0;
-    nodes[i].d.y = c1;
-    nodes[i].d.w = j;  // the node covers sorted leaves [min(i, j), max(i, j)]
-    if (i == 0)
-        nodes[0].d.z = -1;
-    if (lo / kRefitTile != hi / kRefitTile) {
-        top.list[atomicAdd(top.count, 1u)] = (uint32_t)i;
-        top.need[2 * (size_t)lo] = 1;
-        top.need[2 * (size_t)hi + 1] = 1;
-    }
-}
-
-__device__ __forceinline__ void store_child_box(BNode *nd, int slot, float4 lo, float4 hi)
-{
-    if (slot == 0) {
-        nd->a = make_float4(lo.x, lo.y, lo.z, hi.x);
-        nd->b.x = hi.y;
-        nd->b.y = hi.z;
-    } else {
-        nd->b.z = lo.x;
-        nd->b.w = lo.y;
-        nd->c = make_float4(lo.z, hi.x, hi.y, hi.z);
-    }
-}
+// The tree is built and refit bottom-up in tiles of kTreeTile sorted leaves, one
+// workgroup each; a node whose leaf range crosses a tile boundary is a "top"
+// node, made by k_top_nodes.
+constexpr int kTreeTile = 1024;  // leaves per workgroup, one per lane
+constexpr uint16_t kNoSplit = 0xffffu;
 
 __device__ __forceinline__ void write_root(float *rootBox, float4 lo, float4 hi)
 {
@@ -135,18 +51,6 @@ __device__ __forceinline__ void write_root(float *rootBox, float4 lo, float4 hi)
     rootBox[5] = hi.z;
 }
 
-// Refit, stage 1: one workgroup per tile of kRefitTile sorted leaves, one
-// leaf per lane.  Every leaf walks up; at a node whose leaf range lies inside
-// the tile the first of its two children to arrive leaves its box in LDS and
-// stops, the second merges and continues.  All hand-offs stay inside the
-// workgroup (LDS + workgroup-scope fences), so no lane ever waits and no
-// device-wide fence is needed.  At a node whose range leaves the tile (a
-// "top" node) the lane stores its box in the node and stops.
-//
-// The workgroup also writes the union of the tile's leaf boxes up to a leaf
-// position (prefix) where a top node's range ends and from it (suffix) where
-// one starts, and the tile's box.  Box unions are exact (min / max), so stage
-// 2 can assemble any top node's box from these pieces in any order.
 __device__ __forceinline__ void put6(float *dst, const float v[6])
 {
 #pragma unroll
@@ -154,102 +58,166 @@ __device__ __forceinline__ void put6(float *dst, const float v[6])
         dst[k] = v[k];
 }
 
-__global__ __launch_bounds__(kRefitTile) void k_refit_tiles(const uint32_t *__restrict__ ids,
-                                                            const float *__restrict__ box32, int n,
-                                                            BNode *__restrict__ nodes,
-                                                            const uint32_t *__restrict__ leafParent,
-                                                            const uint8_t *__restrict__ need,
-                                                            float *__restrict__ prefix, float *__restrict__ suffix,
-                                                            float *__restrict__ tileBox, float *rootBox)
+// Stage 1: the radix tree of a tile's leaves, bottom-up.  The tree is fixed by
+// the common-prefix lengths of neighbouring keys alone: the parent of a node
+// over leaves [lo, hi] splits at hi or at lo - 1, whichever neighbour shares
+// the longer prefix (Apetrei, "Fast and Simple Agglomerative LBVH
+// Construction", 2014), so a walk from every leaf needs no search in the keys.
+// At a split inside the tile the first child to arrive leaves its box,
+// reference and far end in LDS and stops, the second merges and goes on.  All
+// hand-offs stay inside the workgroup, so no lane waits and no device-wide
+// fence is needed.  Karras' numbering is kept: a node that is its parent's left
+// child is node hi, a right child node lo, the root node 0, so a node inside
+// the tile has its index inside the tile too.
+//
+// A split that only one child reached belongs to a top node; that child (a
+// "piece" of the tile, like one whose parent splits on the tile's border) goes
+// to piece[lo] as a box, and the union of the tile's leaves from lo on (suffix)
+// and up to hi (prefix) is kept for the top nodes that start or end there.  Box
+// unions are exact (min / max), so stage 2 can assemble any top node's box
+// from these in any order.  Indices inside the tile that no node took are top
+// nodes; they are listed.
+//
+// Bound by the latency of the walk's LDS steps (and the 64-B node stores).  In
+// the pair step at 1,310,720 leaves (another mesh's kernels beside) it takes
+// 114 us and the top nodes 35; searching every node's range and split in the
+// global keys (about 60 dependent loads each) took 116 us before a refit of
+// 119 + 15.  The batch's 3.0 M leaves: 176 + 37 us, before 188 + 162 + 8.
+template <typename K>
+__global__ __launch_bounds__(kTreeTile) void k_tree_tiles(const K *__restrict__ codes,
+                                                          const uint32_t *__restrict__ ids,
+                                                          const float *__restrict__ box32, int n,
+                                                          BNode *__restrict__ nodes, uint32_t *__restrict__ topList,
+                                                          uint32_t *topCount, float *__restrict__ prefix,
+                                                          float *__restrict__ suffix, float *__restrict__ piece,
+                                                          float *__restrict__ tileBox, float *rootBox)
 {
-    __shared__ float s_box[kRefitTile][2][6];
-    __shared__ uint32_t s_flag[kRefitTile];
-    __shared__ float s_wave[kRefitTile / 64][6];
-    __shared__ int4 s_d[kRefitTile];  // links of internal nodes [tile0, tile0 + kRefitTile)
-    const int tile0 = blockIdx.x * kRefitTile;
-    const int tile1 = min(tile0 + kRefitTile, n);
-    const int pos = tile0 + threadIdx.x;
+    __shared__ float s_box[kTreeTile][2][6];        // per split: the children's boxes,
+    __shared__ uint32_t s_ref[kTreeTile][2];        // references,
+    __shared__ uint16_t s_far[kTreeTile][2];        // far ends (offset in the tile)
+    __shared__ uint16_t s_child[kTreeTile][2];      // and own splits (kNoSplit: a leaf)
+    __shared__ uint32_t s_flag[kTreeTile];          // arrivals: 1, + kRightCame for a right child
+    __shared__ uint16_t s_idx[kTreeTile], s_end[kTreeTile];  // per split: its node's index and other end
+    __shared__ uint16_t s_parent[kTreeTile];        // and its parent's index (kNoSplit: none in the tile)
+    __shared__ int8_t s_delta[kTreeTile + 1];       // prefix length of (pos - 1, pos)
+    __shared__ uint8_t s_taken[kTreeTile], s_start[kTreeTile], s_stop[kTreeTile];
+    __shared__ float s_wave[kTreeTile / 64][6];
+    __shared__ uint32_t s_ntop, s_top0;
+    constexpr uint32_t kRightCame = 0x100u;
+    const int tile0 = blockIdx.x * kTreeTile;
+    const int tile1 = min(tile0 + kTreeTile, n);
+    const int me = threadIdx.x, pos = tile0 + me;
     const bool valid = pos < tile1;
-    s_flag[threadIdx.x] = 0;
-    // A node whose leaf range lies inside the tile has its index inside the
-    // tile too (internal node i covers leaves [min(i, j), max(i, j)]), so the
-    // walks below read the links of those nodes from one coalesced load here
-    // instead of one dependent global load per level.
-    if (pos < n - 1)
-        s_d[threadIdx.x] = nodes[pos].d;
+    if (me == 0)
+        s_ntop = 0;
+    s_flag[me] = 0;
+    s_taken[me] = s_start[me] = s_stop[me] = 0;
+    if (valid)
+        s_delta[me] = (int8_t)delta(codes, n, pos, pos - 1);
+    if (pos == tile1 - 1)
+        s_delta[me + 1] = (int8_t)delta(codes, n, pos, pos + 1);
     __syncthreads();
-    float4 lo = make_float4(__builtin_inff(), __builtin_inff(), __builtin_inff(), 0.0f);
-    float4 hi = make_float4(-__builtin_inff(), -__builtin_inff(), -__builtin_inff(), 0.0f);
+    float4 lo4 = make_float4(__builtin_inff(), __builtin_inff(), __builtin_inff(), 0.0f);
+    float4 hi4 = make_float4(-__builtin_inff(), -__builtin_inff(), -__builtin_inff(), 0.0f);
     if (valid) {
         const uint32_t tri = ids[pos];
-        lo = reinterpret_cast<const float4 *>(box32 + (size_t)kBox32Stride * tri)[0];
-        hi = reinterpret_cast<const float4 *>(box32 + (size_t)kBox32Stride * tri)[1];
-        float4 wl = lo, wh = hi;
-        int node = (int)leafParent[pos];
-        int child = (int)(kLeafBit | tri);
-        // Each step moves to a strictly larger leaf range, so a walk ends
-        // within the tile's depth; the bound only guards malformed input.
-        // The walk reads and writes LDS only: a node inside the tile gets its
-        // child boxes from LDS after the walk, and the one global store is the
-        // box the walk carries into its top node.  (A global store inside
-        // the loop would hold every step's fence until the store lands.)
-        bool outside = false;  // the walk stopped at a top node with no links in LDS
-        for (int step = 0; step < kRefitTile; ++step) {
-            if (node < tile0 || node >= tile0 + kRefitTile || node >= n - 1) {
-                outside = true;
-                break;
+        lo4 = reinterpret_cast<const float4 *>(box32 + (size_t)kBox32Stride * tri)[0];
+        hi4 = reinterpret_cast<const float4 *>(box32 + (size_t)kBox32Stride * tri)[1];
+        float4 wl = lo4, wh = hi4;
+        uint32_t ref = kLeafBit | tri;
+        int lo = me, hi = me;  // offsets in the tile
+        uint16_t mine = kNoSplit;
+        // each step moves to a strictly larger range, so a walk ends within
+        // the tile's depth; the bound only guards malformed input
+        for (int step = 0; step <= kTreeTile; ++step) {
+            const int dl = s_delta[lo], dr = s_delta[hi + 1];
+            const bool left = dr > dl;  // a left child: its parent splits behind hi
+            if (mine != kNoSplit) {
+                const int idx = left ? hi : lo;
+                s_idx[mine] = (uint16_t)idx;
+                s_end[mine] = (uint16_t)(left ? lo : hi);
+                s_taken[idx] = 1;
+                s_parent[mine] = kNoSplit;  // until its parent is met
+                for (int c = 0; c < 2; ++c)
+                    if (s_child[mine][c] != kNoSplit)
+                        s_parent[s_child[mine][c]] = (uint16_t)idx;
+                ref = (uint32_t)(tile0 + idx);
             }
-            const int local = node - tile0;
-            const int4 d = s_d[local];
-            const int slot = (d.x == child) ? 0 : 1;
-            const int lo_leaf = min(node, d.w), hi_leaf = max(node, d.w);
-            if (lo_leaf < tile0 || hi_leaf >= tile1 || (lo_leaf / kRefitTile) != (hi_leaf / kRefitTile)) {
-                store_child_box(nodes + node, slot, wl, wh);
-                break;
-            }
-            float *mine = s_box[local][slot];
-            mine[0] = wl.x;
-            mine[1] = wl.y;
-            mine[2] = wl.z;
-            mine[3] = wh.x;
-            mine[4] = wh.y;
-            mine[5] = wh.z;
-            __threadfence_block();
-            if (atomicAdd(&s_flag[local], 1u) == 0)
-                break;
-            __threadfence_block();
-            const float *o = s_box[local][1 - slot];
-            wl = make_float4(fminf(wl.x, o[0]), fminf(wl.y, o[1]), fminf(wl.z, o[2]), 0.0f);
-            wh = make_float4(fmaxf(wh.x, o[3]), fmaxf(wh.y, o[4]), fmaxf(wh.z, o[5]), 0.0f);
-            child = node;
-            node = d.z;
-            if (node < 0) {  // the whole tree fits in this tile
+            if (dl < 0 && dr < 0) {  // the whole tree
                 write_root(rootBox, wl, wh);
                 break;
             }
-        }
-        if (outside) {
-            BNode *nd = nodes + node;
-            store_child_box(nd, nd->d.x == child ? 0 : 1, wl, wh);
+            const int split = left ? hi : lo - 1;
+            if (split < 0 || tile0 + split + 1 >= tile1) {  // its sibling lies in the next tile
+                const float b[6] = {wl.x, wl.y, wl.z, wh.x, wh.y, wh.z};
+                put6(piece + 6 * (size_t)(tile0 + lo), b);
+                s_start[lo] = 1;
+                s_stop[hi] = 1;
+                break;
+            }
+            const int side = left ? 0 : 1;
+            float *slot = s_box[split][side];
+            slot[0] = wl.x;
+            slot[1] = wl.y;
+            slot[2] = wl.z;
+            slot[3] = wh.x;
+            slot[4] = wh.y;
+            slot[5] = wh.z;
+            s_ref[split][side] = ref;
+            s_far[split][side] = (uint16_t)(left ? lo : hi);
+            s_child[split][side] = mine;
+            __threadfence_block();
+            if (atomicAdd(&s_flag[split], left ? 1u : 1u + kRightCame) == 0)
+                break;
+            __threadfence_block();
+            const float *o = s_box[split][1 - side];
+            wl = make_float4(fminf(wl.x, o[0]), fminf(wl.y, o[1]), fminf(wl.z, o[2]), 0.0f);
+            wh = make_float4(fmaxf(wh.x, o[3]), fmaxf(wh.y, o[4]), fmaxf(wh.z, o[5]), 0.0f);
+            if (left)
+                hi = s_far[split][1];
+            else
+                lo = s_far[split][0];
+            mine = (uint16_t)split;
         }
     }
-    __syncthreads();  // every walk's LDS boxes
-    // nodes inside the tile: both child boxes, from LDS
-    if (pos < n - 1) {
-        const int4 d = s_d[threadIdx.x];
-        const int lo_leaf = min(pos, d.w), hi_leaf = max(pos, d.w);
-        if (lo_leaf >= tile0 && hi_leaf < tile1 && (lo_leaf / kRefitTile) == (hi_leaf / kRefitTile)) {
-            const float *b0 = s_box[threadIdx.x][0], *b1 = s_box[threadIdx.x][1];
-            BNode *nd = nodes + pos;
-            nd->a = make_float4(b0[0], b0[1], b0[2], b0[3]);
-            nd->b = make_float4(b0[4], b0[5], b1[0], b1[1]);
-            nd->c = make_float4(b1[2], b1[3], b1[4], b1[5]);
-        }
+    __syncthreads();
+    const uint32_t came = s_flag[me];
+    if ((came & 255u) == 2u) {
+        // a node of the tile, whole
+        const float *b0 = s_box[me][0], *b1 = s_box[me][1];
+        BNode *nd = nodes + tile0 + s_idx[me];
+        nd->a = make_float4(b0[0], b0[1], b0[2], b0[3]);
+        nd->b = make_float4(b0[4], b0[5], b1[0], b1[1]);
+        nd->c = make_float4(b1[2], b1[3], b1[4], b1[5]);
+        // a parent outside the tile writes its children's links itself
+        const int parent = s_parent[me] == kNoSplit ? -1 : tile0 + s_parent[me];
+        nd->d = make_int4((int)s_ref[me][0], (int)s_ref[me][1], parent, tile0 + s_end[me]);
+    } else if (came) {
+        // one child of a top node
+        const int side = came & kRightCame ? 1 : 0;
+        const int lo = side ? me + 1 : s_far[me][0], hi = side ? s_far[me][1] : me;
+        put6(piece + 6 * (size_t)(tile0 + lo), s_box[me][side]);
+        s_start[lo] = 1;
+        s_stop[hi] = 1;
     }
+    if (gridDim.x == 1)  // one tile: no top node
+        return;
+    // indices no node of the tile took: slots from LDS, one global reservation
+    // per tile (one per wave held the kernel to the rate of one counter: 215
+    // us at 3.0 M leaves)
+    const int lane = me & 63, wave = me >> 6;
+    const bool top = pos < n - 1 && valid && !s_taken[me];
+    const unsigned long long tops = __ballot(top);
+    uint32_t slot = 0;
+    if (lane == 0 && tops)
+        slot = atomicAdd(&s_ntop, (uint32_t)__popcll(tops));
+    slot = __shfl(slot, 0, 64) + (uint32_t)__popcll(tops & ((1ull << lane) - 1ull));
+    __syncthreads();
+    if (me == 0)
+        s_top0 = s_ntop ? atomicAdd(topCount, s_ntop) : 0u;
     // prefix / suffix unions over the tile's positions: wave scans, then the
     // waves' totals
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    float pv[6] = {lo.x, lo.y, lo.z, hi.x, hi.y, hi.z}, sv[6] = {lo.x, lo.y, lo.z, hi.x, hi.y, hi.z};
+    float pv[6] = {lo4.x, lo4.y, lo4.z, hi4.x, hi4.y, hi4.z}, sv[6] = {lo4.x, lo4.y, lo4.z, hi4.x, hi4.y, hi4.z};
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) {
 #pragma unroll
@@ -264,7 +232,9 @@ __global__ __launch_bounds__(kRefitTile) void k_refit_tiles(const uint32_t *__re
     if (lane == 63)
         put6(s_wave[wave], pv);
     __syncthreads();
-    for (int w = 0; w < kRefitTile / 64; ++w) {
+    if (top)
+        topList[s_top0 + slot] = (uint32_t)pos;
+    for (int w = 0; w < kTreeTile / 64; ++w) {
         if (w < wave)
 #pragma unroll
             for (int k = 0; k < 6; ++k)
@@ -275,13 +245,12 @@ __global__ __launch_bounds__(kRefitTile) void k_refit_tiles(const uint32_t *__re
                 sv[k] = k < 3 ? fminf(sv[k], s_wave[w][k]) : fmaxf(sv[k], s_wave[w][k]);
     }
     if (valid) {
-        const uchar2 nd2 = reinterpret_cast<const uchar2 *>(need)[pos];
-        if (nd2.y)
+        if (s_stop[me])
             put6(prefix + 6 * (size_t)pos, pv);
-        if (nd2.x)
+        if (s_start[me])
             put6(suffix + 6 * (size_t)pos, sv);
     }
-    if (threadIdx.x == kRefitTile - 1)
+    if (me == kTreeTile - 1)
         put6(tileBox + 6 * (size_t)blockIdx.x, pv);
 }
 
@@ -342,43 +311,84 @@ __global__ __launch_bounds__(1024) void k_tile_table(float *__restrict__ table, 
     }
 }
 
-// Refit, stage 2: every top node at once.  A top node's leaf range [lo, hi]
-// runs from inside tile tl to inside tile th > tl; its box is the suffix of tl
-// at lo, the prefix of th at hi, and (when th > tl + 1) two sparse-table
-// entries covering the whole tiles between.  It goes into the parent's child
-// slot (or the root box), so nothing waits on anything.
-__global__ __launch_bounds__(256) void k_refit_top(BNode *__restrict__ nodes, const uint32_t *__restrict__ topList,
+// Box of the leaves [lo, hi], a child of a top node: a piece of one tile, or
+// the suffix of lo's tile, the prefix of hi's and (with whole tiles between)
+// two sparse-table entries.
+__device__ __forceinline__ void range_box(uint32_t lo, uint32_t hi, const float *__restrict__ prefix,
+                                          const float *__restrict__ suffix, const float *__restrict__ piece,
+                                          const float *__restrict__ table, uint32_t ntiles, float v[6])
+{
+    const uint32_t tl = lo / kTreeTile, th = hi / kTreeTile;
+    const float *a = tl == th ? piece + 6 * (size_t)lo : suffix + 6 * (size_t)lo;
+    const float *b = tl == th ? a : prefix + 6 * (size_t)hi;
+#pragma unroll
+    for (int c = 0; c < 6; ++c)
+        v[c] = c < 3 ? fminf(a[c], b[c]) : fmaxf(a[c], b[c]);
+    if (th > tl + 1) {
+        const uint32_t first = tl + 1, len = th - first;
+        const int j = 31 - __clz(len);
+        const float *x = table + 6 * ((size_t)j * ntiles + first);
+        const float *y = table + 6 * ((size_t)j * ntiles + th - (1u << j));
+#pragma unroll
+        for (int c = 0; c < 6; ++c)
+            v[c] = c < 3 ? fminf(v[c], fminf(x[c], y[c])) : fmaxf(v[c], fmaxf(x[c], y[c]));
+    }
+}
+
+// Stage 2: every top node at once, a few per tile: its range and split from the
+// keys by Karras' searches, its children's boxes from the tiles' pieces.  It
+// writes its children's parent links, so nothing waits on anything.
+template <typename K>
+__global__ __launch_bounds__(256) void k_top_nodes(const K *__restrict__ codes, const uint32_t *__restrict__ ids, int n,
+                                                   BNode *__restrict__ nodes, const uint32_t *__restrict__ topList,
                                                    const uint32_t *__restrict__ topCount,
                                                    const float *__restrict__ prefix, const float *__restrict__ suffix,
-                                                   const float *__restrict__ table, uint32_t ntiles, float *rootBox)
+                                                   const float *__restrict__ piece, const float *__restrict__ table,
+                                                   uint32_t ntiles, float *rootBox)
 {
     const uint32_t ntop = *topCount;
     for (uint32_t k = blockIdx.x * 256 + threadIdx.x; k < ntop; k += gridDim.x * 256) {
-        const uint32_t p = topList[k];
-        const int4 d = nodes[p].d;
-        const uint32_t lo = p < (uint32_t)d.w ? p : (uint32_t)d.w;
-        const uint32_t hi = p < (uint32_t)d.w ? (uint32_t)d.w : p;
-        const uint32_t tl = lo / kRefitTile, th = hi / kRefitTile;
-        float v[6];
-        const float *a = suffix + 6 * (size_t)lo, *b = prefix + 6 * (size_t)hi;
-#pragma unroll
-        for (int c = 0; c < 6; ++c)
-            v[c] = c < 3 ? fminf(a[c], b[c]) : fmaxf(a[c], b[c]);
-        if (th > tl + 1) {
-            const uint32_t first = tl + 1, len = th - 1 - first + 1;
-            const int j = 31 - __clz(len);
-            const float *x = table + 6 * ((size_t)j * ntiles + first);
-            const float *y = table + 6 * ((size_t)j * ntiles + (th - 1) - (1u << j) + 1);
-#pragma unroll
-            for (int c = 0; c < 6; ++c)
-                v[c] = c < 3 ? fminf(v[c], fminf(x[c], y[c])) : fmaxf(v[c], fmaxf(x[c], y[c]));
-        }
-        const float4 blo = make_float4(v[0], v[1], v[2], 0.0f), bhi = make_float4(v[3], v[4], v[5], 0.0f);
-        if (d.z < 0) {
-            write_root(rootBox, blo, bhi);
-        } else {
-            BNode *pn = nodes + d.z;
-            store_child_box(pn, pn->d.x == (int)p ? 0 : 1, blo, bhi);
+        const int i = (int)topList[k];
+        const int d = (delta(codes, n, i, i + 1) - delta(codes, n, i, i - 1)) >= 0 ? 1 : -1;
+        const int dmin = delta(codes, n, i, i - d);
+        int lmax = 2;
+        while (delta(codes, n, i, i + lmax * d) > dmin)
+            lmax <<= 1;
+        int l = 0;
+        for (int t = lmax >> 1; t >= 1; t >>= 1)
+            if (delta(codes, n, i, i + (l + t) * d) > dmin)
+                l += t;
+        const int j = i + l * d;
+        const int dnode = delta(codes, n, i, j);
+        int s = 0;
+        int t = l;
+        do {
+            t = (t + 1) >> 1;
+            if (delta(codes, n, i, i + (s + t) * d) > dnode)
+                s += t;
+        } while (t > 1);
+        const int gamma = i + s * d + (d < 0 ? d : 0);
+        const int lo = i < j ? i : j;
+        const int hi = i < j ? j : i;
+        float b0[6], b1[6];
+        range_box((uint32_t)lo, (uint32_t)gamma, prefix, suffix, piece, table, ntiles, b0);
+        range_box((uint32_t)gamma + 1, (uint32_t)hi, prefix, suffix, piece, table, ntiles, b1);
+        BNode *nd = nodes + i;
+        nd->a = make_float4(b0[0], b0[1], b0[2], b0[3]);
+        nd->b = make_float4(b0[4], b0[5], b1[0], b1[1]);
+        nd->c = make_float4(b1[2], b1[3], b1[4], b1[5]);
+        nd->d.x = lo == gamma ? (int)(kLeafBit | ids[gamma]) : gamma;
+        nd->d.y = hi == gamma + 1 ? (int)(kLeafBit | ids[gamma + 1]) : gamma + 1;
+        nd->d.w = j;  // the node covers sorted leaves [min(i, j), max(i, j)]
+        if (lo != gamma)
+            nodes[gamma].d.z = i;
+        if (hi != gamma + 1)
+            nodes[gamma + 1].d.z = i;
+        if (i == 0) {
+            nd->d.z = -1;
+            write_root(rootBox,
+                       make_float4(fminf(b0[0], b1[0]), fminf(b0[1], b1[1]), fminf(b0[2], b1[2]), 0.0f),
+                       make_float4(fmaxf(b0[3], b1[3]), fmaxf(b0[4], b1[4]), fmaxf(b0[5], b1[5]), 0.0f));
         }
     }
 }
@@ -425,28 +435,6 @@ void launch_fill_u32(uint32_t *p, uint32_t value, size_t n, hipStream_t s)
     hipLaunchKernelGGL(k_fill_u32, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, p, value, n);
 }
 
-uint32_t hierarchy_zeroed_u32(uint32_t n) { return (uint32_t)top_work_zeroed(n); }
-
-// work: top_work(work, n), its first top_work_zeroed(n) u32 already zero
-void launch_hierarchy(const uint32_t *codes, const uint32_t *ids, uint32_t n, BNode *nodes,
-                      uint32_t *leafParent, uint32_t *work, hipStream_t s)
-{
-    if (n < 2)
-        return;
-    hipLaunchKernelGGL(k_hierarchy<uint32_t>, dim3((n - 1 + 255) / 256), dim3(256), 0, s, codes, ids, (int)n, nodes,
-                       leafParent, top_work(work, n));
-}
-
-void launch_hierarchy64(const uint64_t *codes, const uint32_t *ids, uint32_t n, BNode *nodes,
-                        uint32_t *leafParent, uint32_t *work, hipStream_t s)
-{
-    if (n < 2)
-        return;
-    launch_fill_u32(work, 0u, top_work_zeroed(n), s);
-    hipLaunchKernelGGL(k_hierarchy<uint64_t>, dim3((n - 1 + 255) / 256), dim3(256), 0, s, codes, ids, (int)n, nodes,
-                       leafParent, top_work(work, n));
-}
-
 static int table_levels(uint32_t ntiles)
 {
     int L = 1;
@@ -455,23 +443,25 @@ static int table_levels(uint32_t ntiles)
     return L;
 }
 
-size_t refit_scratch_floats(uint32_t n)
+size_t tree_scratch_floats(uint32_t n)
 {
-    const uint32_t ntiles = (n + kRefitTile - 1) / kRefitTile;
-    return 12 * (size_t)n + 6 * (size_t)ntiles * table_levels(ntiles) + 6;
+    const uint32_t ntiles = (n + kTreeTile - 1) / kTreeTile;
+    return 18 * (size_t)n + 6 * (size_t)ntiles * table_levels(ntiles) + 6;
 }
 
-// scratch: refit_scratch_floats(n) floats (prefix, suffix, tile table)
-void launch_refit(const uint32_t *ids, const float *box32, uint32_t n, BNode *nodes,
-                  const uint32_t *leafParent, uint32_t *work, float *scratch, float *rootBox, hipStream_t s)
+// work: n + 1 u32 (the top-node count, zero on entry, then the top-node list);
+// scratch: tree_scratch_floats(n) floats (prefix, suffix, pieces, tile table)
+template <typename K>
+static void tree(const K *codes, const uint32_t *ids, const float *box32, uint32_t n, BNode *nodes, uint32_t *work,
+                 float *scratch, float *rootBox, hipStream_t s)
 {
     if (n < 2)
         return;
-    const uint32_t ntiles = (n + kRefitTile - 1) / kRefitTile;
-    float *prefix = scratch, *suffix = scratch + 6 * (size_t)n, *table = scratch + 12 * (size_t)n;
-    const TopWork top = top_work(work, n);
-    hipLaunchKernelGGL(k_refit_tiles, dim3(ntiles), dim3(kRefitTile), 0, s, ids, box32, (int)n, nodes, leafParent,
-                       (const uint8_t *)top.need, prefix, suffix, table, rootBox);
+    const uint32_t ntiles = (n + kTreeTile - 1) / kTreeTile;
+    float *prefix = scratch, *suffix = prefix + 6 * (size_t)n, *piece = suffix + 6 * (size_t)n;
+    float *table = piece + 6 * (size_t)n;
+    hipLaunchKernelGGL(k_tree_tiles<K>, dim3(ntiles), dim3(kTreeTile), 0, s, codes, ids, box32, (int)n, nodes, work + 1,
+                       work, prefix, suffix, piece, table, rootBox);
     if (ntiles < 2)
         return;
     const size_t lds = ntiles <= kLdsTiles ? sizeof(float) * 6 * ntiles : 0;
@@ -479,8 +469,22 @@ void launch_refit(const uint32_t *ids, const float *box32, uint32_t n, BNode *no
         (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_tile_table),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     hipLaunchKernelGGL(k_tile_table, dim3(1), dim3(1024), lds, s, table, ntiles, table_levels(ntiles));
-    hipLaunchKernelGGL(k_refit_top, dim3(256), dim3(256), 0, s, nodes, (const uint32_t *)top.list,
-                       (const uint32_t *)top.count, prefix, suffix, table, ntiles, rootBox);
+    hipLaunchKernelGGL(k_top_nodes<K>, dim3(256), dim3(256), 0, s, codes, ids, (int)n, nodes,
+                       (const uint32_t *)(work + 1), (const uint32_t *)work, prefix, suffix, piece, table, ntiles,
+                       rootBox);
+}
+
+void launch_tree(const uint32_t *codes, const uint32_t *ids, const float *box32, uint32_t n, BNode *nodes,
+                 uint32_t *work, float *scratch, float *rootBox, hipStream_t s)
+{
+    tree(codes, ids, box32, n, nodes, work, scratch, rootBox, s);
+}
+
+void launch_tree64(const uint64_t *codes, const uint32_t *ids, const float *box32, uint32_t n, BNode *nodes,
+                   uint32_t *work, float *scratch, float *rootBox, hipStream_t s)
+{
+    launch_fill_u32(work, 0u, 1, s);
+    tree(codes, ids, box32, n, nodes, work, scratch, rootBox, s);
 }
 
 }  // namespace sbg

@@ -87,8 +87,8 @@ struct sbg_mesh_s {
     DevBuf<double> V;
     DevBuf<uint32_t> T;
     DevBuf<double> tri64;
-    DevBuf<float> tri32, box32, blockBounds, bounds, rootBox, refitScratch;
-    DevBuf<uint32_t> keys, vals, keysAlt, valsAlt, leafParent, flags;
+    DevBuf<float> tri32, box32, blockBounds, bounds, rootBox, treeScratch;
+    DevBuf<uint32_t> keys, vals, keysAlt, valsAlt, treeWork;
     DevBuf<BNode> nodes;
     uint32_t root = 0;
     const uint32_t *sortedIds = nullptr;  // triangles in Morton order (vals or valsAlt)
@@ -226,13 +226,12 @@ static void mesh_free_buffers(sbg_mesh m)
     m->blockBounds.release();
     m->bounds.release();
     m->rootBox.release();
-    m->refitScratch.release();
+    m->treeScratch.release();
     m->keys.release();
     m->vals.release();
     m->keysAlt.release();
     m->valsAlt.release();
-    m->leafParent.release();
-    m->flags.release();
+    m->treeWork.release();
     m->nodes.release();
     m->gridCells.release();
     m->gridTemp.release();
@@ -733,10 +732,9 @@ int sbg_mesh_prepare(sbg_mesh m)
     TRY(m->vals.ensure(nt));
     TRY(m->keysAlt.ensure(nt));
     TRY(m->valsAlt.ensure(nt));
-    TRY(m->leafParent.ensure(nt));
     TRY(m->nodes.ensure(nt > 1 ? nt - 1 : 1));
-    TRY(m->flags.ensure(2 * nt + 1));
-    TRY(m->refitScratch.ensure(refit_scratch_floats((uint32_t)nt)));
+    TRY(m->treeWork.ensure(nt + 1));
+    TRY(m->treeScratch.ensure(tree_scratch_floats((uint32_t)nt)));
     TRY(m->hist.ensure(sort_hist_entries(nt)));
     const hipStream_t s = m->stream;
     const bool onAux = s != c->stream;
@@ -757,8 +755,7 @@ int sbg_mesh_prepare(sbg_mesh m)
         launch_records(m->V.p, m->T.p, (uint32_t)nt, m->tri64.p, m->tri32.p, m->box32.p,
                        m->blockBounds.p, nb, s);
         launch_bounds_reduce(m->blockBounds.p, nb, m->bounds.p, s);
-        launch_morton(m->box32.p, m->bounds.p, (uint32_t)nt, m->keys.p, m->vals.p, m->flags.p,
-                      nt > 1 ? hierarchy_zeroed_u32((uint32_t)nt) : 0u, s);
+        launch_morton(m->box32.p, m->bounds.p, (uint32_t)nt, m->keys.p, m->vals.p, m->treeWork.p, s);
         TRY(check_launch("records"));
     }
     uint32_t *sk = m->keys.p, *sv = m->vals.p;
@@ -780,9 +777,8 @@ int sbg_mesh_prepare(sbg_mesh m)
                                    s));
         } else {
             m->root = 0;
-            launch_hierarchy(sk, sv, (uint32_t)nt, m->nodes.p, m->leafParent.p, m->flags.p, s);
-            launch_refit(sv, m->box32.p, (uint32_t)nt, m->nodes.p, m->leafParent.p, m->flags.p, m->refitScratch.p,
-                         m->rootBox.p, s);
+            launch_tree(sk, sv, m->box32.p, (uint32_t)nt, m->nodes.p, m->treeWork.p, m->treeScratch.p, m->rootBox.p,
+                        s);
         }
         TRY(check_launch("bvh"));
     }

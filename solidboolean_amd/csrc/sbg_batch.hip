@@ -48,10 +48,10 @@ struct sbg_batch_s {
     DevBuf<double> V;
     DevBuf<uint32_t> T, meshOf, target, triBegin;
     DevBuf<double> tri64;
-    DevBuf<float> tri32, box32, blockBounds, rootBox, meshBox, refitScratch;
+    DevBuf<float> tri32, box32, blockBounds, rootBox, meshBox, treeScratch;
     DevBuf<int> meshBounds, waveBounds;
     DevBuf<uint64_t> keys, keysAlt, codes;
-    DevBuf<uint32_t> ids, leafParent, work, meshRoot, hist;
+    DevBuf<uint32_t> ids, work, meshRoot, hist;
     DevBuf<BNode> nodes;
     DevBuf<uint2> front[2], spill;
     DevBuf<uint32_t> words;  // kWords device counters
@@ -166,9 +166,7 @@ int enqueue(sbg_batch b, int precision)
     b->keysInAlt = radix_sort_u64(b->keys.p, b->keysAlt.p, nt, keyRange, 1, b->hist.p, s) != 0;
     const uint64_t *sortedKeys = b->keysInAlt ? b->keysAlt.p : b->keys.p;
     launch_batch_codes(sortedKeys, nt, b->localBits, b->mortonBits, b->triBegin.p, b->codes.p, b->ids.p, s);
-    launch_hierarchy64(b->codes.p, b->ids.p, nt, b->nodes.p, b->leafParent.p, b->work.p, s);
-    launch_refit(b->ids.p, b->box32.p, nt, b->nodes.p, b->leafParent.p, b->work.p, b->refitScratch.p, b->rootBox.p,
-                 s);
+    launch_tree64(b->codes.p, b->ids.p, b->box32.p, nt, b->nodes.p, b->work.p, b->treeScratch.p, b->rootBox.p, s);
     launch_fill_u32(b->meshRoot.p, ~0u, b->nmeshes, s);
     launch_fill_u32(reinterpret_cast<uint32_t *>(b->meshBox.p), 0u, 6 * b->nmeshes, s);  // empty meshes: zero box
     launch_mesh_roots(b->nodes.p, b->ids.p, b->triBegin.p, (uint32_t)b->nmeshes, nt, b->box32.p, b->rootBox.p,
@@ -313,8 +311,8 @@ int sbg_batch_create(sbg_context ctx, const double *xyz, const uint32_t *tris, c
         (rc = b->meshBox.ensure(6 * nmeshes)) || (rc = b->meshBounds.ensure(6 * nmeshes)) ||
         (rc = b->waveBounds.ensure(6 * ((nt + 63) / 64))) ||
         (rc = b->keys.ensure(nt)) || (rc = b->keysAlt.ensure(nt)) || (rc = b->codes.ensure(nt)) ||
-        (rc = b->ids.ensure(nt)) || (rc = b->leafParent.ensure(nt)) || (rc = b->work.ensure(2 * nt + 1)) ||
-        (rc = b->refitScratch.ensure(refit_scratch_floats((uint32_t)nt))) ||
+        (rc = b->ids.ensure(nt)) || (rc = b->work.ensure(nt + 1)) ||
+        (rc = b->treeScratch.ensure(tree_scratch_floats((uint32_t)nt))) ||
         (rc = b->meshRoot.ensure(nmeshes)) || (rc = b->nodes.ensure(nt > 1 ? nt - 1 : 1)) ||
         (rc = b->words.ensure(kWords)) || (rc = b->flags.ensure(nt + 4)) || (rc = b->bits.ensure(3 * nt + 4)) ||
         (rc = b->votes.ensure(nt)) || (rc = b->pts.ensure(4 * nt)) || (rc = b->rayList.ensure(ray_list_u32(nt))))
@@ -693,11 +691,11 @@ int sbg_batch_destroy(sbg_batch b)
     DevBuf<double> *d64[] = {&b->V, &b->tri64, &b->seg, &b->pts};
     for (auto *p : d64)
         p->release();
-    DevBuf<float> *f32[] = {&b->tri32, &b->box32, &b->blockBounds, &b->rootBox, &b->meshBox, &b->refitScratch};
+    DevBuf<float> *f32[] = {&b->tri32, &b->box32, &b->blockBounds, &b->rootBox, &b->meshBox, &b->treeScratch};
     for (auto *p : f32)
         p->release();
     DevBuf<uint32_t> *u32[] = {&b->T,    &b->meshOf,     &b->target,   &b->triBegin, &b->ids,
-                               &b->leafParent, &b->work, &b->meshRoot, &b->hist,     &b->words,
+                               &b->work, &b->meshRoot, &b->hist,     &b->words,
                                &b->gdWork, &b->rayList, &b->gridCells, &b->gridTemp};
     for (auto *p : u32)
         p->release();

@@ -40,9 +40,9 @@ void launch_normals64(const double *tri64, uint32_t nt, double *out, hipStream_t
 int records_blocks(uint32_t nt);
 void launch_boxes64(const double *tri64, uint32_t nt, double *out, hipStream_t s);
 void launch_bounds_reduce(const float *blockBounds, int nblocks, float *bounds, hipStream_t s);
-// also clears zero[0, nzero) (the hierarchy's scratch, one launch fewer)
+// also clears *zero (the tree's top-node count, one launch fewer)
 void launch_morton(const float *box32, const float *bounds, uint32_t nt, uint32_t *keys, uint32_t *vals,
-                   uint32_t *zero, uint32_t nzero, hipStream_t s);
+                   uint32_t *zero, hipStream_t s);
 
 // k_sort.hip: stable LSD radix sort; keys (and optional u32 values) ping-pong
 // between the two buffers; returns 1 when the result ended in the alt buffers.
@@ -68,20 +68,14 @@ int radix_sort_u64(uint64_t *keys, uint64_t *keysAlt, size_t n, const int *bitRa
                    uint32_t *hist, hipStream_t s, const uint32_t *count = nullptr);
 
 // k_lbvh.hip
-// work: 2n + 1 u32 of scratch shared by the two (top-node count, the leaf
-// positions where top nodes' ranges start and end, top-node list);
-// refit scratch: refit_scratch_floats(n) floats (per-tile prefix / suffix box
-// unions and the tile sparse table)
-size_t refit_scratch_floats(uint32_t n);
-// launch_hierarchy expects the first hierarchy_zeroed_u32(n) u32 of work to
-// be zero (launch_morton clears them); launch_hierarchy64 clears them itself
-uint32_t hierarchy_zeroed_u32(uint32_t n);
-void launch_hierarchy(const uint32_t *codes, const uint32_t *ids, uint32_t n, BNode *nodes,
-                      uint32_t *leafParent, uint32_t *work, hipStream_t s);
-void launch_hierarchy64(const uint64_t *codes, const uint32_t *ids, uint32_t n, BNode *nodes,
-                        uint32_t *leafParent, uint32_t *work, hipStream_t s);
-void launch_refit(const uint32_t *ids, const float *box32, uint32_t n, BNode *nodes,
-                  const uint32_t *leafParent, uint32_t *work, float *scratch, float *rootBox, hipStream_t s);
+// The tree over sorted codes: work holds n + 1 u32 (the first zero on entry:
+// launch_morton clears it, launch_tree64 clears it itself), scratch
+// tree_scratch_floats(n) floats (box unions within tiles and the tile table)
+size_t tree_scratch_floats(uint32_t n);
+void launch_tree(const uint32_t *codes, const uint32_t *ids, const float *box32, uint32_t n, BNode *nodes,
+                 uint32_t *work, float *scratch, float *rootBox, hipStream_t s);
+void launch_tree64(const uint64_t *codes, const uint32_t *ids, const float *box32, uint32_t n, BNode *nodes,
+                   uint32_t *work, float *scratch, float *rootBox, hipStream_t s);
 void launch_fill_u32(uint32_t *p, uint32_t value, size_t n, hipStream_t s);
 void launch_copy16(const void *src, void *dst, size_t n16, hipStream_t s);
 void launch_copy_u32(const uint32_t *src, uint32_t *dst, size_t n, hipStream_t s);

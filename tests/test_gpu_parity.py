@@ -141,6 +141,29 @@ def test_bvh_exact_across_refit_tiles(gpu, level):
     check_bvh(mesh, boxes64)
 
 
+@pytest.mark.parametrize("nt", [2, 3, 63, 65, 1023, 1024, 1025, 2047, 2048, 2049, 5000])
+@pytest.mark.parametrize("spread", ["even", "clumps", "equal"])
+def test_bvh_tile_sizes(gpu, nt, spread):
+    """Triangle soups of sizes at the tree tiles' edges: evenly spread, in a
+    few clumps of equal Morton codes (whose order and splits the triangle
+    positions decide) and all the same; parents named by their children."""
+    rng = np.random.default_rng(nt)
+    c = rng.random((nt, 1, 3))
+    if spread == "clumps":
+        c = np.round(c * 2)
+    elif spread == "equal":
+        c = np.zeros((nt, 1, 3))
+    v = (c + 1e-3 * rng.random((nt if spread == "even" else 1, 3, 3))).reshape(-1, 3)
+    mesh = gpu.mesh(v, np.arange(3 * nt).reshape(-1, 3))
+    corners = v.reshape(nt, 3, 3)
+    check_bvh(mesh, np.concatenate([corners.min(axis=1), corners.max(axis=1)], axis=1))
+    nodes, root, _ = mesh.bvh()
+    assert root == 0 and nodes[0]["parent"] == -1
+    for k in ("c0", "c1"):
+        inner = nodes[k] < 0x80000000
+        assert np.array_equal(nodes["parent"][nodes[k][inner]], np.nonzero(inner)[0])
+
+
 def test_pair_set(case):
     name, g, A, B = case
     p = A.find_pairs(B).array().astype(np.int64)
