@@ -5,12 +5,13 @@
 // Breadth-first over node pairs: each level's kernel reads the frontier written
 // by the previous one.  A thread loads the two nodes of its pair (64 B each,
 // both child boxes inside), tests the up-to-4 child combinations with the FP32
-// outward-rounded boxes (a superset test), and appends surviving internal pairs
-// to the next frontier.  Leaf-leaf survivors are rechecked with the exact FP64
-// closed box test on the 96-B FP64 records before they are appended to the
-// candidate queue.  Appends are wave-aggregated: one atomic per wave per queue,
-// offsets from a 64-lane prefix sum.  Queues past capacity raise `overflow`;
-// the host grows them and repeats the search, so nothing is ever dropped.
+// outward-rounded boxes (a superset test), and appends the surviving pairs to
+// the next frontier.  A pair of leaves met there is rechecked with the exact
+// FP64 closed box test on the 96-B FP64 records and becomes a candidate (one
+// test per lane; tested where the pair was found, a lane waited for the loads
+// of up to four in turn).  Appends take one atomic per wave or workgroup and
+// queue, offsets from ballots.  Queues past capacity raise `overflow`; the
+// host grows them and repeats the search, so nothing is ever dropped.
 #include "sbg_device.h"
 #include "sbg_internal.h"
 
@@ -41,29 +42,6 @@ __device__ __forceinline__ Box64 record_box(const double *__restrict__ tri64, ui
     return tri_box64({r0.x, r0.y, r1.x}, {r2.x, r2.y, r3.x}, {r4.x, r4.y, r5.x});
 }
 
-// wave-wide exclusive prefix of `cnt`; returns this lane's offset in the queue
-// (one atomic per wave) or ~0u when the queue would overflow.
-__device__ __forceinline__ uint32_t wave_reserve(uint32_t cnt, uint32_t *counter, uint32_t cap, uint32_t *overflow,
-                                                 uint32_t &waveBaseOut)
-{
-    const int lane = threadIdx.x & 63;
-    uint32_t incl = cnt;
-    for (int off = 1; off < 64; off <<= 1) {
-        uint32_t v = __shfl_up(incl, off, 64);
-        if (lane >= off)
-            incl += v;
-    }
-    const uint32_t total = __shfl(incl, 63, 64);
-    uint32_t base = 0;
-    if (lane == 63 && total)
-        base = atomicAdd(counter, total);
-    base = __shfl(base, 63, 64);
-    waveBaseOut = base;
-    if (total && base + total > cap && lane == 0)
-        atomicOr(overflow, 1u);
-    return base + incl - cnt;
-}
-
 // Children of a node reference: one (a leaf) or two, with their FP32 boxes.
 struct Kids {
     uint32_t c0, c1;
@@ -91,43 +69,51 @@ __device__ __forceinline__ Kids kids_of(const BNode *__restrict__ nodes, const f
     return k;
 }
 
-// Expansion of one node pair: child pair s = 2u + v (u over A's children, v
-// over B's) goes to the frontier (bit s of next) or, when both are leaves
-// whose exact FP64 boxes overlap, to the candidates (bit s of cand).  Every
-// field is a named register, so nothing lands in scratch memory.
-struct Expansion {
-    uint32_t a0, a1, b0, b1;
-    uint32_t next, cand;
-};
+__device__ __forceinline__ bool both_leaves(uint2 pr) { return (pr.x & pr.y & kLeafBit) != 0u; }
 
-// 0: pruned, 1: to the frontier, 2: candidate
-__device__ __forceinline__ uint32_t expand_one(const TraverseArgs &t, uint32_t ca, uint32_t cb, const FBox &ba,
-                                               const FBox &bb)
+// whether a pair of leaves is a candidate: the exact FP64 closed box test
+__device__ __forceinline__ bool leaves_overlap(const TraverseArgs &t, uint2 pr)
 {
-    if (!fbox_overlap(ba, bb))
-        return 0u;
-    if ((ca & kLeafBit) && (cb & kLeafBit))
-        return box64_overlap(record_box(t.tri64A, ca & ~kLeafBit), record_box(t.tri64B, cb & ~kLeafBit)) ? 2u : 0u;
-    return 1u;
+    return box64_overlap(record_box(t.tri64A, pr.x & ~kLeafBit), record_box(t.tri64B, pr.y & ~kLeafBit));
 }
 
-__device__ __forceinline__ Expansion expand_pair(const TraverseArgs &t, uint2 pr, bool valid)
+__device__ __forceinline__ uint64_t cand_key(uint2 pr)
 {
-    Expansion x = {0, 0, 0, 0, 0, 0};
-    if (!valid)
-        return x;
+    return ((uint64_t)(pr.x & ~kLeafBit) << 32) | (pr.y & ~kLeafBit);
+}
+
+// Expansion of one node pair: child pair s = 2u + v (u over A's children, v
+// over B's) goes on when its FP32 boxes overlap (bit s of next).  A pair of
+// leaves has no children: cand says whether it is a candidate.  Every field is
+// a named register, so nothing lands in scratch memory.
+struct Expansion {
+    uint32_t a0, a1, b0, b1;
+    uint32_t next;
+    bool cand;
+};
+
+__device__ __forceinline__ void expand_nodes(const TraverseArgs &t, uint2 pr, Expansion &x)
+{
     const Kids ka = kids_of(t.nodesA, t.boxA, pr.x);
     const Kids kb = kids_of(t.nodesB, t.boxB, pr.y);
     x.a0 = ka.c0;
     x.a1 = ka.c1;
     x.b0 = kb.c0;
     x.b1 = kb.c1;
-    const uint32_t r0 = expand_one(t, ka.c0, kb.c0, ka.b0, kb.b0);
-    const uint32_t r1 = kb.two ? expand_one(t, ka.c0, kb.c1, ka.b0, kb.b1) : 0u;
-    const uint32_t r2 = ka.two ? expand_one(t, ka.c1, kb.c0, ka.b1, kb.b0) : 0u;
-    const uint32_t r3 = ka.two && kb.two ? expand_one(t, ka.c1, kb.c1, ka.b1, kb.b1) : 0u;
-    x.next = (r0 == 1u ? 1u : 0u) | (r1 == 1u ? 2u : 0u) | (r2 == 1u ? 4u : 0u) | (r3 == 1u ? 8u : 0u);
-    x.cand = (r0 == 2u ? 1u : 0u) | (r1 == 2u ? 2u : 0u) | (r2 == 2u ? 4u : 0u) | (r3 == 2u ? 8u : 0u);
+    x.next = (fbox_overlap(ka.b0, kb.b0) ? 1u : 0u) | (kb.two && fbox_overlap(ka.b0, kb.b1) ? 2u : 0u) |
+             (ka.two && fbox_overlap(ka.b1, kb.b0) ? 4u : 0u) |
+             (ka.two && kb.two && fbox_overlap(ka.b1, kb.b1) ? 8u : 0u);
+}
+
+__device__ __forceinline__ Expansion expand_pair(const TraverseArgs &t, uint2 pr, bool valid)
+{
+    Expansion x = {0, 0, 0, 0, 0, false};
+    if (!valid)
+        return x;
+    if (both_leaves(pr))
+        x.cand = leaves_overlap(t, pr);
+    else
+        expand_nodes(t, pr, x);
     return x;
 }
 
@@ -137,10 +123,51 @@ __device__ __forceinline__ uint2 slot_pair(const Expansion &x, int s)
     return make_uint2(s < 2 ? x.a0 : x.a1, (s & 1) ? x.b1 : x.b0);
 }
 
-__device__ __forceinline__ uint64_t cand_key(const Expansion &x, int s)
+// The wave's child pairs in slot order, lane by lane within a slot: one ballot
+// per slot (counts by shuffled prefix sums took six dependent LDS permutes).
+struct SlotMasks {
+    unsigned long long m[4];
+    __device__ __forceinline__ uint32_t total() const
+    {
+        return (uint32_t)(__popcll(m[0]) + __popcll(m[1]) + __popcll(m[2]) + __popcll(m[3]));
+    }
+};
+
+__device__ __forceinline__ SlotMasks slot_masks(uint32_t next)
 {
-    const uint2 p = slot_pair(x, s);
-    return ((uint64_t)(p.x & ~kLeafBit) << 32) | (p.y & ~kLeafBit);
+    return {{__ballot(next & 1u), __ballot(next & 2u), __ballot(next & 4u), __ballot(next & 8u)}};
+}
+
+__device__ __forceinline__ unsigned long long lanes_below()
+{
+    return (1ull << (threadIdx.x & 63)) - 1ull;
+}
+
+// writes the wave's child pairs of `next` to out[base ...), those below cap
+__device__ __forceinline__ void put_slots(const Expansion &x, uint32_t next, const SlotMasks &sm, uint2 *out,
+                                          uint32_t base, uint32_t cap)
+{
+    const unsigned long long below = lanes_below();
+#pragma unroll
+    for (int sl = 0; sl < 4; ++sl) {
+        const uint32_t pos = base + (uint32_t)__popcll(sm.m[sl] & below);
+        if ((next >> sl & 1u) && pos < cap)
+            out[pos] = slot_pair(x, sl);
+        base += (uint32_t)__popcll(sm.m[sl]);
+    }
+}
+
+// first of `total` slots of a queue, taken by one lane of the wave (every lane
+// gets it); past the capacity the overflow flag is raised
+__device__ __forceinline__ uint32_t wave_take(uint32_t total, uint32_t *counter, uint32_t cap, uint32_t *overflow)
+{
+    uint32_t base = 0;
+    if ((threadIdx.x & 63) == 0 && total) {
+        base = atomicAdd(counter, total);
+        if (base + total > cap)
+            atomicOr(overflow, 1u);
+    }
+    return __shfl(base, 0, 64);
 }
 
 // Workgroup size of the grid-wide breadth-first levels (the launches' grids
@@ -148,51 +175,16 @@ __device__ __forceinline__ uint64_t cand_key(const Expansion &x, int s)
 constexpr int kExpandThreads = 256;
 constexpr int kExpandWaves = kExpandThreads / 64;
 
-// Offsets of this lane's na next-frontier pairs and nb candidates in their
-// queues, for a workgroup of kExpandThreads lanes: the two counts travel
-// packed in one 32-bit prefix sum (at most 4 each per lane, so a workgroup's
-// totals stay below 2^16), and the workgroup takes one atomic per queue.
-// Every lane of the workgroup calls it.
-__device__ __forceinline__ uint2 group_reserve2(uint32_t na, uint32_t nb, uint32_t *countA, uint32_t capA,
-                                                uint32_t *countB, uint32_t capB, uint32_t *overflow)
-{
-    __shared__ uint32_t s_wave[kExpandWaves], s_pre[kExpandWaves], s_base[2];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const uint32_t mine = na | nb << 16;
-    uint32_t incl = mine;
-    for (int off = 1; off < 64; off <<= 1) {
-        const uint32_t v = __shfl_up(incl, off, 64);
-        if (lane >= off)
-            incl += v;
-    }
-    if (lane == 63)
-        s_wave[wave] = incl;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        uint32_t run = 0;
-        for (int w = 0; w < kExpandWaves; ++w) {
-            s_pre[w] = run;
-            run += s_wave[w];
-        }
-        const uint32_t ta = run & 0xffffu, tb = run >> 16;
-        const uint32_t ba = ta ? atomicAdd(countA, ta) : 0u, bb = tb ? atomicAdd(countB, tb) : 0u;
-        if ((ta && ba + ta > capA) || (tb && bb + tb > capB))
-            atomicOr(overflow, 1u);
-        s_base[0] = ba;
-        s_base[1] = bb;
-    }
-    __syncthreads();
-    const uint32_t off = s_pre[wave] + incl - mine;
-    return make_uint2(s_base[0] + (off & 0xffffu), s_base[1] + (off >> 16));
-}
-
 // One breadth-first level over the whole grid: frontier `in` (inCount pairs)
-// to `out`, candidates appended.  Workgroups of kExpandThreads lanes.
+// to `out`, candidates appended.  Workgroups of kExpandThreads lanes, which
+// take one atomic per queue.
 __device__ __forceinline__ void expand_level(const TraverseArgs &t, const uint2 *__restrict__ in,
                                              const uint32_t *__restrict__ inCount, uint2 *__restrict__ out,
                                              uint32_t *outCount, uint32_t outCap, uint64_t *__restrict__ cand,
                                              uint32_t *candCount, uint32_t candCap, uint32_t *overflow)
 {
+    __shared__ uint32_t s_count[2][kExpandWaves], s_at[2][kExpandWaves];  // next pairs, candidates
+    const int wave = threadIdx.x >> 6;
     // both frontier buffers hold outCap pairs; a count past it has already
     // raised `overflow` and the whole search is repeated with larger queues
     const uint32_t n = *inCount < outCap ? *inCount : outCap;
@@ -200,24 +192,35 @@ __device__ __forceinline__ void expand_level(const TraverseArgs &t, const uint2 
     for (uint32_t base = blockIdx.x * kExpandThreads; base < n; base += stride) {  // uniform over the workgroup
         const uint32_t i = base + threadIdx.x;
         const bool valid = i < n;
-        const Expansion x = expand_pair(t, valid ? in[i] : make_uint2(0, 0), valid);
-        const uint2 o = group_reserve2(__popc(x.next), __popc(x.cand), outCount, outCap, candCount, candCap,
-                                       overflow);
-        const uint32_t on = o.x, oc = o.y;
-        uint32_t kn = 0, kc = 0;
-#pragma unroll
-        for (int sl = 0; sl < 4; ++sl) {
-            if ((x.next >> sl) & 1u) {
-                if (on + kn < outCap)
-                    out[on + kn] = slot_pair(x, sl);
-                ++kn;
-            }
-            if ((x.cand >> sl) & 1u) {
-                if (oc + kc < candCap)
-                    cand[oc + kc] = cand_key(x, sl);
-                ++kc;
+        const uint2 pr = valid ? in[i] : make_uint2(0, 0);
+        const Expansion x = expand_pair(t, pr, valid);
+        const SlotMasks sm = slot_masks(x.next);
+        const unsigned long long cm = __ballot(x.cand);
+        if ((threadIdx.x & 63) == 0) {
+            s_count[0][wave] = sm.total();
+            s_count[1][wave] = (uint32_t)__popcll(cm);
+        }
+        __syncthreads();
+        if (threadIdx.x < 2) {
+            const uint32_t *cnt = s_count[threadIdx.x];
+            uint32_t total = 0;
+            for (int w = 0; w < kExpandWaves; ++w)
+                total += cnt[w];
+            uint32_t at = total ? atomicAdd(threadIdx.x ? candCount : outCount, total) : 0u;
+            if (total && at + total > (threadIdx.x ? candCap : outCap))
+                atomicOr(overflow, 1u);
+            for (int w = 0; w < kExpandWaves; ++w) {
+                s_at[threadIdx.x][w] = at;
+                at += cnt[w];
             }
         }
+        __syncthreads();
+        const uint32_t on = s_at[0][wave];
+        uint32_t oc = s_at[1][wave];
+        put_slots(x, x.next, sm, out, on, outCap);
+        oc += (uint32_t)__popcll(cm & lanes_below());
+        if (x.cand && oc < candCap)
+            cand[oc] = cand_key(pr);
     }
 }
 
@@ -257,38 +260,24 @@ __global__ __launch_bounds__(1024) void k_search_top(TraverseArgs t, uint2 *__re
         for (uint32_t b = 0; b < nIn; b += 1024) {
             const uint32_t i = b + threadIdx.x;
             const bool valid = i < nIn;
-            const Expansion x = expand_pair(t, valid ? in[i] : make_uint2(0, 0), valid);
-            // next-frontier slots: a wave prefix, one LDS atomic per wave
-            const uint32_t nn = __popc(x.next);
-            uint32_t incl = nn;
-            for (int off = 1; off < 64; off <<= 1) {
-                const uint32_t v = __shfl_up(incl, off, 64);
-                if (lane >= off)
-                    incl += v;
-            }
-            const uint32_t total = __shfl(incl, 63, 64);
-            uint32_t wbase = 0;
-            if (lane == 63 && total)
-                wbase = atomicAdd(&s_next, total);
-            wbase = __shfl(wbase, 63, 64);
-            const uint32_t on = wbase + incl - nn;
-            if (total && wbase + total > fcap && lane == 0)
+            const uint2 pr = valid ? in[i] : make_uint2(0, 0);
+            const Expansion x = expand_pair(t, pr, valid);
+            // next-frontier slots: one LDS atomic per wave
+            const SlotMasks sm = slot_masks(x.next);
+            const uint32_t total = sm.total();
+            uint32_t on = 0;
+            if (lane == 0 && total)
+                on = atomicAdd(&s_next, total);
+            on = __shfl(on, 0, 64);
+            if (total && on + total > fcap && lane == 0)
                 atomicOr(overflow, 1u);
-            uint32_t wb;
-            const uint32_t oc = wave_reserve(__popc(x.cand), candCount, candCap, overflow, wb);
-            uint32_t kn = 0, kc = 0;
-#pragma unroll
-            for (int sl = 0; sl < 4; ++sl) {
-                if ((x.next >> sl) & 1u) {
-                    if (on + kn < fcap)
-                        out[on + kn] = slot_pair(x, sl);
-                    ++kn;
-                }
-                if ((x.cand >> sl) & 1u) {
-                    if (oc + kc < candCap)
-                        cand[oc + kc] = cand_key(x, sl);
-                    ++kc;
-                }
+            put_slots(x, x.next, sm, out, on, fcap);
+            const unsigned long long cm = __ballot(x.cand);
+            if (cm) {
+                const uint32_t oc = wave_take((uint32_t)__popcll(cm), candCount, candCap, overflow) +
+                                    (uint32_t)__popcll(cm & lanes_below());
+                if (x.cand && oc < candCap)
+                    cand[oc] = cand_key(pr);
             }
         }
         // the next level reads this one's output: workgroup-scope ordering of
@@ -323,14 +312,20 @@ __global__ __launch_bounds__(kExpandThreads) void k_expand_at(TraverseArgs t, ui
 
 // Persistent depth-first stage.  One wave per workgroup keeps a stack of node
 // pairs in LDS (spilling to a per-wave region of global memory when full).
-// Each step pops up to 64 pairs (one per lane), expands them as k_expand
-// does, appends candidates with one atomic per wave, and pushes the surviving
-// child pairs back with a 64-lane prefix sum.  An empty wave claims the next
-// few seed pairs (the breadth-first frontier) from a shared counter.  Waves never wait for
-// each other: a wave leaves when its own stacks are empty and no seed is left.
-// Spill overflow or the iteration cap raise `overflow` (the host then repeats
-// the search breadth-first), so nothing is dropped silently.
+// Each step pops up to 64 pairs (one per lane), expands them and pushes the
+// surviving child pairs back.  Pairs of leaves are set aside in LDS until 64 of
+// them fill a wave for the exact test, so a step waits for two 64-B node loads
+// and nothing else; candidates are set aside too and leave 64 or more at a time
+// with one atomic.  (The tests and the atomic inside the step: 100 us at the
+// 1,310,720-triangle pair; so: see launch_search_levels.)  An empty wave claims
+// the next few seed pairs (the breadth-first frontier) from a shared counter.
+// Waves never wait for each other: a wave leaves when its own lists are empty
+// and no seed is left.  Spill overflow or the iteration cap raise `overflow`
+// (the host then repeats the search breadth-first), so nothing is dropped
+// silently.
 constexpr int kDfsLds = 1024;
+constexpr int kDfsLeaves = 64 + 4 * 64;  // one step adds at most 256 to fewer than 64
+constexpr int kDfsCands = 128;           // one test adds at most 64 to fewer than 64
 constexpr uint32_t kDfsMaxIter = 1u << 24;
 
 // With levelBase, the seeds are the frontier of level min(*levelBase +
@@ -344,7 +339,8 @@ __global__ __launch_bounds__(64) void k_traverse_dfs(TraverseArgs t, const uint2
                                                      uint32_t spillPerWave, uint64_t *__restrict__ cand,
                                                      uint32_t *candCount, uint32_t candCap, uint32_t *overflow)
 {
-    __shared__ uint2 s_stack[kDfsLds];
+    __shared__ uint2 s_stack[kDfsLds], s_leaf[kDfsLeaves];
+    __shared__ uint64_t s_cand[kDfsCands];
     const int lane = threadIdx.x;
     if (levelBase) {
         uint32_t level = *levelBase + levelAdd;
@@ -357,10 +353,42 @@ __global__ __launch_bounds__(64) void k_traverse_dfs(TraverseArgs t, const uint2
     uint32_t grab = nseed / gridDim.x;
     grab = grab < 1u ? 1u : (grab > 64u ? 64u : grab);
     uint2 *gstack = spill + (size_t)blockIdx.x * spillPerWave;
-    int sp = 0;          // LDS entries (same value in every lane)
-    uint32_t gsp = 0;    // spilled entries (same value in every lane)
+    int sp = 0;          // LDS entries (same value in every lane, as the rest)
+    uint32_t gsp = 0;    // spilled entries
+    uint32_t nleaf = 0, ncand = 0;
+    bool seeds_left = true;
+    const unsigned long long below = lanes_below();
+    auto flush = [&]() {
+        const uint32_t base = wave_take(ncand, candCount, candCap, overflow);
+        for (uint32_t k = lane; k < ncand; k += 64)
+            if (base + k < candCap)
+                cand[base + k] = s_cand[k];
+        ncand = 0;
+        __syncthreads();
+    };
+    auto test_leaves = [&]() {  // up to 64 of them
+        const uint32_t m = nleaf < 64u ? nleaf : 64u;
+        nleaf -= m;
+        bool hit = false;
+        uint2 pr = make_uint2(0, 0);
+        if ((uint32_t)lane < m) {
+            pr = s_leaf[nleaf + lane];
+            hit = leaves_overlap(t, pr);
+        }
+        const unsigned long long hm = __ballot(hit);
+        if (hit)
+            s_cand[ncand + (uint32_t)__popcll(hm & below)] = cand_key(pr);
+        ncand += (uint32_t)__popcll(hm);
+        __syncthreads();
+        if (ncand >= 64u)
+            flush();
+    };
     uint32_t iter = 0;
     for (; iter < kDfsMaxIter; ++iter) {
+        if (nleaf >= 64u) {
+            test_leaves();
+            continue;
+        }
         if (sp == 0 && gsp > 0) {
             const uint32_t m = gsp < (uint32_t)(kDfsLds / 2) ? gsp : (uint32_t)(kDfsLds / 2);
             for (uint32_t k = lane; k < m; k += 64)
@@ -369,18 +397,25 @@ __global__ __launch_bounds__(64) void k_traverse_dfs(TraverseArgs t, const uint2
             sp = (int)m;
             __syncthreads();
         }
-        if (sp == 0) {
+        if (sp == 0 && seeds_left) {
             uint32_t start = 0;
             if (lane == 0)
                 start = atomicAdd(head, grab);
             start = __shfl(start, 0, 64);
-            if (start >= nseed)
+            seeds_left = start < nseed;
+            if (seeds_left) {
+                const uint32_t m = nseed - start < grab ? nseed - start : grab;
+                if ((uint32_t)lane < m)
+                    s_stack[lane] = seeds[start + lane];
+                sp = (int)m;
+                __syncthreads();
+            }
+        }
+        if (sp == 0) {
+            if (nleaf == 0)
                 break;
-            const uint32_t m = nseed - start < grab ? nseed - start : grab;
-            if ((uint32_t)lane < m)
-                s_stack[lane] = seeds[start + lane];
-            sp = (int)m;
-            __syncthreads();
+            test_leaves();
+            continue;
         }
         const int take = sp < 64 ? sp : 64;
         const bool valid = lane < take;
@@ -389,40 +424,31 @@ __global__ __launch_bounds__(64) void k_traverse_dfs(TraverseArgs t, const uint2
             pr = s_stack[sp - take + lane];
         sp -= take;
         __syncthreads();
-        const Expansion x = expand_pair(t, pr, valid);
-        const uint32_t nn = __popc(x.next);
-        uint32_t wb;
-        const uint32_t oc = wave_reserve(__popc(x.cand), candCount, candCap, overflow, wb);
-        uint32_t kc = 0;
-#pragma unroll
-        for (int sl = 0; sl < 4; ++sl)
-            if ((x.cand >> sl) & 1u) {
-                if (oc + kc < candCap)
-                    cand[oc + kc] = cand_key(x, sl);
-                ++kc;
+        Expansion x = {0, 0, 0, 0, 0, false};
+        if (valid) {
+            if (both_leaves(pr)) {  // a seed of two leaves: on to the tests
+                x.a0 = pr.x;
+                x.b0 = pr.y;
+                x.next = 1u;
+            } else {
+                expand_nodes(t, pr, x);
             }
-        // push children: LDS when they fit, else the wave's spill region
-        uint32_t incl = nn;
-        for (int off = 1; off < 64; off <<= 1) {
-            const uint32_t v = __shfl_up(incl, off, 64);
-            if (lane >= off)
-                incl += v;
         }
-        const uint32_t total = __shfl(incl, 63, 64);
-        const uint32_t mine = incl - nn;
+        // pairs of leaves apart from the others
+        const uint32_t la0 = x.a0 >> 31, la1 = x.a1 >> 31, lb0 = x.b0 >> 31, lb1 = x.b1 >> 31;
+        const uint32_t leaves = x.next & (la0 & lb0 | (la0 & lb1) << 1 | (la1 & lb0) << 2 | (la1 & lb1) << 3);
+        const uint32_t inner = x.next & ~leaves;
+        const SlotMasks lm = slot_masks(leaves);
+        put_slots(x, leaves, lm, s_leaf, nleaf, (uint32_t)kDfsLeaves);
+        nleaf += lm.total();
+        // push the others: LDS when they fit, else the wave's spill region
+        const SlotMasks im = slot_masks(inner);
+        const uint32_t total = im.total();
         if (sp + (int)total <= kDfsLds) {
-            uint32_t kn = 0;
-#pragma unroll
-            for (int sl = 0; sl < 4; ++sl)
-                if ((x.next >> sl) & 1u)
-                    s_stack[sp + mine + kn++] = slot_pair(x, sl);
+            put_slots(x, inner, im, s_stack, (uint32_t)sp, (uint32_t)kDfsLds);
             sp += (int)total;
         } else if (gsp + total <= spillPerWave) {
-            uint32_t kn = 0;
-#pragma unroll
-            for (int sl = 0; sl < 4; ++sl)
-                if ((x.next >> sl) & 1u)
-                    gstack[gsp + mine + kn++] = slot_pair(x, sl);
+            put_slots(x, inner, im, gstack, gsp, spillPerWave);
             gsp += total;
         } else {
             if (lane == 0)
@@ -431,6 +457,8 @@ __global__ __launch_bounds__(64) void k_traverse_dfs(TraverseArgs t, const uint2
         }
         __syncthreads();
     }
+    if (ncand)
+        flush();
     if (iter == kDfsMaxIter && lane == 0)
         atomicOr(overflow, 8u);
 }
