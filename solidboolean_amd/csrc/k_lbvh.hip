@@ -38,7 +38,6 @@ __device__ __forceinline__ int delta(const uint64_t *__restrict__ codes, int n, 
 // The tree is built and refit bottom-up in tiles of kTreeTile sorted leaves, one
 // workgroup each; a node whose leaf range crosses a tile boundary is a "top"
 // node, made by k_top_nodes.
-constexpr int kTreeTile = 1024;  // leaves per workgroup, one per lane
 constexpr uint16_t kNoSplit = 0xffffu;
 
 __device__ __forceinline__ void write_root(float *rootBox, float4 lo, float4 hi)
@@ -56,6 +55,17 @@ __device__ __forceinline__ void put6(float *dst, const float v[6])
 #pragma unroll
     for (int k = 0; k < 6; ++k)
         dst[k] = v[k];
+}
+
+// one more piece of the workgroup's tile in the list for the pair search
+__device__ __forceinline__ void list_piece(const TreePieces &out, uint32_t *n, uint32_t ref, const float b[6])
+{
+    if (!out.count)
+        return;
+    const uint32_t k = atomicAdd(n, 1u);
+    float4 *dst = out.piece + 2 * ((size_t)blockIdx.x * kTilePieces + k);
+    dst[0] = make_float4(b[0], b[1], b[2], __uint_as_float(ref));
+    dst[1] = make_float4(b[3], b[4], b[5], 0.0f);
 }
 
 // Stage 1: the radix tree of a tile's leaves, bottom-up.  The tree is fixed by
@@ -90,7 +100,7 @@ __global__ __launch_bounds__(kTreeTile) void k_tree_tiles(const K *__restrict__ 
                                                           BNode *__restrict__ nodes, uint32_t *__restrict__ topList,
                                                           uint32_t *topCount, float *__restrict__ prefix,
                                                           float *__restrict__ suffix, float *__restrict__ piece,
-                                                          float *__restrict__ tileBox, float *rootBox)
+                                                          float *__restrict__ tileBox, TreePieces out, float *rootBox)
 {
     __shared__ float s_box[kTreeTile][2][6];        // per split: the children's boxes,
     __shared__ uint32_t s_ref[kTreeTile][2];        // references,
@@ -102,14 +112,14 @@ __global__ __launch_bounds__(kTreeTile) void k_tree_tiles(const K *__restrict__ 
     __shared__ int8_t s_delta[kTreeTile + 1];       // prefix length of (pos - 1, pos)
     __shared__ uint8_t s_taken[kTreeTile], s_start[kTreeTile], s_stop[kTreeTile];
     __shared__ float s_wave[kTreeTile / 64][6];
-    __shared__ uint32_t s_ntop, s_top0;
+    __shared__ uint32_t s_ntop, s_top0, s_npiece;
     constexpr uint32_t kRightCame = 0x100u;
     const int tile0 = blockIdx.x * kTreeTile;
     const int tile1 = min(tile0 + kTreeTile, n);
     const int me = threadIdx.x, pos = tile0 + me;
     const bool valid = pos < tile1;
     if (me == 0)
-        s_ntop = 0;
+        s_ntop = s_npiece = 0;
     s_flag[me] = 0;
     s_taken[me] = s_start[me] = s_stop[me] = 0;
     if (valid)
@@ -145,12 +155,16 @@ __global__ __launch_bounds__(kTreeTile) void k_tree_tiles(const K *__restrict__ 
             }
             if (dl < 0 && dr < 0) {  // the whole tree
                 write_root(rootBox, wl, wh);
+                const float b[6] = {wl.x, wl.y, wl.z, wh.x, wh.y, wh.z};
+                put6(tileBox, b);
+                list_piece(out, &s_npiece, ref, b);
                 break;
             }
             const int split = left ? hi : lo - 1;
             if (split < 0 || tile0 + split + 1 >= tile1) {  // its sibling lies in the next tile
                 const float b[6] = {wl.x, wl.y, wl.z, wh.x, wh.y, wh.z};
                 put6(piece + 6 * (size_t)(tile0 + lo), b);
+                list_piece(out, &s_npiece, ref, b);
                 s_start[lo] = 1;
                 s_stop[hi] = 1;
                 break;
@@ -197,11 +211,15 @@ __global__ __launch_bounds__(kTreeTile) void k_tree_tiles(const K *__restrict__ 
         const int side = came & kRightCame ? 1 : 0;
         const int lo = side ? me + 1 : s_far[me][0], hi = side ? s_far[me][1] : me;
         put6(piece + 6 * (size_t)(tile0 + lo), s_box[me][side]);
+        list_piece(out, &s_npiece, s_ref[me][side], s_box[me][side]);
         s_start[lo] = 1;
         s_stop[hi] = 1;
     }
-    if (gridDim.x == 1)  // one tile: no top node
+    if (gridDim.x == 1) {  // one tile: no top node, the root its only piece
+        if (me == 0 && out.count)
+            out.count[0] = 1;
         return;
+    }
     // indices no node of the tile took: slots from LDS, one global reservation
     // per tile (one per wave held the kernel to the rate of one counter: 215
     // us at 3.0 M leaves)
@@ -234,6 +252,8 @@ __global__ __launch_bounds__(kTreeTile) void k_tree_tiles(const K *__restrict__ 
     __syncthreads();
     if (top)
         topList[s_top0 + slot] = (uint32_t)pos;
+    if (me == 0 && out.count)
+        out.count[blockIdx.x] = s_npiece;
     for (int w = 0; w < kTreeTile / 64; ++w) {
         if (w < wave)
 #pragma unroll
@@ -443,9 +463,13 @@ static int table_levels(uint32_t ntiles)
     return L;
 }
 
+uint32_t tree_tiles(uint32_t n) { return (n + kTreeTile - 1) / kTreeTile; }
+
+float *tree_tile_boxes(float *scratch, uint32_t n) { return scratch + 18 * (size_t)n; }
+
 size_t tree_scratch_floats(uint32_t n)
 {
-    const uint32_t ntiles = (n + kTreeTile - 1) / kTreeTile;
+    const uint32_t ntiles = tree_tiles(n);
     return 18 * (size_t)n + 6 * (size_t)ntiles * table_levels(ntiles) + 6;
 }
 
@@ -453,15 +477,15 @@ size_t tree_scratch_floats(uint32_t n)
 // scratch: tree_scratch_floats(n) floats (prefix, suffix, pieces, tile table)
 template <typename K>
 static void tree(const K *codes, const uint32_t *ids, const float *box32, uint32_t n, BNode *nodes, uint32_t *work,
-                 float *scratch, float *rootBox, hipStream_t s)
+                 float *scratch, TreePieces pieces, float *rootBox, hipStream_t s)
 {
     if (n < 2)
         return;
-    const uint32_t ntiles = (n + kTreeTile - 1) / kTreeTile;
+    const uint32_t ntiles = tree_tiles(n);
     float *prefix = scratch, *suffix = prefix + 6 * (size_t)n, *piece = suffix + 6 * (size_t)n;
-    float *table = piece + 6 * (size_t)n;
+    float *table = tree_tile_boxes(scratch, n);
     hipLaunchKernelGGL(k_tree_tiles<K>, dim3(ntiles), dim3(kTreeTile), 0, s, codes, ids, box32, (int)n, nodes, work + 1,
-                       work, prefix, suffix, piece, table, rootBox);
+                       work, prefix, suffix, piece, table, pieces, rootBox);
     if (ntiles < 2)
         return;
     const size_t lds = ntiles <= kLdsTiles ? sizeof(float) * 6 * ntiles : 0;
@@ -475,16 +499,16 @@ static void tree(const K *codes, const uint32_t *ids, const float *box32, uint32
 }
 
 void launch_tree(const uint32_t *codes, const uint32_t *ids, const float *box32, uint32_t n, BNode *nodes,
-                 uint32_t *work, float *scratch, float *rootBox, hipStream_t s)
+                 uint32_t *work, float *scratch, TreePieces pieces, float *rootBox, hipStream_t s)
 {
-    tree(codes, ids, box32, n, nodes, work, scratch, rootBox, s);
+    tree(codes, ids, box32, n, nodes, work, scratch, pieces, rootBox, s);
 }
 
 void launch_tree64(const uint64_t *codes, const uint32_t *ids, const float *box32, uint32_t n, BNode *nodes,
                    uint32_t *work, float *scratch, float *rootBox, hipStream_t s)
 {
     launch_fill_u32(work, 0u, 1, s);
-    tree(codes, ids, box32, n, nodes, work, scratch, rootBox, s);
+    tree(codes, ids, box32, n, nodes, work, scratch, TreePieces{nullptr, nullptr}, rootBox, s);
 }
 
 }  // namespace sbg

@@ -232,6 +232,91 @@ __global__ __launch_bounds__(kExpandThreads) void k_expand(TraverseArgs t, const
     expand_level(t, in, inCount, out, outCount, outCap, cand, candCount, candCap, overflow);
 }
 
+// ---- first frontier from the trees' tiles --------------------------------------
+// The levels from two roots down to subtrees of a tile's size hold few pairs
+// and cost a launch or a workgroup's round each.  Instead every pair of tiles
+// is tested by its boxes at once (1,280 x 1,280 at the 1,310,720-triangle
+// pair), one workgroup per tile of A and 256 tiles of B, and the pieces of the
+// tiles that overlap give the frontier, some tens of tests per pair of tiles.
+// A pass from the roots took 730 us against 637 at the 81,920-triangle pair,
+// 973 against 879 at two 393,132-triangle cubes, 1,706 against 1,681 at
+// 1,310,720 triangles.
+constexpr int kSearchOut = 1024;  // frontier pairs a workgroup gathers before it takes slots
+
+__global__ __launch_bounds__(256) void k_search_tiles(TileSet a, TileSet b, uint2 *__restrict__ frontier,
+                                                      uint32_t *count, uint32_t cap, uint32_t *overflow)
+{
+    __shared__ uint32_t s_tile[256], s_ntile, s_nout, s_base;
+    __shared__ float4 s_piece[2 * kTilePieces];
+    __shared__ uint2 s_out[kSearchOut];
+    const uint32_t ta = blockIdx.x, tb0 = blockIdx.y * 256 + threadIdx.x;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (threadIdx.x == 0)
+        s_ntile = s_nout = 0;
+    __syncthreads();
+    if (tb0 < b.ntiles) {
+        const float *p = a.box + 6 * (size_t)ta, *q = b.box + 6 * (size_t)tb0;
+        if (fbox_overlap({p[0], p[1], p[2], p[3], p[4], p[5]}, {q[0], q[1], q[2], q[3], q[4], q[5]}))
+            s_tile[atomicAdd(&s_ntile, 1u)] = tb0;
+    }
+    __syncthreads();
+    const uint32_t ntile = s_ntile;
+    if (ntile == 0)
+        return;
+    const uint32_t na = a.pieces.count[ta];
+    for (uint32_t k = threadIdx.x; k < 2 * na; k += 256)
+        s_piece[k] = a.pieces.piece[2 * (size_t)ta * kTilePieces + k];
+    __syncthreads();
+    for (uint32_t k = wave; k < ntile; k += 4) {
+        const uint32_t tb = s_tile[k], nb = b.pieces.count[tb];
+        const float4 *pb = b.pieces.piece + 2 * (size_t)tb * kTilePieces;
+        for (uint32_t j0 = 0; j0 < na * nb; j0 += 64) {
+            const uint32_t j = j0 + lane, ia = j / nb, ib = j - ia * nb;
+            bool hit = false;
+            uint2 pr = make_uint2(0, 0);
+            if (ia < na) {
+                const float4 al = s_piece[2 * ia], ah = s_piece[2 * ia + 1], bl = pb[2 * ib], bh = pb[2 * ib + 1];
+                hit = fbox_overlap({al.x, al.y, al.z, ah.x, ah.y, ah.z}, {bl.x, bl.y, bl.z, bh.x, bh.y, bh.z});
+                pr = make_uint2(__float_as_uint(al.w), __float_as_uint(bl.w));
+            }
+            const unsigned long long m = __ballot(hit);
+            if (!m)
+                continue;
+            uint32_t at = 0;
+            if (lane == 0)
+                at = atomicAdd(&s_nout, (uint32_t)__popcll(m));
+            at = __shfl(at, 0, 64) + (uint32_t)__popcll(m & lanes_below());
+            if (hit && at < (uint32_t)kSearchOut) {
+                s_out[at] = pr;
+            } else if (hit) {  // more than a workgroup gathers: a slot of its own
+                const uint32_t slot = atomicAdd(count, 1u);
+                if (slot < cap)
+                    frontier[slot] = pr;
+                else
+                    atomicOr(overflow, 1u);
+            }
+        }
+    }
+    __syncthreads();
+    const uint32_t n = s_nout < (uint32_t)kSearchOut ? s_nout : (uint32_t)kSearchOut;
+    if (threadIdx.x == 0 && n) {
+        s_base = atomicAdd(count, n);
+        if (s_base + n > cap)
+            atomicOr(overflow, 1u);
+    }
+    __syncthreads();
+    for (uint32_t k = threadIdx.x; k < n; k += 256)
+        if (s_base + k < cap)
+            frontier[s_base + k] = s_out[k];
+}
+
+void launch_search_tiles(const TileSet &a, const TileSet &b, uint2 *frontier, uint32_t *count, uint32_t cap,
+                         uint32_t *overflow, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_search_tiles, dim3(a.ntiles, (b.ntiles + 255) / 256), dim3(256), 0, s, a, b, frontier, count,
+                       cap, overflow);
+}
+
 // ---- top of the search in one workgroup -------------------------------------
 // The first levels of a tree-vs-tree search hold a handful of node pairs, and a
 // grid-wide launch per level costs a launch's latency for a few lanes of work
@@ -293,31 +378,14 @@ __global__ __launch_bounds__(1024) void k_search_top(TraverseArgs t, uint2 *__re
         *levelOut = (uint32_t)level;
 }
 
-// Breadth-first level *topLevel + j over the whole grid, or nothing when that
-// is at or past lastLevel (the launches after the top kernel are queued before
-// it is known where it stopped).
-__global__ __launch_bounds__(kExpandThreads) void k_expand_at(TraverseArgs t, uint2 *__restrict__ front0,
-                                                   uint2 *__restrict__ front1, uint32_t *__restrict__ cnt,
-                                                   const uint32_t *__restrict__ topLevel, uint32_t j,
-                                                   uint32_t lastLevel, uint32_t fcap, uint64_t *__restrict__ cand,
-                                                   uint32_t *candCount, uint32_t candCap, uint32_t *overflow)
-{
-    const uint32_t level = *topLevel + j;
-    if (level >= lastLevel)
-        return;
-    const uint2 *in = (level & 1) ? front1 : front0;
-    uint2 *out = (level & 1) ? front0 : front1;
-    expand_level(t, in, cnt + level, out, cnt + level + 1, fcap, cand, candCount, candCap, overflow);
-}
-
 // Persistent depth-first stage.  One wave per workgroup keeps a stack of node
 // pairs in LDS (spilling to a per-wave region of global memory when full).
 // Each step pops up to 64 pairs (one per lane), expands them and pushes the
 // surviving child pairs back.  Pairs of leaves are set aside in LDS until 64 of
 // them fill a wave for the exact test, so a step waits for two 64-B node loads
 // and nothing else; candidates are set aside too and leave 64 or more at a time
-// with one atomic.  (The tests and the atomic inside the step: 100 us at the
-// 1,310,720-triangle pair; so: see launch_search_levels.)  An empty wave claims
+// with one atomic (47 us at the 1,310,720-triangle pair, 100 with the tests and
+// the atomic inside the step).  An empty wave claims
 // the next few seed pairs (the breadth-first frontier) from a shared counter.
 // Waves never wait for each other: a wave leaves when its own lists are empty
 // and no seed is left.  Spill overflow or the iteration cap raise `overflow`
@@ -328,14 +396,14 @@ constexpr int kDfsLeaves = 64 + 4 * 64;  // one step adds at most 256 to fewer t
 constexpr int kDfsCands = 128;           // one test adds at most 64 to fewer than 64
 constexpr uint32_t kDfsMaxIter = 1u << 24;
 
-// With levelBase, the seeds are the frontier of level min(*levelBase +
-// levelAdd, lastLevel): `seeds` / `seedsAlt` are the even / odd levels'
-// frontier buffers and seedCount the per-level counts.
+// With levelBase, the seeds are the frontier of level *levelBase: `seeds` /
+// `seedsAlt` are the even / odd levels' frontier buffers and seedCount the
+// per-level counts.
 __global__ __launch_bounds__(64) void k_traverse_dfs(TraverseArgs t, const uint2 *__restrict__ seeds,
                                                      const uint2 *__restrict__ seedsAlt,
                                                      const uint32_t *__restrict__ seedCount, uint32_t seedCap,
-                                                     const uint32_t *__restrict__ levelBase, uint32_t levelAdd,
-                                                     uint32_t lastLevel, uint32_t *head, uint2 *__restrict__ spill,
+                                                     const uint32_t *__restrict__ levelBase, uint32_t *head,
+                                                     uint2 *__restrict__ spill,
                                                      uint32_t spillPerWave, uint64_t *__restrict__ cand,
                                                      uint32_t *candCount, uint32_t candCap, uint32_t *overflow)
 {
@@ -343,8 +411,7 @@ __global__ __launch_bounds__(64) void k_traverse_dfs(TraverseArgs t, const uint2
     __shared__ uint64_t s_cand[kDfsCands];
     const int lane = threadIdx.x;
     if (levelBase) {
-        uint32_t level = *levelBase + levelAdd;
-        level = level < lastLevel ? level : lastLevel;
+        const uint32_t level = *levelBase;
         seeds = (level & 1) ? seedsAlt : seeds;
         seedCount += level;
     }
@@ -468,28 +535,25 @@ void launch_traverse_dfs(const TraverseArgs &t, const uint2 *seeds, const uint32
                          uint32_t *candCount, uint32_t candCap, uint32_t *overflow, hipStream_t s)
 {
     hipLaunchKernelGGL(k_traverse_dfs, dim3(waves), dim3(64), 0, s, t, seeds, seeds, seedCount, seedCap,
-                       (const uint32_t *)nullptr, 0u, 0u, head, spill, spillPerWave, cand, candCount, candCap,
-                       overflow);
+                       (const uint32_t *)nullptr, head, spill, spillPerWave, cand, candCount, candCap, overflow);
 }
 
-// The single-pair search after k_seed: the top kernel, `extra` grid-wide
-// levels after it (each a no-op past lastLevel), then the depth-first stage
-// from the level reached.  levelWord: one u32 of scratch.
+// The single-pair search after its first frontier: the one-workgroup levels,
+// then the depth-first stage from the level reached.  Up to 8 grid-wide levels
+// between the two cost a launch and a grid's start each and no longer pay now
+// that the depth-first steps are short: 734 us a pass with 8, 714 with 4, 637
+// with none at the 81,920-triangle pair, 1,700 / 1,683 / 1,681 at 1,310,720.
+// levelWord: one u32 of scratch.
 void launch_search_levels(const TraverseArgs &t, uint2 *front0, uint2 *front1, uint32_t *cnt, uint32_t fcap,
-                          uint32_t topMax, int lastLevel, int extra, uint32_t *levelWord, uint32_t *head,
-                          uint2 *spill, uint32_t spillPerWave, int waves, uint64_t *cand, uint32_t *candCount,
-                          uint32_t candCap, uint32_t *overflow, int expandGrid, hipStream_t s)
+                          uint32_t topMax, int lastLevel, uint32_t *levelWord, uint32_t *head, uint2 *spill,
+                          uint32_t spillPerWave, int waves, uint64_t *cand, uint32_t *candCount, uint32_t candCap,
+                          uint32_t *overflow, hipStream_t s)
 {
     hipLaunchKernelGGL(k_search_top, dim3(1), dim3(1024), 0, s, t, front0, front1, cnt, fcap, cand, candCount,
                        candCap, overflow, lastLevel, topMax, levelWord);
-    for (int j = 0; j < extra; ++j)
-        hipLaunchKernelGGL(k_expand_at, dim3(expandGrid * 256 / kExpandThreads), dim3(kExpandThreads), 0, s, t,
-                           front0, front1, cnt,
-                           (const uint32_t *)levelWord, (uint32_t)j, (uint32_t)lastLevel, fcap, cand, candCount,
-                           candCap, overflow);
     hipLaunchKernelGGL(k_traverse_dfs, dim3(waves), dim3(64), 0, s, t, (const uint2 *)front0, (const uint2 *)front1,
-                       (const uint32_t *)cnt, fcap, (const uint32_t *)levelWord, (uint32_t)extra,
-                       (uint32_t)lastLevel, head, spill, spillPerWave, cand, candCount, candCap, overflow);
+                       (const uint32_t *)cnt, fcap, (const uint32_t *)levelWord, head, spill, spillPerWave, cand,
+                       candCount, candCap, overflow);
 }
 
 // root pair: both meshes non-empty; a root may itself be a leaf (1 triangle)

@@ -90,6 +90,8 @@ struct sbg_mesh_s {
     DevBuf<float> tri32, box32, blockBounds, bounds, rootBox, treeScratch;
     DevBuf<uint32_t> keys, vals, keysAlt, valsAlt, treeWork;
     DevBuf<BNode> nodes;
+    DevBuf<float4> pieces;  // the tree's pieces per tile, for the pair search
+    DevBuf<uint32_t> pieceCount;
     uint32_t root = 0;
     const uint32_t *sortedIds = nullptr;  // triangles in Morton order (vals or valsAlt)
     bool prepared = false;
@@ -233,6 +235,8 @@ static void mesh_free_buffers(sbg_mesh m)
     m->valsAlt.release();
     m->treeWork.release();
     m->nodes.release();
+    m->pieces.release();
+    m->pieceCount.release();
     m->gridCells.release();
     m->gridTemp.release();
     m->gridCode.release();
@@ -734,6 +738,8 @@ int sbg_mesh_prepare(sbg_mesh m)
     TRY(m->valsAlt.ensure(nt));
     TRY(m->nodes.ensure(nt > 1 ? nt - 1 : 1));
     TRY(m->treeWork.ensure(nt + 1));
+    TRY(m->pieces.ensure(2 * (size_t)kTilePieces * tree_tiles((uint32_t)nt)));
+    TRY(m->pieceCount.ensure(tree_tiles((uint32_t)nt)));
     TRY(m->treeScratch.ensure(tree_scratch_floats((uint32_t)nt)));
     TRY(m->hist.ensure(sort_hist_entries(nt)));
     const hipStream_t s = m->stream;
@@ -777,8 +783,8 @@ int sbg_mesh_prepare(sbg_mesh m)
                                    s));
         } else {
             m->root = 0;
-            launch_tree(sk, sv, m->box32.p, (uint32_t)nt, m->nodes.p, m->treeWork.p, m->treeScratch.p, m->rootBox.p,
-                        s);
+            launch_tree(sk, sv, m->box32.p, (uint32_t)nt, m->nodes.p, m->treeWork.p, m->treeScratch.p,
+                        TreePieces{m->pieces.p, m->pieceCount.p}, m->rootBox.p, s);
         }
         TRY(check_launch("bvh"));
     }
@@ -951,6 +957,13 @@ int sbg_pairs_destroy(sbg_pairs p)
 
 static int queue_grids(sbg_mesh a, sbg_mesh b);
 
+// m's tree tiles as the first frontier of a pair search reads them
+static TileSet tile_set(sbg_mesh m)
+{
+    return {tree_tile_boxes(m->treeScratch.p, (uint32_t)m->nt), {m->pieces.p, m->pieceCount.p},
+            tree_tiles((uint32_t)m->nt)};
+}
+
 int sbg_find_pairs(sbg_mesh a, sbg_mesh b, sbg_pairs *out)
 {
     if (!out || !a || !b)
@@ -1010,15 +1023,21 @@ int sbg_find_pairs(sbg_mesh a, sbg_mesh b, sbg_pairs *out)
         {
             Stage st(c, SBG_STAGE_TRAVERSE);
             launch_fill_u32(cnt, 0u, kMaxLevels + 8, c->stream);
-            launch_seed(t, a->root, b->root, a->rootBox.p, b->rootBox.p, c->front[0].p, cnt, p->pairs.p, candCount,
-                        c->stream);
+            const uint32_t tilesA = tree_tiles((uint32_t)na), tilesB = tree_tiles((uint32_t)nb);
+            // from the tiles wherever a tree has several of them
+            const bool byTiles = tilesA > 1 && tilesB > 1 && (uint64_t)tilesA * tilesB <= kTilePairsMax;
+            if (byTiles)
+                launch_search_tiles(tile_set(a), tile_set(b), c->front[0].p, cnt, fcap, overflow, c->stream);
+            else
+                launch_seed(t, a->root, b->root, a->rootBox.p, b->rootBox.p, c->front[0].p, cnt, p->pairs.p, candCount,
+                            c->stream);
             if (dfs) {
-                // up to bfs_levels breadth-first levels with no host round
-                // trip (the small top levels in one workgroup), then one
-                // persistent launch over the frontier, then one sync
-                launch_search_levels(t, c->front[0].p, c->front[1].p, cnt, fcap, kTopMax, c->tune.bfs_levels,
-                                     kExtraLevels, topLevel, head, c->spill.p, c->spillPerWave, c->tune.dfs_waves,
-                                     p->pairs.p, candCount, ccap, overflow, kExpandGrid, c->stream);
+                // up to bfs_levels breadth-first levels in one workgroup
+                // while they are small, then one persistent launch over the
+                // frontier, then one sync
+                launch_search_levels(t, c->front[0].p, c->front[1].p, cnt, fcap, kTopMax, c->tune.bfs_levels, topLevel,
+                                     head, c->spill.p, c->spillPerWave, c->tune.dfs_waves, p->pairs.p, candCount,
+                                     ccap, overflow, c->stream);
                 rc = check_launch("depth-first search");
                 done = true;
             }

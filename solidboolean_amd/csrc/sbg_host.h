@@ -97,10 +97,11 @@ constexpr int kLevelsPerSync = 8;
 constexpr int kBfsLevels = 24;
 constexpr int kDfsWaves = 512;
 // the single-pair search expands levels of at most kTopMax node pairs in one
-// workgroup, then queues kExtraLevels grid-wide levels (no-ops once
-// bfs_levels is reached) before the depth-first stage
+// workgroup before the depth-first stage
 constexpr uint32_t kTopMax = 2048;
-constexpr int kExtraLevels = 8;
+// most pairs of tree tiles whose boxes are tested all against all for the
+// first frontier (larger trees start from their roots)
+constexpr uint64_t kTilePairsMax = (uint64_t)1 << 26;
 // longest run of one first triangle the quick pair sort orders by insertion
 constexpr uint32_t kSortRunMax = 64;
 constexpr uint32_t kSpillInit = 2048, kSpillMax = 1u << 15;

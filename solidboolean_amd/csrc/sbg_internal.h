@@ -72,8 +72,23 @@ int radix_sort_u64(uint64_t *keys, uint64_t *keysAlt, size_t n, const int *bitRa
 // launch_morton clears it, launch_tree64 clears it itself), scratch
 // tree_scratch_floats(n) floats (box unions within tiles and the tile table)
 size_t tree_scratch_floats(uint32_t n);
+// pieces: filled for the pair search (launch_search_tiles)
+constexpr int kTreeTile = 1024;  // sorted leaves per tile
+// The largest subtrees inside each tile ("pieces": what the nodes crossing its
+// borders have for children there; the root for a tree of one tile): 2 float4
+// each, (lo xyz, node reference) and (hi xyz, 0), kTilePieces slots per tile.
+// Nodes crossing one border lie on one path of the tree, on which the common
+// prefix of the keys grows from 8 (24-bit codes in 32 bits) to 31 and, by
+// index, from 32 to 63 bits: 55 at most, each with one piece in the tile.
+constexpr int kTilePieces = 128;
+struct TreePieces {
+    float4 *piece;
+    uint32_t *count;  // per tile (null: no list wanted)
+};
+uint32_t tree_tiles(uint32_t n);
+float *tree_tile_boxes(float *scratch, uint32_t n);  // tile t's box: 6 floats at 6 t
 void launch_tree(const uint32_t *codes, const uint32_t *ids, const float *box32, uint32_t n, BNode *nodes,
-                 uint32_t *work, float *scratch, float *rootBox, hipStream_t s);
+                 uint32_t *work, float *scratch, TreePieces pieces, float *rootBox, hipStream_t s);
 void launch_tree64(const uint64_t *codes, const uint32_t *ids, const float *box32, uint32_t n, BNode *nodes,
                    uint32_t *work, float *scratch, float *rootBox, hipStream_t s);
 void launch_fill_u32(uint32_t *p, uint32_t value, size_t n, hipStream_t s);
@@ -98,13 +113,23 @@ void launch_expand(const TraverseArgs &t, const uint2 *in, const uint32_t *inCou
 void launch_traverse_dfs(const TraverseArgs &t, const uint2 *seeds, const uint32_t *seedCount, uint32_t seedCap,
                          uint32_t *head, uint2 *spill, uint32_t spillPerWave, int waves, uint64_t *cand,
                          uint32_t *candCount, uint32_t candCap, uint32_t *overflow, hipStream_t s);
-// the single-pair search after launch_seed: levels in one workgroup while a
-// level holds at most topMax pairs, `extra` grid-wide levels, then the
-// depth-first stage (levels up to lastLevel breadth-first)
+// The first frontier of a single-pair search from the tiles of both trees
+// instead of their roots: every pair of pieces whose boxes overlap, in tiles
+// whose boxes do.
+struct TileSet {
+    const float *box;
+    TreePieces pieces;
+    uint32_t ntiles;
+};
+void launch_search_tiles(const TileSet &a, const TileSet &b, uint2 *frontier, uint32_t *count, uint32_t cap,
+                         uint32_t *overflow, hipStream_t s);
+// the single-pair search after its first frontier (launch_search_tiles or
+// launch_seed): levels in one workgroup while a level holds at most topMax
+// pairs (levels up to lastLevel), then the depth-first stage
 void launch_search_levels(const TraverseArgs &t, uint2 *front0, uint2 *front1, uint32_t *cnt, uint32_t fcap,
-                          uint32_t topMax, int lastLevel, int extra, uint32_t *levelWord, uint32_t *head,
-                          uint2 *spill, uint32_t spillPerWave, int waves, uint64_t *cand, uint32_t *candCount,
-                          uint32_t candCap, uint32_t *overflow, int expandGrid, hipStream_t s);
+                          uint32_t topMax, int lastLevel, uint32_t *levelWord, uint32_t *head, uint2 *spill,
+                          uint32_t spillPerWave, int waves, uint64_t *cand, uint32_t *candCount, uint32_t candCap,
+                          uint32_t *overflow, hipStream_t s);
 void launch_seed(const TraverseArgs &t, uint32_t rootA, uint32_t rootB, const float *rootBoxA,
                  const float *rootBoxB, uint2 *frontier, uint32_t *count, uint64_t *cand,
                  uint32_t *candCount, hipStream_t s);

@@ -637,6 +637,28 @@ def test_tuning_changes_speed_not_results(gpu):
         gpu.set_tuning(**saved)
 
 
+@pytest.mark.parametrize("na,nb", [(16, 16), (17, 16), (16, 23), (40, 23), (64, 5)])
+def test_search_from_tiles(gpu, na, nb):
+    """The pair search's first frontier where its rule changes: meshes of one
+    tree tile (1,024 leaves), just over one and several, with each other and
+    with a small mesh, against brute force over the FP64 boxes; an overlap of
+    nearly all boxes overfills the queues and the workgroups' lists."""
+    a = mg.transform(mg.torus(1.0, 0.3, 2 * na, na), mg.random_rotation(mg.SplitMix64(na)), (0.0, 0.0, 0.0))
+    b = mg.transform(mg.torus(0.8, 0.3, 2 * nb, nb), mg.random_rotation(mg.SplitMix64(nb + 100)), (0.4, 0.2, 0.1))
+    flat = mg.Mesh(b.vertices * 1e-3, b.triangles)  # all of it inside a few of a's triangles' boxes
+    wide = mg.Mesh(np.concatenate([a.vertices, [[-9.0, -9.0, -9.0], [9.0, 9.0, 9.0]]]),
+                   np.concatenate([a.triangles, np.stack([np.arange(700), np.full(700, a.nv), np.full(700, a.nv + 1)], 1)
+                                   % (a.nv + 2)]))
+    for x, y in ((a, b), (b, a), (wide, b), (wide, flat)):
+        X, Y = gpu.mesh(x.vertices, x.triangles), gpu.mesh(y.vertices, y.triangles)
+        bx, by = X.boxes(), Y.boxes()
+        hit = np.ones((x.nt, y.nt), bool)
+        for k in range(3):
+            hit &= (bx[:, None, k] <= by[None, :, 3 + k]) & (bx[:, None, 3 + k] >= by[None, :, k])
+        want = np.argwhere(hit)
+        assert np.array_equal(X.find_pairs(Y).array().astype(np.int64), want)
+
+
 def test_components_vs_oracle(gpu):
     """sbg_components against the oracle's restatement of the reference's face
     grouping: whole meshes, blocked bands, random blocked sets, several
