@@ -92,47 +92,34 @@ __device__ __forceinline__ int fsign(const F3 &a, const F3 &b, const F3 &c, floa
     return fsign_n(a, fcross(b, c), E);
 }
 
+__device__ __forceinline__ F3 vpick(bool first, const F3 &a, const F3 &b)
+{
+    return {first ? a.x : b.x, first ? a.y : b.y, first ? a.z : b.z};
+}
+
 // CONSTRUCT_INTERSECTION's predicates (tri_tri_intersect.c:286-296, 324-332):
 // 1 = intersection (segment computed later in FP64), 0 = rejection, -2 = uncertain
 __device__ __forceinline__ int f_construct(const F3 &p1, const F3 &q1, const F3 &r1, const F3 &p2, const F3 &q2,
                                            const F3 &r2, float E)
 {
-    const F3 v = fsub(p2, p1);
-    F3 v1 = fsub(q1, p1);
-    F3 v2 = fsub(r2, p1);
-    int s = fsign(v, v1, v2, E);
-    if (!s)
+    const F3 v = fsub(p2, p1), v1 = fsub(q1, p1), v2 = fsub(r2, p1);
+    const int first = fsign(v, v1, v2, E);
+    if (!first)
         return -2;
-    if (s > 0) {
-        v1 = fsub(r1, p1);
-        s = fsign(v, v1, v2, E);
-        if (!s)
-            return -2;
-        return s < 0 ? 1 : 0;
-    }
-    v2 = fsub(q2, p1);
-    s = fsign(v, v1, v2, E);
-    if (!s)
+    const F3 w1 = fsub(r1, p1), w2 = fsub(q2, p1);
+    const int second = fsign(v, vpick(first > 0, w1, v1), vpick(first > 0, v2, w2), E);
+    if (!second)
         return -2;
-    return s < 0 ? 0 : 1;
+    return (first > 0) == (second < 0) ? 1 : 0;
 }
 
-// TRI_TRI_INTER_3D (tri_tri_intersect.c:360-385) for non-zero signs
-__device__ __forceinline__ int f_inter3d(const F3 &p1, const F3 &q1, const F3 &r1, const F3 &p2, const F3 &q2,
-                                         const F3 &r2, int sp2, int sq2, int sr2, float E)
+__device__ __forceinline__ void turn_tri(F3 &p, F3 &q, F3 &r, int turn, bool swap)
 {
-    if (sp2 > 0) {
-        if (sq2 > 0)
-            return f_construct(p1, r1, q1, r2, p2, q2, E);
-        if (sr2 > 0)
-            return f_construct(p1, r1, q1, q2, r2, p2, E);
-        return f_construct(p1, q1, r1, p2, q2, r2, E);
-    }
-    if (sq2 < 0)
-        return f_construct(p1, q1, r1, r2, p2, q2, E);
-    if (sr2 < 0)
-        return f_construct(p1, q1, r1, q2, r2, p2, E);
-    return f_construct(p1, r1, q1, p2, q2, r2, E);
+    const F3 a = vpick(turn == 0, p, vpick(turn == 1, q, r)), b = vpick(turn == 0, q, vpick(turn == 1, r, p)),
+             c = vpick(turn == 0, r, vpick(turn == 1, p, q));
+    p = a;
+    q = vpick(swap, c, b);
+    r = vpick(swap, b, c);
 }
 
 // Returns a certified GdExit rejection (0, 1, 2), GD_HIT when the certified path
@@ -156,22 +143,13 @@ __device__ __forceinline__ int gd_filter(const F3 &p1, const F3 &q1, const F3 &r
         return -1;
     if (sp2 == sq2 && sp2 == sr2)
         return GD_REJECT_PLANE2;
-    int r;
-    if (sp1 > 0) {
-        if (sq1 > 0)
-            r = f_inter3d(r1, p1, q1, p2, r2, q2, sp2, sr2, sq2, E);
-        else if (sr1 > 0)
-            r = f_inter3d(q1, r1, p1, p2, r2, q2, sp2, sr2, sq2, E);
-        else
-            r = f_inter3d(p1, q1, r1, p2, q2, r2, sp2, sq2, sr2, E);
-    } else {
-        if (sq1 < 0)
-            r = f_inter3d(r1, p1, q1, p2, q2, r2, sp2, sq2, sr2, E);
-        else if (sr1 < 0)
-            r = f_inter3d(q1, r1, p1, p2, q2, r2, sp2, sq2, sr2, E);
-        else
-            r = f_inter3d(p1, q1, r1, p2, r2, q2, sp2, sr2, sq2, E);
-    }
+    // the FP64 test's permutations (gd_fp64), for certain signs
+    const GdTurn g1 = gd_turn(sp1, sq1, sr1);
+    const GdTurn g2 = gd_turn(sp2, g1.swap ? sr2 : sq2, g1.swap ? sq2 : sr2);
+    F3 a1 = p1, b1 = q1, c1 = r1, a2 = p2, b2 = vpick(g1.swap, r2, q2), c2 = vpick(g1.swap, q2, r2);
+    turn_tri(a1, b1, c1, g1.turn, g2.swap);
+    turn_tri(a2, b2, c2, g2.turn, false);
+    const int r = f_construct(a1, b1, c1, a2, b2, c2, E);
     if (r == -2)
         return -1;
     return r ? GD_HIT : GD_REJECT_INTERVAL;
