@@ -249,21 +249,6 @@ __global__ __launch_bounds__(256) void k_batch_seed(TraverseArgs t, const uint32
         atomicOr(overflow, 1u);
 }
 
-// both triangles of every hit are intersected
-__global__ __launch_bounds__(256) void k_mark_both(const uint64_t *__restrict__ pairs,
-                                                   const uint8_t *__restrict__ status,
-                                                   const uint32_t *__restrict__ count, uint32_t cap,
-                                                   uint8_t *__restrict__ flags)
-{
-    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-    const uint32_t n = *count < cap ? *count : cap;
-    if (i >= n || status[i] != 1)
-        return;
-    const uint64_t pr = pairs[i];
-    flags[(uint32_t)(pr >> 32)] = 1;
-    flags[(uint32_t)pr] = 1;
-}
-
 __global__ __launch_bounds__(256) void k_batch_bounds_init(int *__restrict__ mb, uint32_t nmeshes)
 {
     const uint32_t i = blockIdx.x * 256 + threadIdx.x;
@@ -322,13 +307,6 @@ void launch_batch_seed(const TraverseArgs &t, const uint32_t *meshRoot, const fl
     if (npairs)
         hipLaunchKernelGGL(k_batch_seed, dim3(blocks_for(npairs)), dim3(256), 0, s, t, meshRoot, meshBox, npairs,
                            frontier, frontCount, frontCap, cand, candCount, candCap, overflow);
-}
-
-void launch_mark_both(const uint64_t *pairs, const uint8_t *status, const uint32_t *count, uint32_t cap,
-                      uint8_t *flags, hipStream_t s)
-{
-    if (cap)
-        hipLaunchKernelGGL(k_mark_both, dim3(blocks_for(cap)), dim3(256), 0, s, pairs, status, count, cap, flags);
 }
 
 }  // namespace sbg

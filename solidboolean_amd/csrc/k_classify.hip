@@ -37,31 +37,42 @@ constexpr int kCodeGroup = 8;    // entry codes a fast lane loads at once (4-8 b
 constexpr int kWaveHits = 256;   // hits a wave gathers for one deferred ray
 constexpr int kWaveLoads = 2;    // cell entries a wave lane tests per round
 
+// Flags the triangles of every hit: pair's first triangle in flagsA, second in
+// flagsB (either may be null; a batch's triangles share one array).  count
+// (may be null): device-side number of pairs, at most n.
 __global__ __launch_bounds__(256) void k_mark_intersected(const uint64_t *__restrict__ pairs,
-                                                          const uint8_t *__restrict__ status, uint32_t n, int side,
-                                                          uint8_t *__restrict__ flags)
+                                                          const uint8_t *__restrict__ status, uint32_t n,
+                                                          const uint32_t *__restrict__ count, uint8_t *flagsA,
+                                                          uint8_t *flagsB)
 {
     const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (count && *count < n)
+        n = *count;
     if (i >= n || status[i] != 1)
         return;
     const uint64_t pr = pairs[i];
-    flags[side == 0 ? (uint32_t)(pr >> 32) : (uint32_t)pr] = 1;
+    if (flagsA)
+        flagsA[(uint32_t)(pr >> 32)] = 1;
+    if (flagsB)
+        flagsB[(uint32_t)pr] = 1;
 }
 
-// (v0 + v1 + v2) / 3.0 (src/solidboolean.cpp:497-499)
-__global__ __launch_bounds__(256) void k_centroids(const double *__restrict__ tri64, const uint8_t *__restrict__ flags,
-                                                   uint32_t nt, double *__restrict__ pts)
+// zeroes up to four arrays of u32
+__global__ __launch_bounds__(256) void k_clear(ClearList list)
 {
-    const uint32_t t = blockIdx.x * 256 + threadIdx.x;
-    if (t >= nt || (flags && flags[t]))
-        return;
-    const double *r = tri64 + (size_t)kTri64Stride * t;
-    pts[3 * (size_t)t] = (r[0] + r[4] + r[8]) / 3.0;
-    pts[3 * (size_t)t + 1] = (r[1] + r[5] + r[9]) / 3.0;
-    pts[3 * (size_t)t + 2] = (r[2] + r[6] + r[10]) / 3.0;
+    uint32_t i = blockIdx.x * 256 + threadIdx.x;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        if (i < list.n[k]) {
+            list.p[k][i] = 0u;
+            return;
+        }
+        i -= list.n[k];
+    }
 }
 
-// The same centroids in visiting order: query q (triangle order[q]) gets
+// The centroids (v0 + v1 + v2) / 3.0 (src/solidboolean.cpp:497-499) of a mesh's
+// triangles in visiting order: query q (triangle order[q]) gets
 // (x, y, z, tag) at q4 + 4q, with tag = the target mesh (target[t], 0 without
 // a target list), kTagSkip for a triangle flagged as intersected (with flags;
 // without, the queries do not depend on the intersections and the rays read
@@ -69,13 +80,10 @@ __global__ __launch_bounds__(256) void k_centroids(const double *__restrict__ tr
 // then reads its point without first waiting for order[q].
 constexpr double kTagSkip = -1.0, kTagNone = -2.0;
 
-__global__ __launch_bounds__(256) void k_centroids_ordered(const double *__restrict__ tri64,
-                                                           const uint8_t *__restrict__ flags,
-                                                           const uint32_t *__restrict__ order,
-                                                           const uint32_t *__restrict__ target, uint32_t nt,
-                                                           double *__restrict__ q4)
+__device__ __forceinline__ void centroid_query(const double *__restrict__ tri64, const uint8_t *__restrict__ flags,
+                                               const uint32_t *__restrict__ order, const uint32_t *__restrict__ target,
+                                               uint32_t nt, double *__restrict__ q4, uint32_t q)
 {
-    const uint32_t q = blockIdx.x * 256 + threadIdx.x;
     if (q >= nt)
         return;
     const uint32_t t = order[q];
@@ -88,6 +96,27 @@ __global__ __launch_bounds__(256) void k_centroids_ordered(const double *__restr
     const double *r = tri64 + (size_t)kTri64Stride * t;
     out[0] = make_double2((r[0] + r[4] + r[8]) / 3.0, (r[1] + r[5] + r[9]) / 3.0);
     out[1] = make_double2((r[2] + r[6] + r[10]) / 3.0, m == ~0u ? kTagNone : (double)m);
+}
+
+__global__ __launch_bounds__(256) void k_centroids_ordered(const double *__restrict__ tri64,
+                                                           const uint8_t *__restrict__ flags,
+                                                           const uint32_t *__restrict__ order,
+                                                           const uint32_t *__restrict__ target, uint32_t nt,
+                                                           double *__restrict__ q4)
+{
+    centroid_query(tri64, flags, order, target, nt, q4, blockIdx.x * 256 + threadIdx.x);
+}
+
+// Where both sides of a small boolean share a launch, the first blocksA
+// workgroups take side A.  One side alone has kernels of its own: with the
+// arguments behind a run-time choice of the side the x/y ray kernel took 180 us
+// against 173 at 1,310,720 triangles, the wave kernel 110 against 100.
+__global__ __launch_bounds__(256) void k_centroids_sides(QuerySides sides, uint32_t blocksA)
+{
+    const bool second = blockIdx.x >= blocksA;
+    const QuerySide &s = sides.s[second];
+    centroid_query(s.tri64, s.flags, s.order, s.target, s.nt, s.q4,
+                   (blockIdx.x - (second ? blocksA : 0u)) * 256 + threadIdx.x);
 }
 
 // A ray is the segment from p to e = p + dir (src/solidboolean.cpp:60-66):
@@ -618,6 +647,14 @@ __device__ __forceinline__ bool code_may_hit(const uint2 &e, const RayCell &c)
 constexpr int kStage = 384;  // cell entries a wave stages in LDS
 constexpr int kStageRounds = kStage / 64;
 
+// A side's counters, and the parts of its lists (ray_list_u32): records of 8
+// u32 for up to 2n deferred x and y rays (3n when every axis is cast) and n z
+// rays, then n z lanes.
+constexpr int kRayOverflow = 0, kRayDeferred = 1, kRayZLanes = 2, kRayZDeferred = 3;
+__host__ __device__ __forceinline__ uint32_t *ray_deferred(const RaySide &s) { return s.lists; }
+__host__ __device__ __forceinline__ uint32_t *ray_z_deferred(const RaySide &s) { return s.lists + 16 * (size_t)s.n; }
+__host__ __device__ __forceinline__ uint32_t *ray_z_lanes(const RaySide &s) { return s.lists + 24 * (size_t)s.n; }
+
 // Code test of entries [k0, k0 + 64) of a cell of len entries, as a bit mask,
 // in groups of kCodeGroup independent loads (indices clamped into the cell,
 // the excess masked off).  The whole chunk is tested before any candidate's
@@ -640,14 +677,15 @@ __device__ __forceinline__ unsigned long long pass_mask(const CodeAt &code_at, c
     return pass;
 }
 
+// laneList: the lanes to run (total of them; z lanes that k_third_axis listed),
+// without LIST the first `total` lanes.
 template <bool Q4, bool LIST, bool FILTER>
-__global__ __launch_bounds__(256) void k_rays_grid(GridSet gs, const double *__restrict__ tri64,
-                                                   const double *__restrict__ pts,
-                                                   const uint32_t *__restrict__ order, const uint8_t *__restrict__ skip,
-                                                   uint32_t n, uint32_t lanes, const uint32_t *__restrict__ laneList,
-                                                   const uint32_t *__restrict__ laneCount,
-                                                   uint8_t *__restrict__ bits, uint32_t *__restrict__ ovfList,
-                                                   uint32_t *ovfCount, uint32_t *overflow)
+__device__ __forceinline__ void rays_grid_block(const GridSet &gs, const double *__restrict__ tri64,
+                                                const double *__restrict__ pts, const uint32_t *__restrict__ order,
+                                                const uint8_t *__restrict__ skip, uint32_t n, uint32_t total,
+                                                const uint32_t *__restrict__ laneList, uint8_t *__restrict__ bits,
+                                                uint32_t *__restrict__ ovfList, uint32_t *ovfCount,
+                                                uint32_t *overflow, uint32_t block)
 {
     // each of the workgroup's four waves stages into its own LDS region
     __shared__ uint2 s_codeW[4][kStage];
@@ -656,16 +694,15 @@ __global__ __launch_bounds__(256) void k_rays_grid(GridSet gs, const double *__r
     const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     uint2 *s_code = s_codeW[wave];
     uint32_t *s_tri = s_triW[wave], *s_base = s_baseW[wave], *s_start = s_startW[wave];
-    const uint32_t total = LIST ? *laneCount : lanes;
     // every exit before the staging below is taken by the whole workgroup
-    if (blockIdx.x * 256 >= total)
+    if (block * 256 >= total)
         return;
     if (gs.cells[gs.ncells] > gs.cap) {  // grid truncated: the host rebuilds it larger
         if (threadIdx.x == 0)
             atomicOr(overflow, 2u);
         return;
     }
-    const uint32_t idx = blockIdx.x * 256 + threadIdx.x;
+    const uint32_t idx = block * 256 + threadIdx.x;
     uint32_t g = 0, axis = 0, i = 0, m = 0;
     Ray r;
     int kind = 0;
@@ -799,22 +836,45 @@ __global__ __launch_bounds__(256) void k_rays_grid(GridSet gs, const double *__r
     rec[1] = make_uint4(c.u, c.v, c.pa, 0u);
 }
 
+template <bool Q4, bool LIST, bool FILTER>
+__global__ __launch_bounds__(256) void k_rays_grid(GridSet gs, const double *__restrict__ tri64,
+                                                   const double *__restrict__ pts,
+                                                   const uint32_t *__restrict__ order, const uint8_t *__restrict__ skip,
+                                                   uint32_t n, uint32_t lanes, const uint32_t *__restrict__ laneList,
+                                                   const uint32_t *__restrict__ laneCount,
+                                                   uint8_t *__restrict__ bits, uint32_t *__restrict__ ovfList,
+                                                   uint32_t *ovfCount, uint32_t *overflow)
+{
+    rays_grid_block<Q4, LIST, FILTER>(gs, tri64, pts, order, skip, n, LIST ? *laneCount : lanes, laneList, bits,
+                                      ovfList, ovfCount, overflow, blockIdx.x);
+}
+
+template <bool Q4, bool LIST, bool FILTER>
+__global__ __launch_bounds__(256) void k_rays_grid_sides(RaySides sides, uint32_t blocksA, uint32_t axes)
+{
+    const bool second = blockIdx.x >= blocksA;
+    const RaySide &s = sides.s[second];
+    rays_grid_block<Q4, LIST, FILTER>(s.gs, s.tri64, s.pts, s.order, s.skip, s.n,
+                                      LIST ? s.counters[kRayZLanes] : axes * s.n, ray_z_lanes(s), s.bits,
+                                      LIST ? ray_z_deferred(s) : ray_deferred(s),
+                                      s.counters + (LIST ? kRayZDeferred : kRayDeferred), s.counters + kRayOverflow,
+                                      blockIdx.x - (second ? blocksA : 0u));
+}
+
 // One wave per deferred ray (record of 8 u32 written by k_rays_grid: lane
 // g = axis * n + q, cell range, output index, the ray's codes): the 64 lanes split
 // the cell's entries, hit keys are gathered in LDS (up to kWaveHits) and the
 // distinct ones counted; more hits than that raise `overflow`.
+// The workgroup's share of a list: rays first, first + stride, ...
 template <bool Q4>
-__global__ __launch_bounds__(64) void k_rays_wave(GridSet gs, const double *__restrict__ tri64,
-                                                  const double *__restrict__ pts,
-                                                  const uint32_t *__restrict__ order, uint32_t n,
-                                                  uint8_t *__restrict__ bits, const uint32_t *__restrict__ list,
-                                                  const uint32_t *__restrict__ count, uint32_t *overflow)
+__device__ __forceinline__ void rays_wave(const GridSet &gs, const double *__restrict__ tri64,
+                                          const double *__restrict__ pts, uint32_t n, uint8_t *__restrict__ bits,
+                                          const uint32_t *__restrict__ list, uint32_t total, uint32_t *overflow,
+                                          uint32_t first, uint32_t stride, long long (*s_key)[kWaveHits])
 {
-    __shared__ long long s_key[3][kWaveHits];
     const int lane = threadIdx.x;
     const unsigned long long below = (1ull << lane) - 1ull;
-    const uint32_t total = *count;
-    for (uint32_t k = blockIdx.x; k < total; k += gridDim.x) {
+    for (uint32_t k = first; k < total; k += stride) {
         // the fast path's record of the ray: lane, cell range, output index, codes
         const uint4 *rec = reinterpret_cast<const uint4 *>(list) + 2 * (size_t)k;
         const uint4 r0 = rec[0], r1 = rec[1];
@@ -889,16 +949,45 @@ __global__ __launch_bounds__(64) void k_rays_wave(GridSet gs, const double *__re
     }
 }
 
+template <bool Q4>
+__global__ __launch_bounds__(64) void k_rays_wave(GridSet gs, const double *__restrict__ tri64,
+                                                  const double *__restrict__ pts, uint32_t n,
+                                                  uint8_t *__restrict__ bits, const uint32_t *__restrict__ list,
+                                                  const uint32_t *__restrict__ count, uint32_t *overflow)
+{
+    __shared__ long long s_key[3][kWaveHits];
+    rays_wave<Q4>(gs, tri64, pts, n, bits, list, *count, overflow, blockIdx.x, gridDim.x, s_key);
+}
+
+// Rays of both sides in turn, from opposite ends of the launch, so that two
+// short lists spread over its waves.  Z: the deferred z rays.
+template <bool Q4, bool Z>
+__global__ __launch_bounds__(64, 4) void k_rays_wave_sides(RaySides sides)
+{
+    __shared__ long long s_key[3][kWaveHits];
+    for (int k = 0; k < 2; ++k) {
+        const RaySide &s = sides.s[k];
+        if (s.n)
+            rays_wave<Q4>(s.gs, s.tri64, s.pts, s.n, s.bits, Z ? ray_z_deferred(s) : ray_deferred(s),
+                          s.counters[Z ? kRayZDeferred : kRayDeferred], s.counters + kRayOverflow,
+                          k ? gridDim.x - 1 - blockIdx.x : blockIdx.x, gridDim.x, s_key);
+    }
+}
+
 // The vote needs the z ray only where the x and y rays disagree: lists the
 // lanes 2n + q of those queries (one atomic per wave).
 template <bool Q4>
-__global__ __launch_bounds__(256) void k_third_axis(const double *__restrict__ pts,
-                                                    const uint32_t *__restrict__ order,
-                                                    const uint8_t *__restrict__ skip, uint32_t n,
-                                                    const uint8_t *__restrict__ bits, uint32_t *__restrict__ list,
-                                                    uint32_t *count)
+__global__ __launch_bounds__(256) void k_third_axis(RaySides sides, uint32_t blocksA)
 {
-    const uint32_t q = blockIdx.x * 256 + threadIdx.x;
+    const RaySide &side = sides.s[blockIdx.x >= blocksA];
+    const double *__restrict__ pts = side.pts;
+    const uint32_t *__restrict__ order = side.order;
+    const uint8_t *__restrict__ skip = side.skip;
+    const uint32_t n = side.n;
+    const uint8_t *__restrict__ bits = side.bits;
+    uint32_t *__restrict__ list = ray_z_lanes(side);
+    uint32_t *count = side.counters + kRayZLanes;
+    const uint32_t q = (blockIdx.x >= blocksA ? blockIdx.x - blocksA : blockIdx.x) * 256 + threadIdx.x;
     bool need = false;
     if (q < n) {
         const uint32_t i = order ? order[q] : q;
@@ -958,37 +1047,84 @@ __global__ __launch_bounds__(256) void k_ray_work(GridSet gs, const double *__re
 }
 
 // decideGroupSide's vote (src/solidboolean.cpp:492-508): inside iff
-// (float)inside / 3 > 0.5, i.e. at least 2 of the 3 rays.  The z bit is read
-// only where the x and y bits differ (it is not cast elsewhere), which gives
-// the same majority.
-__global__ __launch_bounds__(256) void k_vote(const uint8_t *__restrict__ bits, const uint8_t *__restrict__ skip,
-                                              uint32_t n, uint8_t *__restrict__ out)
+// (float)inside / 3 > 0.5, i.e. at least 2 of the 3 rays: x and y where they
+// agree, else z (which is cast only there).  Skipped queries get 2.  Four
+// queries per lane, a byte each; the votes may go straight to page-locked host
+// memory (256 B per wave and store).  The first lane hands out the overflow
+// bits and the grid's entry count (pubFlags, pubTotal; may be null).
+__global__ __launch_bounds__(256) void k_vote(VoteSides sides, uint32_t blocksA)
 {
-    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    const VoteSide &s = sides.s[blockIdx.x >= blocksA];
+    const uint32_t idx = (blockIdx.x >= blocksA ? blockIdx.x - blocksA : blockIdx.x) * 256 + threadIdx.x;
+    if (idx == 0) {
+        if (s.pubFlags)
+            *s.pubFlags = *s.overflow;
+        if (s.pubTotal)
+            *s.pubTotal = *s.total;
+    }
+    const uint32_t i = 4 * idx, n = s.n;
     if (i >= n)
         return;
-    if (skip && skip[i]) {
-        out[i] = 2;
-        return;
+    const uint32_t m = n - i < 4u ? n - i : 4u;
+    uint32_t x = 0, y = 0, z = 0, skip = 0;
+    if (m == 4u) {
+        // bytes of four neighbouring queries, at any alignment
+        __builtin_memcpy(&x, s.bits + i, 4);
+        __builtin_memcpy(&y, s.bits + (size_t)n + i, 4);
+        __builtin_memcpy(&z, s.bits + 2 * (size_t)n + i, 4);
+        if (s.skip)
+            __builtin_memcpy(&skip, s.skip + i, 4);
+    } else {
+        for (uint32_t k = 0; k < m; ++k) {
+            x |= (uint32_t)s.bits[i + k] << 8 * k;
+            y |= (uint32_t)s.bits[(size_t)n + i + k] << 8 * k;
+            z |= (uint32_t)s.bits[2 * (size_t)n + i + k] << 8 * k;
+            if (s.skip)
+                skip |= (uint32_t)s.skip[i + k] << 8 * k;
+        }
     }
-    const int bx = bits[i], by = bits[n + i];
-    const int inside = bx == by ? 2 * bx : bx + by + bits[2 * (size_t)n + i];
-    out[i] = ((float)inside / 3.0f > 0.5f) ? 1 : 0;
+    const uint32_t vote = ((x & y) | ((x ^ y) & z)) & ~(skip * 255u) | skip << 1;
+    if (m == 4u)
+        __builtin_memcpy(s.out + i, &vote, 4);
+    else
+        for (uint32_t k = 0; k < m; ++k)
+            s.out[i + k] = (uint8_t)(vote >> 8 * k);
 }
 
-void launch_mark_intersected(const uint64_t *pairs, const uint8_t *status, uint32_t n, int side,
-                             uint8_t *flags, hipStream_t s)
+static unsigned blocks_of(size_t n) { return (unsigned)((n + 255) / 256); }
+
+void launch_mark_intersected(const uint64_t *pairs, const uint8_t *status, uint32_t n, const uint32_t *count,
+                             uint8_t *flagsA, uint8_t *flagsB, hipStream_t s)
 {
-    if (n == 0)
-        return;
-    hipLaunchKernelGGL(k_mark_intersected, dim3((n + 255) / 256), dim3(256), 0, s, pairs, status, n, side, flags);
+    if (n)
+        hipLaunchKernelGGL(k_mark_intersected, dim3(blocks_of(n)), dim3(256), 0, s, pairs, status, n, count, flagsA,
+                           flagsB);
 }
 
-void launch_centroids(const double *tri64, const uint8_t *flags, uint32_t nt, double *pts, hipStream_t s)
+void launch_clear(const ClearList &list, hipStream_t s)
 {
-    if (nt == 0)
-        return;
-    hipLaunchKernelGGL(k_centroids, dim3((nt + 255) / 256), dim3(256), 0, s, tri64, flags, nt, pts);
+    const size_t n = (size_t)list.n[0] + list.n[1] + list.n[2] + list.n[3];
+    if (n)
+        hipLaunchKernelGGL(k_clear, dim3(blocks_of(n)), dim3(256), 0, s, list);
+}
+
+void launch_centroids_ordered(const QuerySides &sides, hipStream_t s)
+{
+    const unsigned a = blocks_of(sides.s[0].nt), b = blocks_of(sides.s[1].nt);
+    if (a && b) {
+        hipLaunchKernelGGL(k_centroids_sides, dim3(a + b), dim3(256), 0, s, sides, a);
+    } else if (a || b) {
+        const QuerySide &q = sides.s[a ? 0 : 1];
+        hipLaunchKernelGGL(k_centroids_ordered, dim3(a + b), dim3(256), 0, s, q.tri64, q.flags, q.order, q.target, q.nt,
+                           q.q4);
+    }
+}
+
+void launch_vote(const VoteSides &sides, hipStream_t s)
+{
+    const unsigned a = blocks_of(((size_t)sides.s[0].n + 3) / 4), b = blocks_of(((size_t)sides.s[1].n + 3) / 4);
+    if (a + b)
+        hipLaunchKernelGGL(k_vote, dim3(a + b), dim3(256), 0, s, sides, a);
 }
 
 // cells per axis side: G^2 = nt * density / 16, G in [1, 1024]
@@ -1025,100 +1161,88 @@ void launch_grid_build(const float *box32, uint32_t nt, const GridSet &gs, uint3
         grid_build<kGridSlotBitsWide, kGridTrisWide>(box32, nt, gs, cells, scanTemp, gcode, gtri, 0, s);
 }
 
-// Rays of n queries.  allAxes: every query casts x, y and z; otherwise x and
-// y, then z only where they disagree (enough for the vote; the per-axis bits
-// of z are then valid only there).  lists: ray_list_u32(n) u32 (deferred-ray
-// records of 8 u32 for up to 3n rays, then n z lanes); counters: 4 u32, zero
-// on entry ([0] overflow bits, [1] deferred x/y rays, [2] z lanes, [3]
-// deferred z rays).
-template <bool Q4>
-static void rays(const GridSet &gs, const double *tri64, const double *pts, const uint32_t *order,
-                 const uint8_t *skip, uint32_t n, bool allAxes, uint8_t *axisBits, uint32_t *lists,
-                 uint32_t *counters, hipStream_t s)
+template <bool Q4, bool LIST, bool FILTER>
+static void rays_grid(const RaySides &r, uint32_t axes, hipStream_t s)
 {
-    if (n == 0)
+    const unsigned a = blocks_of((size_t)axes * r.s[0].n), b = blocks_of((size_t)axes * r.s[1].n);
+    if (a && b) {
+        hipLaunchKernelGGL((k_rays_grid_sides<Q4, LIST, FILTER>), dim3(a + b), dim3(256), 0, s, r, a, axes);
         return;
-    uint32_t *overflow = counters;
-    const uint32_t lanes = allAxes ? 3u * n : 2u * n;
-    uint32_t *deferred = lists, *zDeferred = lists + 8 * 2 * (size_t)n, *zLanes = lists + 8 * 3 * (size_t)n;
-    if (gs.tri32)
-        hipLaunchKernelGGL((k_rays_grid<Q4, false, true>), dim3((lanes + 255) / 256), dim3(256), 0, s, gs, tri64, pts,
-                           order, skip, n, lanes, nullptr, nullptr, axisBits, deferred, counters + 1, overflow);
+    }
+    const RaySide &x = r.s[a ? 0 : 1];
+    hipLaunchKernelGGL((k_rays_grid<Q4, LIST, FILTER>), dim3(a + b), dim3(256), 0, s, x.gs, x.tri64, x.pts, x.order,
+                       x.skip, x.n, axes * x.n, ray_z_lanes(x), x.counters + kRayZLanes, x.bits,
+                       LIST ? ray_z_deferred(x) : ray_deferred(x), x.counters + (LIST ? kRayZDeferred : kRayDeferred),
+                       x.counters + kRayOverflow);
+}
+
+template <bool Q4, bool LIST>
+static void rays_grid(const RaySides &r, uint32_t axes, hipStream_t s)
+{
+    if ((r.s[0].n ? r.s[0] : r.s[1]).gs.tri32)  // the same on both sides
+        rays_grid<Q4, LIST, true>(r, axes, s);
     else
-        hipLaunchKernelGGL((k_rays_grid<Q4, false, false>), dim3((lanes + 255) / 256), dim3(256), 0, s, gs, tri64, pts,
-                           order, skip, n, lanes, nullptr, nullptr, axisBits, deferred, counters + 1, overflow);
-    hipLaunchKernelGGL(k_rays_wave<Q4>, dim3(8192), dim3(64), 0, s, gs, tri64, pts, order, n, axisBits, deferred,
-                       counters + 1, overflow);
+        rays_grid<Q4, LIST, false>(r, axes, s);
+}
+
+template <bool Q4, bool Z>
+static void rays_wave_launch(const RaySides &r, hipStream_t s)
+{
+    if (r.s[0].n && r.s[1].n) {
+        hipLaunchKernelGGL((k_rays_wave_sides<Q4, Z>), dim3(8192), dim3(64), 0, s, r);
+        return;
+    }
+    const RaySide &x = r.s[0].n ? r.s[0] : r.s[1];
+    hipLaunchKernelGGL(k_rays_wave<Q4>, dim3(8192), dim3(64), 0, s, x.gs, x.tri64, x.pts, x.n, x.bits,
+                       Z ? ray_z_deferred(x) : ray_deferred(x), x.counters + (Z ? kRayZDeferred : kRayDeferred),
+                       x.counters + kRayOverflow);
+}
+
+// Rays of both sides' queries.  allAxes: every query casts x, y and z; otherwise
+// x and y, then z only where they disagree (enough for the vote; the per-axis
+// bits of z are then valid only there).
+template <bool Q4>
+static void rays(const RaySides &r, bool allAxes, hipStream_t s)
+{
+    const unsigned a = blocks_of(r.s[0].n), b = blocks_of(r.s[1].n);
+    if (a + b == 0)
+        return;
+    rays_grid<Q4, false>(r, allAxes ? 3u : 2u, s);
+    rays_wave_launch<Q4, false>(r, s);
     if (allAxes)
         return;
-    hipLaunchKernelGGL(k_third_axis<Q4>, dim3((n + 255) / 256), dim3(256), 0, s, pts, order, skip, n, axisBits,
-                       zLanes, counters + 2);
-    if (gs.tri32)
-        hipLaunchKernelGGL((k_rays_grid<Q4, true, true>), dim3((n + 255) / 256), dim3(256), 0, s, gs, tri64, pts, order,
-                           skip, n, n, zLanes, counters + 2, axisBits, zDeferred, counters + 3, overflow);
-    else
-        hipLaunchKernelGGL((k_rays_grid<Q4, true, false>), dim3((n + 255) / 256), dim3(256), 0, s, gs, tri64, pts, order,
-                           skip, n, n, zLanes, counters + 2, axisBits, zDeferred, counters + 3, overflow);
-    hipLaunchKernelGGL(k_rays_wave<Q4>, dim3(8192), dim3(64), 0, s, gs, tri64, pts, order, n, axisBits, zDeferred,
-                       counters + 3, overflow);
+    hipLaunchKernelGGL(k_third_axis<Q4>, dim3(a + b), dim3(256), 0, s, r, a);
+    rays_grid<Q4, true>(r, 1u, s);
+    rays_wave_launch<Q4, true>(r, s);
 }
 
 size_t ray_list_u32(size_t n) { return 8 * 3 * n + n; }
 
-void launch_rays(const GridSet &gs, const double *tri64, const double *pts, const uint32_t *order,
-                 const uint8_t *skip, uint32_t n, bool allAxes, uint8_t *axisBits, uint32_t *lists,
-                 uint32_t *counters, hipStream_t s)
+void launch_rays(const RaySides &r, bool ordered, bool allAxes, hipStream_t s)
 {
-    rays<false>(gs, tri64, pts, order, skip, n, allAxes, axisBits, lists, counters, s);
-}
-
-void launch_centroids_ordered(const double *tri64, const uint8_t *flags, const uint32_t *order,
-                              const uint32_t *target, uint32_t nt, double *q4, hipStream_t s)
-{
-    if (nt == 0)
-        return;
-    hipLaunchKernelGGL(k_centroids_ordered, dim3((nt + 255) / 256), dim3(256), 0, s, tri64, flags, order, target,
-                       nt, q4);
-}
-
-void launch_rays_xy_ordered(const GridSet &gs, const double *tri64, const double *q4, const uint32_t *order,
-                            uint32_t n, uint8_t *axisBits, uint32_t *lists, uint32_t *counters, hipStream_t s)
-{
-    if (n == 0)
-        return;
-    const uint32_t lanes = 2u * n;
-    if (gs.tri32)
-        hipLaunchKernelGGL((k_rays_grid<true, false, true>), dim3((lanes + 255) / 256), dim3(256), 0, s, gs, tri64, q4,
-                           order, nullptr, n, lanes, nullptr, nullptr, axisBits, lists, counters + 1, counters);
+    if (ordered)
+        rays<true>(r, allAxes, s);
     else
-        hipLaunchKernelGGL((k_rays_grid<true, false, false>), dim3((lanes + 255) / 256), dim3(256), 0, s, gs, tri64, q4,
-                           order, nullptr, n, lanes, nullptr, nullptr, axisBits, lists, counters + 1, counters);
+        rays<false>(r, allAxes, s);
 }
 
-void launch_rays_wave_ordered(const GridSet &gs, const double *tri64, const double *q4, const uint32_t *order,
-                              uint32_t n, uint8_t *axisBits, const uint32_t *lists, uint32_t *counters, hipStream_t s)
+void launch_rays_xy_ordered(const RaySide &r, hipStream_t s)
 {
-    if (n == 0)
-        return;
-    hipLaunchKernelGGL(k_rays_wave<true>, dim3(8192), dim3(64), 0, s, gs, tri64, q4, order, n, axisBits, lists,
-                       counters + 1, counters);
+    if (r.n)
+        rays_grid<true, false>(RaySides{{r, RaySide{}}}, 2u, s);
 }
 
-void launch_ray_work_ordered(const GridSet &gs, const double *q4, const uint32_t *order, uint32_t n,
-                             unsigned long long *work, hipStream_t s)
+void launch_rays_wave_ordered(const RaySide &r, hipStream_t s)
 {
-    if (n == 0)
-        return;
-    const uint32_t lanes = 2u * n;
-    hipLaunchKernelGGL(k_ray_work<true>, dim3((lanes + 255) / 256), dim3(256), 0, s, gs, q4, order, nullptr, n, lanes,
-                       work);
+    if (r.n)
+        rays_wave_launch<true, false>(RaySides{{r, RaySide{}}}, s);
 }
 
-void launch_rays_ordered(const GridSet &gs, const double *tri64, const double *q4, const uint32_t *order,
-                         const uint8_t *skip, uint32_t n, bool allAxes, uint8_t *axisBits, uint32_t *lists,
-                         uint32_t *counters, hipStream_t s)
+void launch_ray_work_ordered(const RaySide &r, unsigned long long *work, hipStream_t s)
 {
-    rays<true>(gs, tri64, q4, order, skip, n, allAxes, axisBits, lists, counters, s);
+    if (r.n)
+        hipLaunchKernelGGL(k_ray_work<true>, dim3(blocks_of(2 * (size_t)r.n)), dim3(256), 0, s, r.gs, r.pts, r.order,
+                           nullptr, r.n, 2u * r.n, work);
 }
 
 // per-axis bits [axis][n] -> per-point triples [n][3]
@@ -1138,13 +1262,6 @@ void launch_interleave_axes(const uint8_t *axisBits, uint32_t n, uint8_t *out, h
     if (n == 0)
         return;
     hipLaunchKernelGGL(k_interleave_axes, dim3((n + 255) / 256), dim3(256), 0, s, axisBits, n, out);
-}
-
-void launch_vote(const uint8_t *axisBits, const uint8_t *skip, uint32_t n, uint8_t *out, hipStream_t s)
-{
-    if (n == 0)
-        return;
-    hipLaunchKernelGGL(k_vote, dim3((n + 255) / 256), dim3(256), 0, s, axisBits, skip, n, out);
 }
 
 }  // namespace sbg

@@ -1457,110 +1457,159 @@ struct RayBufs {
     DevBuf<uint8_t> &flags, &bits, &votes;
     DevBuf<uint32_t> &ovf, &rayList;
     uint32_t *host;  // 4 words: overflow flags, grid entries, -, -
-    hipStream_t s;   // the stream this side's work goes on
     PinnedBuf &votesHost;
 };
 
 static RayBufs ray_bufs(sbg_context c, int set)
 {
     if (set)
-        return {c->pts2,   c->flags2, c->bits2, c->votes2, c->ovf2, c->rayList2, c->pinned + kRayPinned + 4,
-                c->aux,    c->votesHost2};
-    return {c->pts,    c->flags,  c->bits,  c->votes,  c->ovf,  c->rayList,  c->pinned + kRayPinned,
-            c->stream, c->votesHost};
+        return {c->pts2, c->flags2, c->bits2, c->votes2, c->ovf2, c->rayList2, c->pinned + kRayPinned + 4,
+                c->votesHost2};
+    return {c->pts, c->flags, c->bits, c->votes, c->ovf, c->rayList, c->pinned + kRayPinned, c->votesHost};
 }
 
-// Page-locked host memory (hipHostMalloc, sbg_host_alloc, or registered by
-// the caller): a device-to-host copy into it is plain DMA.
-static bool page_locked(const void *p)
+// Page-locked host memory (hipHostMalloc, sbg_host_alloc, or registered by the
+// caller): a device-to-host copy into it is plain DMA.  *device says whether
+// kernels reach it at the same address.
+static bool page_locked(const void *p, bool *device)
 {
     hipPointerAttribute_t at;
+    *device = false;
     if (hipPointerGetAttributes(&at, p) != hipSuccess) {
         (void)hipGetLastError();  // pageable memory is not an error here
         return false;
     }
+    *device = at.type == hipMemoryTypeHost && at.devicePointer == p;
     return at.type == hipMemoryTypeHost;
 }
 
-// Queues the rays of n queries into target's grid, the vote into rb.votes,
-// and the readbacks (overflow flags and the grid's entry count into rb.host;
-// with hostVotes the votes, straight into hostVotes when it is page-locked,
-// else into rb.votesHost for the caller to copy out); nothing waits.  *direct
-// says which.  ordered: dpts is the visiting-order (x, y, z, tag) layout over
-// dorder; otherwise xyz triples by index with optional dorder / dskip.
-static int enqueue_rays(sbg_mesh target, RayBufs rb, const double *dpts, const uint32_t *dorder,
-                        const uint8_t *dskip, size_t n, bool ordered, bool allAxes, uint8_t *hostVotes,
-                        bool *direct)
+// One side of a classification: the rays of n queries into target's grid, the
+// votes to hostVotes (null: none wanted).  pts: visiting-order (x, y, z, tag)
+// over order, whose intersected triangles (rb.flags) carry the skip tag; or xyz
+// triples by index, order null.
+struct RayJob {
+    sbg_mesh target;
+    RayBufs rb;
+    const double *pts;
+    const uint32_t *order;
+    const uint8_t *voteSkip;
+    size_t n;
+    uint8_t *hostVotes;
+    enum { kNone, kKernel, kCopy, kStaged } way;  // how the votes reach hostVotes
+};
+
+// Queues the rays of up to two sides, the votes and the readbacks (overflow
+// flags and the grids' entry counts into rb.host, written by the vote kernel)
+// on stream s; nothing waits.  The votes go straight into hostVotes where that is
+// page-locked, else into rb.votesHost for the caller to copy out.  The
+// counters must be zero where `cleared` says so.
+static int enqueue_rays(RayJob *jobs, int njobs, bool ordered, bool allAxes, bool cleared, hipStream_t s)
 {
-    sbg_context c = target->ctx;
+    sbg_context c = jobs[0].target->ctx;
     const bool filtered = c->tune.ray_precision == SBG_PRECISION_FP32_FILTERED;
-    const bool votes = hostVotes != nullptr;
-    *direct = votes && page_locked(hostVotes);
-    TRY(rb.ovf.ensure(4));
-    if (votes && !*direct)
-        TRY(rb.votesHost.ensure(n));
-    TRY(rb.rayList.ensure(ray_list_u32(n)));
-    rb.host[0] = rb.host[1] = 0;
-    if (target->nt == 0) {
-        Stage st(c, SBG_STAGE_CLASSIFY, rb.s);
-        launch_fill_u32((uint32_t *)rb.bits.p, 0u, (3 * n + 3) / 4, rb.s);
-        launch_vote(rb.bits.p, dskip, (uint32_t)n, rb.votes.p, rb.s);
-        TRY(check_launch("rays"));
-    } else {
-        TRY(ensure_grid(target, rb.s));
-        Stage st(c, SBG_STAGE_CLASSIFY, rb.s);
-        launch_fill_u32(rb.ovf.p, 0u, 4, rb.s);
-        if (ordered)
-            launch_rays_ordered(grid_set(target, filtered), target->tri64.p, dpts, dorder, nullptr, (uint32_t)n, allAxes, rb.bits.p,
-                                rb.rayList.p, rb.ovf.p, rb.s);
-        else
-            launch_rays(grid_set(target, filtered), target->tri64.p, dpts, dorder, dskip, (uint32_t)n, allAxes, rb.bits.p,
-                        rb.rayList.p, rb.ovf.p, rb.s);
-        launch_vote(rb.bits.p, dskip, (uint32_t)n, rb.votes.p, rb.s);
-        TRY(check_launch("rays"));
-        HIP_TRY(hipMemcpyAsync(rb.host, rb.ovf.p, sizeof(uint32_t), hipMemcpyDeviceToHost, rb.s));
-        HIP_TRY(hipMemcpyAsync(rb.host + 1, target->gridCells.p + (grid_cells(target->gridG) - 1),
-                               sizeof(uint32_t), hipMemcpyDeviceToHost, rb.s));
+    RaySides rays = {};
+    VoteSides votes = {};
+    ClearList clear = {};
+    for (int k = 0; k < njobs; ++k) {
+        RayJob &j = jobs[k];
+        const RayBufs &rb = j.rb;
+        const uint32_t n = (uint32_t)j.n;
+        TRY(rb.ovf.ensure(4));
+        j.way = RayJob::kNone;
+        if (j.hostVotes) {
+            bool device = false;
+            j.way = !page_locked(j.hostVotes, &device) ? RayJob::kStaged : device ? RayJob::kKernel : RayJob::kCopy;
+            if (j.way == RayJob::kStaged)
+                TRY(rb.votesHost.ensure(n));
+        }
+        TRY(rb.rayList.ensure(ray_list_u32(n)));
+        rb.host[0] = rb.host[1] = 0;
+        uint8_t *out = j.way == RayJob::kKernel ? j.hostVotes : j.way == RayJob::kStaged ? rb.votesHost.p : rb.votes.p;
+        VoteSide v = {rb.bits.p, j.voteSkip, n, out, nullptr, nullptr, nullptr, nullptr};
+        if (j.target->nt == 0) {
+            launch_fill_u32((uint32_t *)rb.bits.p, 0u, (3 * (size_t)n + 3) / 4, s);
+        } else {
+            TRY(ensure_grid(j.target, s));
+            const GridSet gs = grid_set(j.target, filtered);
+            rays.s[k] = {gs, j.target->tri64.p, j.pts, j.order, nullptr, n, rb.bits.p, rb.rayList.p, rb.ovf.p};
+            v.overflow = rb.ovf.p;
+            v.total = gs.cells + gs.ncells;
+            v.pubFlags = rb.host;
+            v.pubTotal = rb.host + 1;
+            if (!cleared) {
+                clear.p[k] = rb.ovf.p;
+                clear.n[k] = 4;
+            }
+        }
+        votes.s[k] = v;
     }
-    if (votes)
-        HIP_TRY(hipMemcpyAsync(*direct ? hostVotes : rb.votesHost.p, rb.votes.p, n, hipMemcpyDeviceToHost, rb.s));
+    Stage st(c, SBG_STAGE_CLASSIFY, s);
+    launch_clear(clear, s);
+    launch_rays(rays, ordered, allAxes, s);
+    launch_vote(votes, s);
+    TRY(check_launch("rays"));
+    for (int k = 0; k < njobs; ++k)
+        if (jobs[k].way == RayJob::kCopy)
+            HIP_TRY(hipMemcpyAsync(jobs[k].hostVotes, jobs[k].rb.votes.p, jobs[k].n, hipMemcpyDeviceToHost, s));
     return SBG_OK;
 }
 
-// After the stream has drained: SBG_OK, or `retry` when the grid turned out
-// too small (it is marked for a rebuild at its exact size), or an error.
-static int check_rays(sbg_mesh target, RayBufs rb, bool &retry)
+// After the stream has drained: SBG_OK with the votes in place, or `retry` when
+// the grid turned out too small (it is marked for a rebuild at its exact size),
+// or an error.
+static int finish_rays(const RayJob &j, bool &retry)
 {
     retry = false;
-    if (rb.host[0] & 2u) {
-        target->gridCap = (size_t)rb.host[1] + rb.host[1] / 16 + 1024;
-        target->gridReady = false;
+    if (j.rb.host[0] & 2u) {
+        j.target->gridCap = (size_t)j.rb.host[1] + j.rb.host[1] / 16 + 1024;
+        j.target->gridReady = false;
         retry = true;
         return SBG_OK;
     }
-    if (rb.host[0])
+    if (j.rb.host[0])
         return fail(SBG_ERR_OVERFLOW, "a ray has more distinct hits than its key list holds");
+    if (j.way == RayJob::kStaged)
+        std::memcpy(j.hostVotes, j.rb.votesHost.p, j.n);
     return SBG_OK;
 }
 
-// enqueue, wait, check; a grid that turned out too small is rebuilt at its
-// exact size and the rays run again
-static int run_rays(sbg_mesh target, RayBufs rb, const double *dpts, const uint32_t *dorder, const uint8_t *dskip,
-                    size_t n, bool ordered, bool allAxes, uint8_t *hostVotes)
+// Two sides share their launches up to this many queries in all; beyond, each
+// side is queued on a stream of its own.  A step shared / on two streams, us:
+// 372 / 428 at 160 triangles in all, 495 / 559 at 10,240, 566 / 602 at 163,840,
+// 573 / 610 at 339,000, 654 / 668 at 564,000, 804 / 799 at 655,360, 891 / 877
+// at 786,264, 1,790 / 1,698 at 2,621,440 (a large side's deferred rays, long
+// latencies on few waves, run beside the other side's fast rays there).
+constexpr size_t kSharedQueries = 600000;
+
+// enqueue, wait, check; a side whose grid turned out too small is run again
+// with the grid at its exact size.  The queries stand on the context stream.
+static int run_rays(RayJob *jobs, int njobs, bool ordered, bool allAxes, bool cleared)
 {
-    for (int attempt = 0; attempt < 2; ++attempt) {
-        bool direct = false;
-        TRY(enqueue_rays(target, rb, dpts, dorder, dskip, n, ordered, allAxes, hostVotes, &direct));
-        HIP_TRY(hipStreamSynchronize(rb.s));
-        bool retry = false;
-        TRY(check_rays(target, rb, retry));
-        if (!retry) {
-            if (hostVotes && !direct)
-                std::memcpy(hostVotes, rb.votesHost.p, n);
-            return SBG_OK;
-        }
+    sbg_context c = jobs[0].target->ctx;
+    if (njobs == 2 && jobs[0].n + jobs[1].n > kSharedQueries) {
+        const AuxJoin join{c};
+        HIP_TRY(hipEventRecord(c->auxReady, c->stream));
+        HIP_TRY(hipStreamWaitEvent(c->aux, c->auxReady, 0));
+        TRY(enqueue_rays(jobs, 1, ordered, allAxes, cleared, c->stream));
+        TRY(enqueue_rays(jobs + 1, 1, ordered, allAxes, cleared, c->aux));
+        HIP_TRY(hipStreamSynchronize(c->aux));
+    } else {
+        TRY(enqueue_rays(jobs, njobs, ordered, allAxes, cleared, c->stream));
     }
-    return fail(SBG_ERR_OVERFLOW, "ray grid did not fit after a resize");
+    HIP_TRY(hipStreamSynchronize(c->stream));
+    bool again[2] = {false, false};
+    for (int k = 0; k < njobs; ++k)
+        TRY(finish_rays(jobs[k], again[k]));
+    for (int k = 0; k < njobs; ++k)
+        if (again[k]) {
+            TRY(enqueue_rays(jobs + k, 1, ordered, allAxes, false, c->stream));
+            HIP_TRY(hipStreamSynchronize(c->stream));
+            bool still = false;
+            TRY(finish_rays(jobs[k], still));
+            if (still)
+                return fail(SBG_ERR_OVERFLOW, "ray grid did not fit after a resize");
+        }
+    return SBG_OK;
 }
 
 int sbg_classify_points(sbg_mesh target, const double *pts, size_t n, uint8_t *axis_inside, uint8_t *inside)
@@ -1580,7 +1629,8 @@ int sbg_classify_points(sbg_mesh target, const double *pts, size_t n, uint8_t *a
     TRY(c->bits.ensure(3 * n + 4));
     TRY(c->votes.ensure(n));
     HIP_TRY(hipMemcpyAsync(c->pts.p, pts, sizeof(double) * 3 * n, hipMemcpyHostToDevice, c->stream));
-    TRY(run_rays(target, ray_bufs(c, 0), c->pts.p, nullptr, nullptr, n, false, axis_inside != nullptr, inside));
+    RayJob job = {target, ray_bufs(c, 0), c->pts.p, nullptr, nullptr, n, inside, RayJob::kNone};
+    TRY(run_rays(&job, 1, false, axis_inside != nullptr, false));
     std::vector<uint8_t> bits;
     if (axis_inside) {
         bits.resize(3 * n);
@@ -1610,21 +1660,51 @@ static int check_classify_args(sbg_mesh self, sbg_mesh other, sbg_pairs p, int s
     return SBG_OK;
 }
 
-// the queries of sbg_classify_triangles(self, ..., side): intersected flags,
-// then the centroids of the others in visiting order, into rb
-static int enqueue_queries(sbg_mesh self, sbg_pairs p, int side, RayBufs rb)
+// The queries of sbg_classify_triangles for the sides given (self[k] null: not
+// wanted): intersected flags, then the centroids of the others in visiting
+// order, into the sides' buffers; clears the sides' ray counters on the way.
+static int enqueue_queries(sbg_context c, sbg_mesh self[2], sbg_pairs p, const RayBufs *rb[2])
 {
-    sbg_context c = self->ctx;
-    const size_t nt = self->nt;
-    TRY(rb.flags.ensure(nt + 4));
-    TRY(rb.pts.ensure(4 * nt));
-    TRY(rb.bits.ensure(3 * nt + 4));
-    TRY(rb.votes.ensure(nt));
-    Stage st(c, SBG_STAGE_CLASSIFY, rb.s);
-    launch_fill_u32((uint32_t *)rb.flags.p, 0u, (nt + 3) / 4, rb.s);
-    launch_mark_intersected(p->pairs.p, p->status.p, (uint32_t)p->n, side, rb.flags.p, rb.s);
-    launch_centroids_ordered(self->tri64.p, rb.flags.p, self->sortedIds, nullptr, (uint32_t)nt, rb.pts.p, rb.s);
+    ClearList clear = {};
+    QuerySides q = {};
+    for (int k = 0; k < 2; ++k) {
+        if (!self[k])
+            continue;
+        const size_t nt = self[k]->nt;
+        TRY(rb[k]->flags.ensure(nt + 4));
+        TRY(rb[k]->pts.ensure(4 * nt));
+        TRY(rb[k]->bits.ensure(3 * nt + 4));
+        TRY(rb[k]->votes.ensure(nt));
+        TRY(rb[k]->ovf.ensure(4));
+        clear.p[2 * k] = (uint32_t *)rb[k]->flags.p;
+        clear.n[2 * k] = (uint32_t)((nt + 3) / 4);
+        clear.p[2 * k + 1] = rb[k]->ovf.p;
+        clear.n[2 * k + 1] = 4;
+        q.s[k] = {self[k]->tri64.p, rb[k]->flags.p, self[k]->sortedIds, nullptr, (uint32_t)nt, rb[k]->pts.p};
+    }
+    Stage st(c, SBG_STAGE_CLASSIFY, c->stream);
+    launch_clear(clear, c->stream);
+    launch_mark_intersected(p->pairs.p, p->status.p, (uint32_t)p->n, nullptr, self[0] ? rb[0]->flags.p : nullptr,
+                            self[1] ? rb[1]->flags.p : nullptr, c->stream);
+    launch_centroids_ordered(q, c->stream);
     return check_launch("classify");
+}
+
+// the vote of every uncut triangle of the sides wanted: self[0] is the pairs'
+// first mesh, against `other`[0], self[1] the second
+static int classify_sides(sbg_mesh self[2], sbg_mesh other[2], sbg_pairs p, uint8_t *out[2])
+{
+    sbg_context c = p->ctx;
+    // a single side uses the first set of buffers, whichever it is
+    const RayBufs sets[2] = {ray_bufs(c, 0), ray_bufs(c, 1)};
+    const RayBufs *rb[2] = {&sets[0], &sets[self[0] ? 1 : 0]};
+    TRY(enqueue_queries(c, self, p, rb));
+    std::vector<RayJob> jobs;
+    for (int k = 0; k < 2; ++k)
+        if (self[k])
+            jobs.push_back({other[k], *rb[k], rb[k]->pts.p, self[k]->sortedIds, rb[k]->flags.p, self[k]->nt, out[k],
+                            RayJob::kNone});
+    return run_rays(jobs.data(), (int)jobs.size(), true, false, true);
 }
 
 int sbg_classify_triangles(sbg_mesh self, sbg_mesh other, sbg_pairs p, int side, uint8_t *out)
@@ -1632,14 +1712,16 @@ int sbg_classify_triangles(sbg_mesh self, sbg_mesh other, sbg_pairs p, int side,
     if (!self || !other || !p || !out)
         return fail(SBG_ERR_INVALID, "null argument");
     TRY(check_classify_args(self, other, p, side));
-    sbg_context c = self->ctx;
-    TRY(use(c));
+    TRY(use(self->ctx));
     MeshUse mu(self, other);
     if (!self->nt)
         return SBG_OK;
-    const RayBufs rb = ray_bufs(c, 0);
-    TRY(enqueue_queries(self, p, side, rb));
-    return run_rays(other, rb, rb.pts.p, self->sortedIds, rb.flags.p, self->nt, true, false, out);
+    sbg_mesh selfs[2] = {nullptr, nullptr}, others[2] = {nullptr, nullptr};
+    uint8_t *outs[2] = {nullptr, nullptr};
+    selfs[side] = self;
+    others[side] = other;
+    outs[side] = out;
+    return classify_sides(selfs, others, p, outs);
 }
 
 int sbg_classify_pair(sbg_mesh a, sbg_mesh b, sbg_pairs p, uint8_t *out_a, uint8_t *out_b)
@@ -1648,49 +1730,13 @@ int sbg_classify_pair(sbg_mesh a, sbg_mesh b, sbg_pairs p, uint8_t *out_a, uint8
         return fail(SBG_ERR_INVALID, "null argument");
     TRY(check_classify_args(a, b, p, 0));
     TRY(check_classify_args(b, a, p, 1));
-    sbg_context c = a->ctx;
-    TRY(use(c));
+    TRY(use(a->ctx));
     MeshUse mu(a, b);
-    AuxJoin join{c};
-    // side 0 on the context stream, side 1 on the second stream and scratch
-    // set, ordered after everything queued so far; one wait for both
-    const RayBufs ra = ray_bufs(c, 0), rb = ray_bufs(c, 1);
-    HIP_TRY(hipEventRecord(c->auxReady, c->stream));
-    HIP_TRY(hipStreamWaitEvent(c->aux, c->auxReady, 0));
-    // both sides' queries first, then both sides' rays: the second stream
-    // starts its work after a few launches instead of after the first side's
-    // whole sequence
-    if (a->nt)
-        TRY(enqueue_queries(a, p, 0, ra));
-    if (b->nt)
-        TRY(enqueue_queries(b, p, 1, rb));
-    bool directA = false, directB = false;
-    if (a->nt)
-        TRY(enqueue_rays(b, ra, ra.pts.p, a->sortedIds, ra.flags.p, a->nt, true, false, out_a, &directA));
-    if (b->nt)
-        TRY(enqueue_rays(a, rb, rb.pts.p, b->sortedIds, rb.flags.p, b->nt, true, false, out_b, &directB));
-    // each side's votes land in page-locked output arrays directly, or are
-    // copied out of the staging as soon as that side is done (the first
-    // side's copy overlapping the second side's GPU work); a side whose
-    // target grid turned out too small runs again on its own afterwards
-    bool retryA = false, retryB = false;
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    if (a->nt) {
-        TRY(check_rays(b, ra, retryA));
-        if (!retryA && !directA)
-            std::memcpy(out_a, ra.votesHost.p, a->nt);
-    }
-    HIP_TRY(hipStreamSynchronize(c->aux));
-    if (b->nt) {
-        TRY(check_rays(a, rb, retryB));
-        if (!retryB && !directB)
-            std::memcpy(out_b, rb.votesHost.p, b->nt);
-    }
-    if (retryA)
-        TRY(run_rays(b, ra, ra.pts.p, a->sortedIds, ra.flags.p, a->nt, true, false, out_a));
-    if (retryB)
-        TRY(run_rays(a, rb, rb.pts.p, b->sortedIds, rb.flags.p, b->nt, true, false, out_b));
-    return SBG_OK;
+    sbg_mesh selfs[2] = {a->nt ? a : nullptr, b->nt ? b : nullptr}, others[2] = {b, a};
+    uint8_t *outs[2] = {out_a, out_b};
+    if (!selfs[0] && !selfs[1])
+        return SBG_OK;
+    return classify_sides(selfs, others, p, outs);
 }
 
 int sbg_context_set_tuning(sbg_context ctx, const sbg_tuning *t)
@@ -1937,11 +1983,21 @@ static int bench_rays_setup(sbg_mesh self, sbg_mesh other, sbg_pairs p, int side
     TRY(c->rayList.ensure(ray_list_u32(nt)));
     TRY(c->workCounts.ensure(4));
     launch_fill_u32((uint32_t *)c->flags.p, 0u, (nt + 3) / 4, c->stream);
-    launch_mark_intersected(p->pairs.p, p->status.p, (uint32_t)p->n, side, c->flags.p, c->stream);
-    launch_centroids_ordered(self->tri64.p, c->flags.p, self->sortedIds, nullptr, (uint32_t)nt, c->pts.p, c->stream);
+    launch_mark_intersected(p->pairs.p, p->status.p, (uint32_t)p->n, nullptr, side == 0 ? c->flags.p : nullptr,
+                            side == 1 ? c->flags.p : nullptr, c->stream);
+    launch_centroids_ordered({{{self->tri64.p, c->flags.p, self->sortedIds, nullptr, (uint32_t)nt, c->pts.p},
+                               QuerySide{}}},
+                             c->stream);
     TRY(ensure_grid(other, c->stream));
     empty = false;
     return SBG_OK;
+}
+
+static RaySide bench_rays_side(sbg_mesh self, sbg_mesh other)
+{
+    sbg_context c = self->ctx;
+    return {grid_set(other, c->tune.ray_precision == SBG_PRECISION_FP32_FILTERED), other->tri64.p, c->pts.p,
+            self->sortedIds, nullptr, (uint32_t)self->nt, c->bits.p, c->rayList.p, c->ovf.p};
 }
 
 extern "C" {
@@ -1962,20 +2018,18 @@ int sbg_bench_rays(sbg_mesh self, sbg_mesh other, sbg_pairs p, int side, int ite
     if (empty)
         return SBG_OK;
     sbg_context c = self->ctx;
-    const size_t nt = self->nt;
-    const GridSet gs = grid_set(other, c->tune.ray_precision == SBG_PRECISION_FP32_FILTERED);
+    const RaySide side0 = bench_rays_side(self, other);
     std::vector<hipEvent_t> ev(2 * (size_t)iters, nullptr);
     for (auto &e : ev)
         HIP_TRY(hipEventCreate(&e));
     for (int i = 0; i < iters; ++i) {
         launch_fill_u32(c->ovf.p, 0u, 4, c->stream);
         HIP_TRY(hipEventRecord(ev[2 * i], c->stream));
-        launch_rays_xy_ordered(gs, other->tri64.p, c->pts.p, self->sortedIds, (uint32_t)nt, c->bits.p, c->rayList.p,
-                               c->ovf.p, c->stream);
+        launch_rays_xy_ordered(side0, c->stream);
         HIP_TRY(hipEventRecord(ev[2 * i + 1], c->stream));
     }
     launch_fill_u32((uint32_t *)c->workCounts.p, 0u, 8, c->stream);
-    launch_ray_work_ordered(gs, c->pts.p, self->sortedIds, (uint32_t)nt, c->workCounts.p, c->stream);
+    launch_ray_work_ordered(side0, c->workCounts.p, c->stream);
     uint64_t h[4] = {0, 0, 0, 0};
     uint32_t deferred = 0;  // rays the last timed launch handed to the wave kernel
     HIP_TRY(hipMemcpyAsync(h, c->workCounts.p, sizeof(h), hipMemcpyDeviceToHost, c->stream));
@@ -2013,18 +2067,15 @@ int sbg_bench_rays_wave(sbg_mesh self, sbg_mesh other, sbg_pairs p, int side, in
     if (empty)
         return SBG_OK;
     sbg_context c = self->ctx;
-    const uint32_t nt = (uint32_t)self->nt;
-    const GridSet gs = grid_set(other, c->tune.ray_precision == SBG_PRECISION_FP32_FILTERED);
+    const RaySide side0 = bench_rays_side(self, other);
     launch_fill_u32(c->ovf.p, 0u, 4, c->stream);
-    launch_rays_xy_ordered(gs, other->tri64.p, c->pts.p, self->sortedIds, nt, c->bits.p, c->rayList.p, c->ovf.p,
-                           c->stream);
+    launch_rays_xy_ordered(side0, c->stream);
     hipEvent_t e0, e1;
     HIP_TRY(hipEventCreate(&e0));
     HIP_TRY(hipEventCreate(&e1));
     HIP_TRY(hipEventRecord(e0, c->stream));
     for (int i = 0; i < iters; ++i)
-        launch_rays_wave_ordered(gs, other->tri64.p, c->pts.p, self->sortedIds, nt, c->bits.p, c->rayList.p,
-                                 c->ovf.p, c->stream);
+        launch_rays_wave_ordered(side0, c->stream);
     HIP_TRY(hipEventRecord(e1, c->stream));
     uint32_t deferred = 0;
     HIP_TRY(hipMemcpyAsync(&deferred, c->ovf.p + 1, sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
@@ -2189,16 +2240,19 @@ int sbg_classify_points_noalloc(sbg_mesh target, const double *pts, size_t n, ui
     uint32_t *host = c->pinned + kRayPinned;  // page-locked words made with the context
     host[0] = 0;
     HIP_TRY(hipMemcpyAsync(dpts, pts, sizeof(double) * 3 * n, hipMemcpyHostToDevice, s));
+    VoteSide vote = {bits, nullptr, (uint32_t)n, votes, nullptr, nullptr, nullptr, nullptr};
     if (target->nt == 0) {
         launch_fill_u32(reinterpret_cast<uint32_t *>(bits), 0u, (3 * n + 3) / 4, s);
     } else {
         launch_fill_u32(counters, 0u, 4, s);  // kernels, not memsets: the call may be captured
-        launch_rays(grid_set(target, c->tune.ray_precision == SBG_PRECISION_FP32_FILTERED), target->tri64.p, dpts,
-                    nullptr, nullptr, (uint32_t)n, allAxes, bits, lists,
-                    counters, s);
-        HIP_TRY(hipMemcpyAsync(host, counters, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+        launch_rays({{{grid_set(target, c->tune.ray_precision == SBG_PRECISION_FP32_FILTERED), target->tri64.p, dpts,
+                       nullptr, nullptr, (uint32_t)n, bits, lists, counters},
+                      RaySide{}}},
+                    false, allAxes, s);
+        vote.overflow = counters;
+        vote.pubFlags = host;
     }
-    launch_vote(bits, nullptr, (uint32_t)n, votes, s);
+    launch_vote({{vote, VoteSide{}}}, s);
     if (allAxes)
         launch_interleave_axes(bits, (uint32_t)n, axes, s);
     TRY(check_launch("allocation-free rays"));

@@ -93,7 +93,6 @@ void launch_tree64(const uint64_t *codes, const uint32_t *ids, const float *box3
                    uint32_t *work, float *scratch, float *rootBox, hipStream_t s);
 void launch_fill_u32(uint32_t *p, uint32_t value, size_t n, hipStream_t s);
 void launch_copy16(const void *src, void *dst, size_t n16, hipStream_t s);
-void launch_copy_u32(const uint32_t *src, uint32_t *dst, size_t n, hipStream_t s);
 
 // k_traverse.hip
 struct TraverseArgs {
@@ -156,9 +155,13 @@ void launch_compact_hits(const uint64_t *pairs, const uint8_t *status, const dou
 int compact_blocks(uint32_t n);
 
 // k_classify.hip
-void launch_mark_intersected(const uint64_t *pairs, const uint8_t *status, uint32_t n, int side,
-                             uint8_t *flags, hipStream_t s);
-void launch_centroids(const double *tri64, const uint8_t *flags, uint32_t nt, double *pts, hipStream_t s);
+void launch_mark_intersected(const uint64_t *pairs, const uint8_t *status, uint32_t n, const uint32_t *count,
+                             uint8_t *flagsA, uint8_t *flagsB, hipStream_t s);
+struct ClearList {
+    uint32_t *p[4];
+    uint32_t n[4];
+};
+void launch_clear(const ClearList &list, hipStream_t s);
 // Per-axis projection grids of one or more target meshes sharing one cell
 // array (ncells cells + 1 total) and one entry array (cap entries).
 struct GridSet {
@@ -186,40 +189,69 @@ void launch_grid_build(const float *box32, uint32_t nt, const GridSet &gs, uint3
                        uint2 *gcode, uint32_t *gtri, uint32_t maxBlocks, hipStream_t s);
 // the single-pair build's cap: it runs beside the pair search
 constexpr uint32_t kGridBesideSearch = 256;
-// order (may be null): query q uses point order[q].  allAxes: cast x, y and z
-// for every query; otherwise x and y, and z only where they disagree (the
-// vote's answer is the same; z's bits are then valid only there).  lists:
-// ray_list_u32(n) u32 of scratch; counters: 4 u32, zero on entry, counters[0] gets the
-// overflow bits (bit 0: a ray has too many distinct hits, bit 1: the grid was
-// truncated, cells[ncells] > cap).  tri64 records carry the FP64 normal in
-// their pad slots.
+// The two sides of a boolean's classification share every launch (n = 0: no
+// such side).  One side's rays: n queries against one target's grid; query q
+// uses point order[q] (order may be null; visiting-order queries hold (x, y, z,
+// tag) at 4q instead, tag being the target mesh, or skip / no target), and
+// those flagged in skip (by output index; may be null) are left out.
+// Per-axis bits go to bits[axis][n] by output index; lists: ray_list_u32(n) u32
+// of scratch; counters: 4 u32, zero on entry, counters[0] gets the overflow
+// bits (bit 0: a ray has too many distinct hits, bit 1: the grid was truncated,
+// cells[ncells] > cap).  tri64: the target's records, which carry the FP64
+// normal in their pad slots.
+struct RaySide {
+    GridSet gs;
+    const double *tri64, *pts;
+    const uint32_t *order;
+    const uint8_t *skip;
+    uint32_t n;
+    uint8_t *bits;
+    uint32_t *lists, *counters;
+};
+struct RaySides {
+    RaySide s[2];
+};
 size_t ray_list_u32(size_t n);
+// ordered: visiting-order queries.  allAxes: cast x, y and z for every query;
+// otherwise x and y, and z only where they disagree (the vote's answer is the
+// same; z's bits are then valid only there).
+void launch_rays(const RaySides &r, bool ordered, bool allAxes, hipStream_t s);
 // per-axis bits [axis][n] -> [n][3]
 void launch_interleave_axes(const uint8_t *axisBits, uint32_t n, uint8_t *out, hipStream_t s);
-void launch_rays(const GridSet &gs, const double *tri64, const double *pts, const uint32_t *order,
-                 const uint8_t *skip, uint32_t n, bool allAxes, uint8_t *axisBits, uint32_t *lists,
-                 uint32_t *counters, hipStream_t s);
-// Visiting-order queries: q4 holds 4 nt doubles, (x, y, z, tag) of triangle
-// order[q] at 4q (tag: target mesh, or skip where flags is given / no
-// target); the rays write axisBits by triangle like launch_rays and leave out
-// the queries tagged skip or flagged in skip (by triangle; may be null).
-void launch_centroids_ordered(const double *tri64, const uint8_t *flags, const uint32_t *order,
-                              const uint32_t *target, uint32_t nt, double *q4, hipStream_t s);
-void launch_rays_ordered(const GridSet &gs, const double *tri64, const double *q4, const uint32_t *order,
-                         const uint8_t *skip, uint32_t n, bool allAxes, uint8_t *axisBits, uint32_t *lists,
-                         uint32_t *counters, hipStream_t s);
-// measurement: the x/y fast ray kernel alone (lists: ray_list_u32(n) u32, counters: 4 u32
-// zero on entry), and the work counts of one such launch (work: 4 u64, zero on
-// entry: rays cast, entries scanned, entries passing the code test, deferred)
-void launch_rays_xy_ordered(const GridSet &gs, const double *tri64, const double *q4, const uint32_t *order,
-                            uint32_t n, uint8_t *axisBits, uint32_t *lists, uint32_t *counters, hipStream_t s);
-// the wave kernel alone over the rays launch_rays_xy_ordered deferred (same
-// lists and counters)
-void launch_rays_wave_ordered(const GridSet &gs, const double *tri64, const double *q4, const uint32_t *order,
-                              uint32_t n, uint8_t *axisBits, const uint32_t *lists, uint32_t *counters, hipStream_t s);
-void launch_ray_work_ordered(const GridSet &gs, const double *q4, const uint32_t *order, uint32_t n,
-                             unsigned long long *work, hipStream_t s);
-void launch_vote(const uint8_t *axisBits, const uint8_t *skip, uint32_t n, uint8_t *out, hipStream_t s);
+// Visiting-order queries of a mesh's triangles: q4 holds 4 nt doubles, (x, y, z,
+// tag) of triangle order[q] at 4q (skip where flags is given and set).
+struct QuerySide {
+    const double *tri64;
+    const uint8_t *flags;
+    const uint32_t *order, *target;
+    uint32_t nt;
+    double *q4;
+};
+struct QuerySides {
+    QuerySide s[2];
+};
+void launch_centroids_ordered(const QuerySides &sides, hipStream_t s);
+// measurement: the x/y fast ray kernel alone, the wave kernel alone over the
+// rays that one deferred, and the work counts of one x/y launch (work: 4 u64,
+// zero on entry: rays cast, entries scanned, entries passing the code test,
+// deferred)
+void launch_rays_xy_ordered(const RaySide &r, hipStream_t s);
+void launch_rays_wave_ordered(const RaySide &r, hipStream_t s);
+void launch_ray_work_ordered(const RaySide &r, unsigned long long *work, hipStream_t s);
+// the votes of n queries' bits, 2 where skip (may be null) is set; out may be
+// page-locked host memory, as may pubFlags and pubTotal (null: not wanted),
+// which get *overflow and *total
+struct VoteSide {
+    const uint8_t *bits, *skip;
+    uint32_t n;
+    uint8_t *out;
+    const uint32_t *overflow, *total;
+    uint32_t *pubFlags, *pubTotal;
+};
+struct VoteSides {
+    VoteSide s[2];
+};
+void launch_vote(const VoteSides &sides, hipStream_t s);
 
 // k_components.hip: triangle components across opposite half-edges
 size_t component_table_slots(uint32_t nt);
@@ -250,7 +282,5 @@ void launch_mesh_roots(const BNode *nodes, const uint32_t *ids, const uint32_t *
 void launch_batch_seed(const TraverseArgs &t, const uint32_t *meshRoot, const float *meshBox, uint32_t npairs,
                        uint2 *frontier, uint32_t *frontCount, uint32_t frontCap, uint64_t *cand, uint32_t *candCount,
                        uint32_t candCap, uint32_t *overflow, hipStream_t s);
-void launch_mark_both(const uint64_t *pairs, const uint8_t *status, const uint32_t *count, uint32_t cap,
-                      uint8_t *flags, hipStream_t s);
 
 }  // namespace sbg

@@ -659,6 +659,49 @@ def test_search_from_tiles(gpu, na, nb):
         assert np.array_equal(X.find_pairs(Y).array().astype(np.int64), want)
 
 
+@pytest.mark.parametrize("na,nb", [(1, 1), (1, 2), (2, 3), (255, 256), (257, 1021)])
+def test_classify_pair_ragged_sides(gpu, na, nb):
+    """classify_pair over sides that end anywhere in the vote kernel's groups of
+    four and the launches' workgroups of 256, into page-locked arrays at odd
+    offsets and into ordinary ones: the two single-side calls' answers, and
+    nothing written past a side's end."""
+    rng = np.random.default_rng(na + nb)
+
+    def soup(n):
+        c = rng.random((n, 1, 3))
+        return mg.Mesh((c + 0.2 * rng.random((n, 3, 3))).reshape(-1, 3), np.arange(3 * n).reshape(-1, 3))
+
+    a, b = soup(na), soup(nb)
+    A, B = gpu.mesh(a.vertices, a.triangles), gpu.mesh(b.vertices, b.triangles)
+    P = A.find_pairs(B)
+    P.tri_tri(A, B, N.FP32_FILTERED)
+    wa, wb = A.classify_triangles(B, P, 0), B.classify_triangles(A, P, 1)
+    for make in (lambda n: N.host_array(n), lambda n: np.zeros(n, np.uint8)):
+        for lead in (0, 1, 3):
+            bufs = [make(lead + n + 5) for n in (na, nb)]
+            for x in bufs:
+                x[:] = 77
+            got = A.classify_pair(B, P, out=tuple(x[lead:] for x in bufs))
+            assert np.array_equal(got[0], wa) and np.array_equal(got[1], wb)
+            for x, n in zip(bufs, (na, nb)):
+                assert np.all(x[:lead] == 77) and np.all(x[lead + n:] == 77)
+
+
+def test_classify_pair_split_sides(gpu):
+    """A pair past the size up to which both sides share their launches, and
+    one just below: votes equal to the single-side calls'."""
+    for size in (250, 270):
+        a = mg.torus(1.0, 0.3, 2 * size, size)
+        b = mg.transform(mg.torus(1.0, 0.25, 2 * size + 3, size), mg.random_rotation(mg.SplitMix64(size)),
+                         (0.5, 0.1, 0.1))
+        A, B = gpu.mesh(a.vertices, a.triangles), gpu.mesh(b.vertices, b.triangles)
+        P = A.find_pairs(B)
+        P.tri_tri(A, B, N.FP32_FILTERED)
+        va, vb = A.classify_pair(B, P)
+        assert np.array_equal(va, A.classify_triangles(B, P, 0)) and np.array_equal(vb, B.classify_triangles(A, P, 1))
+        assert {0, 1, 2} <= set(va.tolist()) and {0, 1, 2} <= set(vb.tolist())
+
+
 def test_components_vs_oracle(gpu):
     """sbg_components against the oracle's restatement of the reference's face
     grouping: whole meshes, blocked bands, random blocked sets, several
