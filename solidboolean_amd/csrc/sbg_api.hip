@@ -118,6 +118,7 @@ struct sbg_pairs_s {
     DevBuf<double> seg, hitSeg;
     DevBuf<uint64_t> hitPairs;
     DevBuf<uint32_t> blockCounts, nHits, work;
+    PinnedBuf hostHits;   // the compaction's hit count, valid once its stream is done
     bool tested = false;
     // largest first / second index in the list (host-built lists are checked
     // against the meshes before any kernel indexes them)
@@ -302,6 +303,7 @@ static void pairs_free_buffers(sbg_pairs p)
     p->hitPairs.release();
     p->blockCounts.release();
     p->nHits.release();
+    p->hostHits.release();
     p->work.release();
 }
 
@@ -355,6 +357,7 @@ void context_free(sbg_context ctx)
     ctx->ovf2.release();
     ctx->rayList2.release();
     ctx->votesHost.release();
+    ctx->hitStage.release();
     ctx->votesHost2.release();
     ctx->workCounts.release();
     ctx->ccKeys.release();
@@ -1247,6 +1250,7 @@ static int run_tri_tri(sbg_mesh a, sbg_mesh b, sbg_pairs p, int precision, GdSta
     TRY(p->hitSeg.ensure(6 * p->n));
     TRY(p->blockCounts.ensure((size_t)compact_blocks(n)));
     TRY(p->nHits.ensure(1));
+    TRY(p->hostHits.ensure(sizeof(uint32_t)));
     TRY(p->work.ensure(tritri_work_u32((uint32_t)p->n)));
     {
         Stage st(c, SBG_STAGE_TRI_TRI);
@@ -1259,7 +1263,7 @@ static int run_tri_tri(sbg_mesh a, sbg_mesh b, sbg_pairs p, int precision, GdSta
         if (n == 0)  // otherwise the compaction's last block writes the count
             launch_fill_u32(p->nHits.p, 0u, 1, c->stream);
         launch_compact_hits(p->pairs.p, p->status.p, p->seg.p, n, p->blockCounts.p, p->hitPairs.p, p->hitSeg.p,
-                            p->nHits.p, c->stream);
+                            p->nHits.p, (uint32_t *)p->hostHits.p, c->stream);
         TRY(check_launch("compact"));
     }
     return SBG_OK;
@@ -1326,28 +1330,43 @@ int sbg_pairs_hits(sbg_pairs p, size_t *nhits, uint32_t *ab, double *seg)
         return fail(SBG_ERR_INVALID, "null argument");
     if (!p->tested)
         return fail(SBG_ERR_STATE, "sbg_tri_tri has not run on this pair list");
-    TRY(use(p->ctx));
+    sbg_context c = p->ctx;
+    TRY(use(c));
     *nhits = 0;
     if (!p->n)
         return SBG_OK;
-    uint32_t h = 0;
-    HIP_TRY(hipMemcpyAsync(&h, p->nHits.p, sizeof(uint32_t), hipMemcpyDeviceToHost, p->ctx->stream));
-    HIP_TRY(hipStreamSynchronize(p->ctx->stream));
+    HIP_TRY(hipStreamSynchronize(c->stream));
+    const uint32_t h = *(const uint32_t *)p->hostHits.p;
     *nhits = h;
     if (!h || (!ab && !seg))
         return SBG_OK;
+    const size_t abBytes = 2 * sizeof(uint32_t) * (size_t)h, segBytes = 6 * sizeof(double) * (size_t)h;
+    if (abBytes + segBytes <= kHitStage) {
+        // one kernel writes both lists to page-locked staging
+        TRY(c->hitStage.ensure(kHitStage));
+        double *stSeg = (double *)c->hitStage.p;
+        uint32_t *stAb = (uint32_t *)(c->hitStage.p + segBytes);
+        launch_hit_export(p->hitPairs.p, p->hitSeg.p, h, ab ? stAb : nullptr, seg ? stSeg : nullptr, c->stream);
+        TRY(check_launch("hit export"));
+        HIP_TRY(hipStreamSynchronize(c->stream));
+        if (ab)
+            std::memcpy(ab, stAb, abBytes);
+        if (seg)
+            std::memcpy(seg, stSeg, segBytes);
+        return SBG_OK;
+    }
     if (ab) {
         std::vector<uint64_t> v(h);
-        HIP_TRY(hipMemcpyAsync(v.data(), p->hitPairs.p, sizeof(uint64_t) * h, hipMemcpyDeviceToHost, p->ctx->stream));
-        HIP_TRY(hipStreamSynchronize(p->ctx->stream));
+        HIP_TRY(hipMemcpyAsync(v.data(), p->hitPairs.p, sizeof(uint64_t) * h, hipMemcpyDeviceToHost, c->stream));
+        HIP_TRY(hipStreamSynchronize(c->stream));
         for (uint32_t i = 0; i < h; ++i) {
             ab[2 * i] = (uint32_t)(v[i] >> 32);
             ab[2 * i + 1] = (uint32_t)v[i];
         }
     }
     if (seg) {
-        HIP_TRY(hipMemcpyAsync(seg, p->hitSeg.p, sizeof(double) * 6 * h, hipMemcpyDeviceToHost, p->ctx->stream));
-        HIP_TRY(hipStreamSynchronize(p->ctx->stream));
+        HIP_TRY(hipMemcpyAsync(seg, p->hitSeg.p, segBytes, hipMemcpyDeviceToHost, c->stream));
+        HIP_TRY(hipStreamSynchronize(c->stream));
     }
     return SBG_OK;
 }

@@ -105,6 +105,9 @@ constexpr uint64_t kTilePairsMax = (uint64_t)1 << 26;
 // longest run of one first triangle the quick pair sort orders by insertion
 constexpr uint32_t kSortRunMax = 64;
 constexpr uint32_t kSpillInit = 2048, kSpillMax = 1u << 15;
+// intersecting pairs and segments up to this size leave through page-locked
+// staging (74,898 of them)
+constexpr size_t kHitStage = (size_t)4 << 20;
 // sbg_mesh_create's uploads: host threads that fill page-locked staging (two
 // slots each), the slot size, and the smallest share worth a thread of its own
 constexpr int kUploadThreads = 8;
@@ -149,6 +152,7 @@ struct sbg_context_s {
     DevBuf<uint8_t> flags, bits, votes, flags2, bits2, votes2;
     DevBuf<uint32_t> ovf, rayList, ovf2, rayList2;
     PinnedBuf votesHost, votesHost2;  // vote readbacks of the two sets
+    PinnedBuf hitStage;               // sbg_pairs_hits: kHitStage bytes
     DevBuf<unsigned long long> workCounts;  // sbg_bench_rays
     DevBuf<unsigned long long> ccKeys;      // sbg_half_edges: half-edge table
     DevBuf<uint32_t> ccOwners;

@@ -702,6 +702,32 @@ def test_classify_pair_split_sides(gpu):
         assert {0, 1, 2} <= set(va.tolist()) and {0, 1, 2} <= set(vb.tolist())
 
 
+@pytest.mark.parametrize("n,share", [(1, 1.0), (255, 0.3), (256, 0.3), (257, 0.0), (4097, 0.5), (131072, 0.5),
+                                     (131073, 0.5), (140000, 0.02), (76000, 1.0)])
+def test_hits_compaction(gpu, n, share):
+    """The hit lists of pair lists around the compaction's workgroup and
+    one-launch sizes and the readback's staging size: exactly the pairs of
+    status 1 with their segments, in order, asked twice and with a second list
+    tested in between."""
+    a, b = mg.small_pair(1)
+    A, B = gpu.mesh(a.vertices, a.triangles), gpu.mesh(b.vertices, b.triangles)
+    P = A.find_pairs(B)
+    P.tri_tri(A, B, N.FP64)
+    known, status = P.array(), P.results()[0]
+    rng = np.random.default_rng(n)
+    hit = rng.random(n) < share
+    pick = np.where(hit, rng.choice(np.nonzero(status == 1)[0], n), rng.choice(np.nonzero(status != 1)[0], n))
+    Q = gpu.pairs(known[pick])
+    Q.tri_tri(A, B, N.FP64, stats=False)
+    P.tri_tri(A, B, N.FP32_FILTERED, stats=False)
+    st, seg = Q.results()
+    assert np.array_equal(st == 1, hit)
+    for _ in range(2):
+        hp, hs = Q.hits()
+        assert np.array_equal(hp, known[pick][hit]) and np.array_equal(bits(hs), bits(seg[hit]))
+    assert len(P.hits()[0]) == int((status == 1).sum())
+
+
 def test_components_vs_oracle(gpu):
     """sbg_components against the oracle's restatement of the reference's face
     grouping: whole meshes, blocked bands, random blocked sets, several
