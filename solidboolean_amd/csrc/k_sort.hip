@@ -9,12 +9,17 @@
 // and scatters.  ITEMS shrinks with n so that short sorts still spread over
 // many workgroups.  Per key and pass: read 4 (8) B key (+4 B value) twice,
 // write once.
+#include "sbg_device.h"
 #include "sbg_internal.h"
 
 namespace sbg {
 
 constexpr int kSortBlock = 256;
 constexpr int kWaves = kSortBlock / 64;
+
+// up to this many blocks the scatter kernel sums the histogram itself, and the
+// pass needs no scan kernel (a launch of 3 us and its gap)
+constexpr int kScanInScatter = 64;
 
 // keys per thread for a sort of n keys
 static int sort_items(size_t n) { return n >= ((size_t)1 << 20) ? 16 : (n >= ((size_t)1 << 17) ? 8 : 4); }
@@ -84,6 +89,8 @@ __global__ __launch_bounds__(1024) void k_scan(uint32_t *__restrict__ data, size
 // Tiles of 4096 entries (16 per thread): tile sums, a one-block scan of the
 // sums, then each tile rescans its entries from its base.
 constexpr int kScanTile = 4096;
+// up to this many entries one workgroup scans alone (a launch for three)
+constexpr size_t kScanOneBlock = 16384;
 
 __global__ __launch_bounds__(256) void k_scan_tile_sum(const uint32_t *__restrict__ data, size_t m,
                                                        uint32_t *__restrict__ tileSum)
@@ -143,6 +150,10 @@ void launch_scan_large(uint32_t *data, size_t m, uint32_t *temp, hipStream_t s)
 {
     if (m == 0)
         return;
+    if (m <= kScanOneBlock) {
+        hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, s, data, m);
+        return;
+    }
     const size_t tiles = (m + kScanTile - 1) / kScanTile;
     hipLaunchKernelGGL(k_scan_tile_sum, dim3((unsigned)tiles), dim3(256), 0, s, data, m, temp);
     hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, s, temp, tiles);
@@ -180,6 +191,8 @@ __global__ __launch_bounds__(256) void k_scan_rows(uint32_t *__restrict__ hist, 
         rowTotal[blockIdx.x] = s[255];
 }
 
+// rowTotal null: `offsets` still holds the blocks' digit counts (at most
+// kScanInScatter blocks), and every block sums up the ones it needs itself.
 template <typename K, bool HAS_VAL, int ITEMS>
 __global__ __launch_bounds__(kSortBlock) void k_scatter(const K *__restrict__ keys, const uint32_t *__restrict__ vals,
                                                         K *__restrict__ keysOut, uint32_t *__restrict__ valsOut,
@@ -201,7 +214,19 @@ __global__ __launch_bounds__(kSortBlock) void k_scatter(const K *__restrict__ ke
         vreg[r] = (HAS_VAL && idx < n) ? vals[idx] : 0u;
     }
     // digit bases: exclusive scan of the 256 row totals
-    const uint32_t total = rowTotal[threadIdx.x];
+    uint32_t total = 0, earlier = 0;
+    if (rowTotal) {
+        total = rowTotal[threadIdx.x];
+        earlier = offsets[(size_t)threadIdx.x * nblocks + blockIdx.x];
+    } else {
+        const uint32_t *row = offsets + (size_t)threadIdx.x * nblocks;
+#pragma unroll 8
+        for (int b = 0; b < nblocks; ++b) {
+            const uint32_t v = row[b];
+            total += v;
+            earlier += b < (int)blockIdx.x ? v : 0u;
+        }
+    }
     s_base[threadIdx.x] = total;
     __syncthreads();
     for (int off = 1; off < 256; off <<= 1) {
@@ -212,7 +237,7 @@ __global__ __launch_bounds__(kSortBlock) void k_scatter(const K *__restrict__ ke
     }
     const uint32_t digitBase = s_base[threadIdx.x] - total;
     __syncthreads();
-    s_base[threadIdx.x] = digitBase + offsets[(size_t)threadIdx.x * nblocks + blockIdx.x];
+    s_base[threadIdx.x] = digitBase + earlier;
     for (int w = 0; w < kWaves; ++w)
         s_wcnt[w][threadIdx.x] = 0;
     __syncthreads();
@@ -303,6 +328,194 @@ void launch_sort_runs(uint64_t *keys, size_t n, const uint32_t *count, uint32_t 
                            maxRun, flag);
 }
 
+// ---- sorts of one workgroup ---------------------------------------------------
+// Short lists: a launch per pass and kernel (3 to 4 us of work each, as much
+// again of host time) cost more than the sort.  One workgroup of 16 waves keeps
+// the keys in LDS.  Per pass each wave counts the digits of its own run of
+// consecutive keys, 256 lanes turn the counts into offsets, and each wave then
+// places its run in order, 64 keys a round (ranks by ballots), with no barrier
+// between rounds.  A step with / without them, us: 231 / 310 at two 80-triangle
+// meshes (the order kernel 9.1 us for 11 launches of 2 to 4.4, the candidates'
+// 8.9 for four), 315 / 387 at 1,280, 357 / 436 at 5,120, 360 / 431 at 8,366;
+// the limit is what LDS holds.
+constexpr int kOneSortWaves = 16;
+constexpr uint32_t kOneSortMax = 8192;
+
+// one stable pass over n keys by digit_at(i) from src order to dst order:
+// place(i, slot) moves the i-th key.  s_cnt: [kOneSortWaves][256]
+template <typename DigitAt, typename Place>
+__device__ __forceinline__ void one_sort_pass(uint32_t n, uint32_t (*s_cnt)[256], uint32_t *s_scan,
+                                              const DigitAt &digit_at, const Place &place)
+{
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    for (uint32_t k = tid; k < kOneSortWaves * 256u; k += 64 * kOneSortWaves)
+        s_cnt[k >> 8][k & 255] = 0;
+    __syncthreads();
+    const uint32_t per = ((n + kOneSortWaves - 1) / kOneSortWaves + 63u) & ~63u;  // a wave's run
+    const uint32_t first = min(wave * per, n), last = min(first + per, n);
+    for (uint32_t i = first + lane; i < last; i += 64)
+        atomicAdd(&s_cnt[wave][digit_at(i)], 1u);
+    __syncthreads();
+    uint32_t total = 0;
+    if (tid < 256) {
+        for (int w = 0; w < kOneSortWaves; ++w) {
+            const uint32_t v = s_cnt[w][tid];
+            s_cnt[w][tid] = total;
+            total += v;
+        }
+        s_scan[tid] = total;
+    }
+    __syncthreads();
+    for (int off = 1; off < 256; off <<= 1) {
+        const uint32_t v = tid < 256 && tid >= (uint32_t)off ? s_scan[tid - off] : 0u;
+        __syncthreads();
+        if (tid < 256)
+            s_scan[tid] += v;
+        __syncthreads();
+    }
+    if (tid < 256) {
+        const uint32_t base = s_scan[tid] - total;
+        for (int w = 0; w < kOneSortWaves; ++w)
+            s_cnt[w][tid] += base;
+    }
+    __syncthreads();
+    const unsigned long long below = (1ull << lane) - 1ull;
+    for (uint32_t i0 = first; i0 < last; i0 += 64) {  // uniform over the wave
+        const uint32_t i = i0 + lane;
+        const bool valid = i < last;
+        const uint32_t d = valid ? digit_at(i) : 0u;
+        unsigned long long peers = __ballot(valid);
+        for (int b = 0; b < 8; ++b) {
+            const unsigned long long bal = __ballot((d >> b) & 1u);
+            peers &= (d >> b) & 1u ? bal : ~bal;
+        }
+        if (valid) {
+            const uint32_t slot = s_cnt[wave][d] + (uint32_t)__popcll(peers & below);
+            place(i, slot);
+            // the last of the equal ones moves the wave's offset on
+            if ((peers >> lane) == 1ull)
+                s_cnt[wave][d] = slot + 1u;
+        }
+        // the next round's lanes read the offsets this round's moved on
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+    __syncthreads();
+}
+
+// The tree order of a small mesh in one launch: the centroids' bounds from the
+// records kernel's blocks, Morton keys, and their sort; *zero is cleared for
+// the tree kernel.
+__global__ __launch_bounds__(64 * kOneSortWaves) void k_small_order(const float *__restrict__ box32,
+                                                                    const float *__restrict__ blockBounds, int nblocks,
+                                                                    uint32_t n, int keyBits, uint32_t *__restrict__ keys,
+                                                                    uint32_t *__restrict__ vals,
+                                                                    uint32_t *__restrict__ zero)
+{
+    __shared__ uint32_t s_key[2][kOneSortMax];
+    __shared__ uint16_t s_val[2][kOneSortMax];
+    __shared__ uint32_t s_cnt[kOneSortWaves][256], s_scan[256];
+    __shared__ float s_bounds[6];
+    const uint32_t tid = threadIdx.x;
+    if (tid < 64) {
+        float v[6] = {__builtin_inff(), __builtin_inff(), __builtin_inff(),
+                      -__builtin_inff(), -__builtin_inff(), -__builtin_inff()};
+        for (int b = tid; b < nblocks; b += 64)
+            for (int k = 0; k < 6; ++k)
+                v[k] = k < 3 ? fminf(v[k], blockBounds[6 * b + k]) : fmaxf(v[k], blockBounds[6 * b + k]);
+        for (int off = 32; off > 0; off >>= 1)
+            for (int k = 0; k < 6; ++k)
+                v[k] = k < 3 ? fminf(v[k], __shfl_xor(v[k], off)) : fmaxf(v[k], __shfl_xor(v[k], off));
+        if (tid == 0) {
+            for (int k = 0; k < 6; ++k)
+                s_bounds[k] = v[k];
+            *zero = 0u;
+        }
+    }
+    __syncthreads();
+    for (uint32_t i = tid; i < n; i += 64 * kOneSortWaves) {
+        s_key[0][i] = morton30(box_centre(box32, i), s_bounds) >> (30 - keyBits);
+        s_val[0][i] = (uint16_t)i;
+    }
+    __syncthreads();
+    int from = 0;
+    for (int shift = 0; shift < keyBits; shift += 8, from ^= 1)
+        one_sort_pass(
+            n, s_cnt, s_scan, [&](uint32_t i) { return s_key[from][i] >> shift & 255u; },
+            [&](uint32_t i, uint32_t slot) {
+                s_key[from ^ 1][slot] = s_key[from][i];
+                s_val[from ^ 1][slot] = s_val[from][i];
+            });
+    for (uint32_t i = tid; i < n; i += 64 * kOneSortWaves) {
+        keys[i] = s_key[from][i];
+        vals[i] = s_val[from][i];
+    }
+}
+
+bool small_order(size_t n) { return n <= kOneSortMax; }
+
+void launch_small_order(const float *box32, const float *blockBounds, int nblocks, uint32_t n, uint32_t *keys,
+                        uint32_t *vals, uint32_t *zero, hipStream_t s)
+{
+    if (n)
+        hipLaunchKernelGGL(k_small_order, dim3(1), dim3(64 * kOneSortWaves), 0, s, box32, blockBounds, nblocks, n,
+                           kMortonBits, keys, vals, zero);
+}
+
+// A short candidate list in place, by the first triangle (passes over bits
+// [32, 32 + firstBits)) and then each run of equal first triangles by the
+// second, as k_sort_runs does.
+__global__ __launch_bounds__(64 * kOneSortWaves) void k_small_pairs(uint64_t *keys, uint32_t n,
+                                                                    const uint32_t *__restrict__ count, int firstBits,
+                                                                    uint32_t maxRun, uint32_t *flag)
+{
+    __shared__ uint64_t s_key[2][kOneSortMax];
+    __shared__ uint32_t s_cnt[kOneSortWaves][256], s_scan[256];
+    n = (uint32_t)sort_len(n, count);
+    const uint32_t tid = threadIdx.x;
+    for (uint32_t i = tid; i < n; i += 64 * kOneSortWaves)
+        s_key[0][i] = keys[i];
+    __syncthreads();
+    int from = 0;
+    for (int shift = 32; shift < 32 + firstBits; shift += 8, from ^= 1)
+        one_sort_pass(
+            n, s_cnt, s_scan, [&](uint32_t i) { return (uint32_t)(s_key[from][i] >> shift) & 255u; },
+            [&](uint32_t i, uint32_t slot) { s_key[from ^ 1][slot] = s_key[from][i]; });
+    uint64_t *k = s_key[from];
+    for (uint32_t i = tid; i < n; i += 64 * kOneSortWaves) {
+        const uint32_t hi = (uint32_t)(k[i] >> 32);
+        if (i > 0 && (uint32_t)(k[i - 1] >> 32) == hi)
+            continue;
+        uint32_t j = i + 1;
+        while (j < n && j - i <= maxRun && (uint32_t)(k[j] >> 32) == hi)
+            ++j;  // to one past the longest run sorted here
+        if (j - i > maxRun) {
+            atomicOr(flag, 1u);
+            continue;
+        }
+        for (uint32_t x = i + 1; x < j; ++x) {
+            const uint64_t v = k[x];
+            uint32_t y = x;
+            for (; y > i && k[y - 1] > v; --y)
+                k[y] = k[y - 1];
+            k[y] = v;
+        }
+    }
+    __syncthreads();
+    for (uint32_t i = tid; i < n; i += 64 * kOneSortWaves)
+        keys[i] = k[i];
+}
+
+void launch_small_pairs(uint64_t *keys, size_t n, const uint32_t *count, int firstBits, uint32_t maxRun,
+                        uint32_t *flag, hipStream_t s)
+{
+    if (n)
+        hipLaunchKernelGGL(k_small_pairs, dim3(1), dim3(64 * kOneSortWaves), 0, s, keys, (uint32_t)n, count, firstBits,
+                           maxRun, flag);
+}
+
+bool small_pairs(size_t n) { return n <= kOneSortMax; }
+
 void launch_exclusive_scan(uint32_t *data, size_t m, hipStream_t s)
 {
     if (m == 0)
@@ -332,7 +545,10 @@ static void one_pass(const K *kin, const uint32_t *vin, K *kout, uint32_t *vout,
         hipLaunchKernelGGL((k_hist<K, 8>), dim3(nb), dim3(kSortBlock), 0, s, kin, n, count, shift, mask, hist, nb);
     else
         hipLaunchKernelGGL((k_hist<K, 4>), dim3(nb), dim3(kSortBlock), 0, s, kin, n, count, shift, mask, hist, nb);
-    hipLaunchKernelGGL(k_scan_rows, dim3(256), dim3(256), 0, s, hist, nb, rowTotal);
+    if (nb <= kScanInScatter)
+        rowTotal = nullptr;
+    else
+        hipLaunchKernelGGL(k_scan_rows, dim3(256), dim3(256), 0, s, hist, nb, rowTotal);
     if (items == 16)
         hipLaunchKernelGGL((k_scatter<K, HAS_VAL, 16>), dim3(nb), dim3(kSortBlock), 0, s, kin, vin, kout, vout, n,
                            count, shift, mask, hist, nb, rowTotal);

@@ -759,16 +759,21 @@ int sbg_mesh_prepare(sbg_mesh m)
         m->prepared = true;
         return SBG_OK;
     }
+    const bool small = small_order(nt);
     {
         Stage st(c, SBG_STAGE_RECORDS, s);
         launch_records(m->V.p, m->T.p, (uint32_t)nt, m->tri64.p, m->tri32.p, m->box32.p,
                        m->blockBounds.p, nb, s);
-        launch_bounds_reduce(m->blockBounds.p, nb, m->bounds.p, s);
-        launch_morton(m->box32.p, m->bounds.p, (uint32_t)nt, m->keys.p, m->vals.p, m->treeWork.p, s);
+        if (small) {
+            launch_small_order(m->box32.p, m->blockBounds.p, nb, (uint32_t)nt, m->keys.p, m->vals.p, m->treeWork.p, s);
+        } else {
+            launch_bounds_reduce(m->blockBounds.p, nb, m->bounds.p, s);
+            launch_morton(m->box32.p, m->bounds.p, (uint32_t)nt, m->keys.p, m->vals.p, m->treeWork.p, s);
+        }
         TRY(check_launch("records"));
     }
     uint32_t *sk = m->keys.p, *sv = m->vals.p;
-    {
+    if (!small) {
         Stage st(c, SBG_STAGE_SORT, s);
         if (radix_sort_u32(m->keys.p, m->vals.p, m->keysAlt.p, m->valsAlt.p, nt, 0, kMortonBits, m->hist.p, s)) {
             sk = m->keysAlt.p;
@@ -1080,8 +1085,13 @@ int sbg_find_pairs(sbg_mesh a, sbg_mesh b, sbg_pairs *out)
                 // too long for that raises a flag read with the count, and
                 // the list is then sorted the long way
                 const int ranges[2] = {32, 32 + ceil_log2(na)};
-                preInAlt = radix_sort_u64(p->pairs.p, p->alt.p, ns, ranges, 1, c->hist.p, c->stream, candCount) != 0;
-                launch_sort_runs(preInAlt ? p->alt.p : p->pairs.p, ns, candCount, kSortRunMax, runFlag, c->stream);
+                if (small_pairs(ns)) {
+                    launch_small_pairs(p->pairs.p, ns, candCount, ceil_log2(na), kSortRunMax, runFlag, c->stream);
+                } else {
+                    preInAlt =
+                        radix_sort_u64(p->pairs.p, p->alt.p, ns, ranges, 1, c->hist.p, c->stream, candCount) != 0;
+                    launch_sort_runs(preInAlt ? p->alt.p : p->pairs.p, ns, candCount, kSortRunMax, runFlag, c->stream);
+                }
                 preSorted = ns;
                 rc = check_launch("pair sort");
             }

@@ -67,6 +67,17 @@ void launch_sort_runs(uint64_t *keys, size_t n, const uint32_t *count, uint32_t 
 int radix_sort_u64(uint64_t *keys, uint64_t *keysAlt, size_t n, const int *bitRanges, int nRanges,
                    uint32_t *hist, hipStream_t s, const uint32_t *count = nullptr);
 
+// Short lists in one workgroup: the tree order of a small mesh straight from the
+// records kernel's block bounds (in place of launch_bounds_reduce,
+// launch_morton and the radix sort), and a short candidate list (in place of
+// the radix passes over the first triangle and launch_sort_runs), in place
+bool small_order(size_t n);
+void launch_small_order(const float *box32, const float *blockBounds, int nblocks, uint32_t n, uint32_t *keys,
+                        uint32_t *vals, uint32_t *zero, hipStream_t s);
+bool small_pairs(size_t n);
+void launch_small_pairs(uint64_t *keys, size_t n, const uint32_t *count, int firstBits, uint32_t maxRun,
+                        uint32_t *flag, hipStream_t s);
+
 // k_lbvh.hip
 // The tree over sorted codes: work holds n + 1 u32 (the first zero on entry:
 // launch_morton clears it, launch_tree64 clears it itself), scratch

@@ -141,10 +141,12 @@ def test_bvh_exact_across_refit_tiles(gpu, level):
     check_bvh(mesh, boxes64)
 
 
-@pytest.mark.parametrize("nt", [2, 3, 63, 65, 1023, 1024, 1025, 2047, 2048, 2049, 5000])
+@pytest.mark.parametrize("nt", [2, 3, 63, 65, 1023, 1024, 1025, 2047, 2048, 2049, 5000, 8191, 8192,
+                                8193])
 @pytest.mark.parametrize("spread", ["even", "clumps", "equal"])
 def test_bvh_tile_sizes(gpu, nt, spread):
-    """Triangle soups of sizes at the tree tiles' edges: evenly spread, in a
+    """Triangle soups of sizes at the edges of the tree tiles and of the
+    one-workgroup sort: evenly spread, in a
     few clumps of equal Morton codes (whose order and splits the triangle
     positions decide) and all the same; parents named by their children."""
     rng = np.random.default_rng(nt)
@@ -726,6 +728,30 @@ def test_hits_compaction(gpu, n, share):
         hp, hs = Q.hits()
         assert np.array_equal(hp, known[pick][hit]) and np.array_equal(bits(hs), bits(seg[hit]))
     assert len(P.hits()[0]) == int((status == 1).sum())
+
+
+@pytest.mark.parametrize("n", [40, 90, 127, 128, 129, 180])
+def test_pair_sort_sizes(gpu, n):
+    """Candidate lists from a few hundred to tens of thousands, the sizes
+    around the one-workgroup sort's, each searched three times so that the
+    sort is queued after a smaller, an equal and a larger list; runs of one
+    first triangle up to and past the 64 the quick sorts order."""
+    rng = np.random.default_rng(n)
+
+    def soup(k, size):
+        c = rng.random((k, 1, 3))
+        return mg.Mesh((c + size * rng.random((k, 3, 3))).reshape(-1, 3), np.arange(3 * k).reshape(-1, 3))
+
+    A, B = soup(n, 0.8), soup(n, 0.5)
+    small = soup(30, 0.3)
+    gA, gB, gS = (gpu.mesh(m.vertices, m.triangles) for m in (A, B, small))
+    bx, by = gA.boxes(), gB.boxes()
+    hit = np.all((bx[:, None, :3] <= by[None, :, 3:]) & (bx[:, None, 3:] >= by[None, :, :3]), axis=2)
+    want = np.argwhere(hit)
+    for _ in range(3):
+        assert np.array_equal(gA.find_pairs(gB).array().astype(np.int64), want)
+    gS.find_pairs(gS)
+    assert np.array_equal(gA.find_pairs(gB).array().astype(np.int64), want)
 
 
 def test_components_vs_oracle(gpu):
