@@ -513,9 +513,57 @@ void launch_hit_export(const uint64_t *hitPairs, const double *hitSeg, uint32_t 
                            (double2 *)seg);
 }
 
+// pairs with status 1 among n, into *count (zeroed first)
+__global__ __launch_bounds__(256) void k_count_hits(const uint8_t *__restrict__ status, uint32_t n, uint32_t *count)
+{
+    const uint32_t whole = n / 16, stride = gridDim.x * 256;
+    const uint4 *v = reinterpret_cast<const uint4 *>(status);
+    uint32_t c = 0;
+    for (uint32_t k = blockIdx.x * 256 + threadIdx.x; k < whole; k += stride)
+        c += hits_of(v[k]);
+    if (blockIdx.x == 0 && threadIdx.x < n - 16 * whole)
+        c += status[16 * (size_t)whole + threadIdx.x] & 1u;
+    for (int off = 32; off > 0; off >>= 1)
+        c += __shfl_down(c, off);
+    if ((threadIdx.x & 63) == 0 && c)
+        atomicAdd(count, c);
+}
+
+void launch_count_hits(const uint8_t *status, uint32_t n, uint32_t *count, hipStream_t s)
+{
+    launch_fill_u32(count, 0u, 1, s);
+    const unsigned blocks = (n / 16 + 255) / 256;
+    hipLaunchKernelGGL(k_count_hits, dim3(blocks < 1 ? 1 : (blocks > 256 ? 256 : blocks)), dim3(256), 0, s, status, n,
+                       count);
+}
+
+// a candidate list as it is handed out: ab (may be null) its pairs as (a, b)
+// couples, seg (may be null) zeroed where the pair does not intersect
+__global__ __launch_bounds__(256) void k_export_candidates(const uint64_t *__restrict__ pairs,
+                                                           const uint8_t *__restrict__ status, uint32_t n, uint2 *ab,
+                                                           double2 *seg)
+{
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= n)
+        return;
+    if (ab) {
+        const uint64_t p = pairs[i];
+        ab[i] = make_uint2((uint32_t)(p >> 32), (uint32_t)p);
+    }
+    if (seg && status[i] != 1)
+        seg[3 * (size_t)i] = seg[3 * (size_t)i + 1] = seg[3 * (size_t)i + 2] = make_double2(0.0, 0.0);
+}
+
+void launch_export_candidates(const uint64_t *pairs, const uint8_t *status, uint32_t n, uint32_t *ab, double *seg,
+                              hipStream_t s)
+{
+    if (n)
+        hipLaunchKernelGGL(k_export_candidates, dim3((n + 255) / 256), dim3(256), 0, s, pairs, status, n, (uint2 *)ab,
+                           (double2 *)seg);
+}
+
 int compact_blocks(uint32_t n) { return (int)((n + kCompactBlock - 1) / kCompactBlock); }
 
-void launch_fill_u32(uint32_t *p, uint32_t value, size_t n, hipStream_t s);
 
 // up to this many pairs the filtered precision runs as one fused launch
 constexpr uint32_t kFusedMaxPairs = 1u << 18;

@@ -7,8 +7,6 @@
 #include <cstring>
 #include <mutex>
 #include <string>
-#include <thread>
-#include <type_traits>
 #include <vector>
 
 #include "sbg_host.h"
@@ -347,6 +345,7 @@ void context_free(sbg_context ctx)
     ctx->pts.release();
     ctx->flags.release();
     ctx->bits.release();
+    ctx->axes.release();
     ctx->votes.release();
     ctx->ovf.release();
     ctx->rayList.release();
@@ -393,16 +392,7 @@ void context_free(sbg_context ctx)
         delete m;
     }
     ctx->spareMeshes.clear();
-    for (hipStream_t u : ctx->upload)
-        if (u) {
-            (void)hipStreamSynchronize(u);
-            (void)hipStreamDestroy(u);
-        }
-    for (auto &slots : ctx->stageDone)
-        for (hipEvent_t e : slots)
-            if (e)
-                (void)hipEventDestroy(e);
-    ctx->staging.release();
+    copy_free(ctx);
     (void)hipHostFree(ctx->pinned);
     (void)hipEventDestroy(ctx->auxReady);
     (void)hipStreamDestroy(ctx->grids);
@@ -413,114 +403,6 @@ void context_free(sbg_context ctx)
 }  // namespace sbg
 
 namespace sbg {
-
-// The upload streams, the staging slots' events and the page-locked staging,
-// made on the context's first mesh upload.
-static int upload_staging(sbg_context c)
-{
-    for (hipStream_t &u : c->upload)
-        if (!u && hipStreamCreateWithFlags(&u, hipStreamNonBlocking) != hipSuccess) {
-            u = nullptr;
-            return fail(SBG_ERR_HIP, "upload stream creation failed");
-        }
-    for (auto &slots : c->stageDone)
-        for (hipEvent_t &e : slots)
-            if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
-                e = nullptr;
-                return fail(SBG_ERR_HIP, "upload event creation failed");
-            }
-    return c->staging.ensure(2 * kUploadThreads * kStageSlot);
-}
-
-// One upload thread's share, src[first, last) into dst[first, last): the
-// thread converts a slot's worth of elements into one of its two staging
-// slots while the DMA of the other runs on its upload stream, and keeps the
-// largest element of an integer source (the triangles' vertex indices).
-template <typename S, typename D>
-static void upload_share(sbg_context c, int t, D *dst, const S *src, size_t first, size_t last, int *status,
-                         uint64_t *top)
-{
-    *status = SBG_OK;
-    *top = 0;
-    if (hipSetDevice(c->device) != hipSuccess) {
-        *status = SBG_ERR_HIP;
-        return;
-    }
-    const size_t per = kStageSlot / sizeof(D);
-    S hi = 0;
-    int k = 0;
-    for (size_t i = first; i < last; i += per, k ^= 1) {
-        const size_t n = std::min(per, last - i);
-        D *slot = (D *)(c->staging.p + (size_t)(2 * t + k) * kStageSlot);
-        if (hipEventSynchronize(c->stageDone[t][k]) != hipSuccess) {  // its last DMA is done
-            *status = SBG_ERR_HIP;
-            return;
-        }
-        if constexpr (std::is_integral<S>::value) {
-            for (size_t j = 0; j < n; ++j) {
-                const S v = src[i + j];
-                slot[j] = (D)v;
-                hi = v > hi ? v : hi;
-            }
-        } else {
-            std::memcpy(slot, src + i, n * sizeof(D));
-        }
-        const hipStream_t u = c->upload[t % kUploadStreams];
-        if (hipMemcpyAsync(dst + i, slot, n * sizeof(D), hipMemcpyHostToDevice, u) != hipSuccess ||
-            hipEventRecord(c->stageDone[t][k], u) != hipSuccess) {
-            *status = SBG_ERR_HIP;
-            return;
-        }
-    }
-    *top = (uint64_t)hi;
-}
-
-// The mesh's two host-to-device copies, vertices and triangles (narrowed from
-// 64-bit indices when S is), through the page-locked staging: up to
-// kUploadThreads host threads (one per kUploadShare bytes), each taking one
-// contiguous share of both arrays, the calling thread the first.  Returns
-// when every copy has landed, with the largest vertex index in *top.
-template <typename S>
-static int upload_mesh(sbg_context c, sbg_mesh m, const double *xyz, const S *tris, uint64_t *top)
-{
-    *top = 0;
-    const size_t nx = 3 * m->nv, ni = 3 * m->nt;
-    if (nx + ni == 0)
-        return SBG_OK;
-    TRY(upload_staging(c));
-    const size_t bytes = sizeof(double) * nx + sizeof(uint32_t) * ni;
-    const int shares = (int)std::max<size_t>(1, std::min<size_t>(kUploadThreads, bytes / kUploadShare));
-    int status[kUploadThreads][2];
-    uint64_t tops[kUploadThreads][2];
-    auto share = [&](int t) {
-        const size_t sx = (nx + shares - 1) / shares, si = (ni + shares - 1) / shares;
-        const size_t x0 = std::min(nx, t * sx), i0 = std::min(ni, t * si);
-        upload_share<double, double>(c, t, m->V.p, xyz, x0, std::min(nx, x0 + sx), &status[t][0], &tops[t][0]);
-        upload_share<S, uint32_t>(c, t, m->T.p, tris, i0, std::min(ni, i0 + si), &status[t][1], &tops[t][1]);
-    };
-    std::vector<std::thread> pool;
-    for (int t = 1; t < shares; ++t) {
-        try {
-            pool.emplace_back(share, t);
-        } catch (...) {  // no thread to be had: this share on the calling thread
-            share(t);
-        }
-    }
-    share(0);
-    for (std::thread &th : pool)
-        th.join();
-    hipError_t e = hipSuccess;
-    for (hipStream_t u : c->upload) {
-        const hipError_t eu = hipStreamSynchronize(u);
-        e = e != hipSuccess ? e : eu;
-    }
-    for (int t = 0; t < shares; ++t) {
-        if (status[t][0] != SBG_OK || status[t][1] != SBG_OK || e != hipSuccess)
-            return fail(SBG_ERR_HIP, "mesh upload failed: %s", hipGetErrorString(e != hipSuccess ? e : hipGetLastError()));
-        *top = std::max(*top, tops[t][1]);
-    }
-    return SBG_OK;
-}
 
 // sbg_mesh_create and sbg_mesh_create64: the indices are checked against
 // nverts (and against 32 bits, which the device stores) after the upload,
@@ -546,7 +428,7 @@ static int mesh_create(sbg_context ctx, const double *xyz, size_t nverts, const 
         r = m->T.ensure(3 * ntris);
     uint64_t top = 0;
     if (r == SBG_OK)
-        r = upload_mesh(ctx, m, xyz, tris, &top);
+        r = upload_mesh(ctx, m->V.p, m->T.p, xyz, 3 * nverts, tris, 3 * ntris, &top);
     if (r == SBG_OK && ntris && (top >= nverts || top > 0xffffffffull)) {
         // the first offending index for the message
         r = fail(SBG_ERR_INVALID, "vertex index %llu beyond 32 bits", (unsigned long long)top);
@@ -826,8 +708,7 @@ int sbg_mesh_normals(sbg_mesh m, double *out)
         TRY(c->pts.ensure(3 * m->nt));
         launch_normals64(m->tri64.p, (uint32_t)m->nt, c->pts.p, c->stream);
         TRY(check_launch("normals64"));
-        HIP_TRY(hipMemcpyAsync(out, c->pts.p, sizeof(double) * 3 * m->nt, hipMemcpyDeviceToHost, c->stream));
-        HIP_TRY(hipStreamSynchronize(c->stream));
+        TRY(copy_out(c, {{c->pts.p, out, sizeof(double) * 3 * m->nt}}));
     }
     return SBG_OK;
 }
@@ -846,9 +727,7 @@ int sbg_mesh_boxes(sbg_mesh m, double *out)
     TRY(c->pts.ensure(6 * m->nt));
     launch_boxes64(m->tri64.p, (uint32_t)m->nt, c->pts.p, c->stream);
     TRY(check_launch("boxes64"));
-    HIP_TRY(hipMemcpyAsync(out, c->pts.p, sizeof(double) * 6 * m->nt, hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    return SBG_OK;
+    return copy_out(c, {{c->pts.p, out, sizeof(double) * 6 * m->nt}});
 }
 
 int sbg_components(sbg_mesh m, const uint8_t *blocked, uint32_t *labels)
@@ -872,15 +751,14 @@ int sbg_components(sbg_mesh m, const uint8_t *blocked, uint32_t *labels)
     TRY(c->ccLabels.ensure(nt));
     if (blocked) {
         TRY(c->ccBlocked.ensure(nt));
-        HIP_TRY(hipMemcpyAsync(c->ccBlocked.p, blocked, nt, hipMemcpyHostToDevice, c->stream));
+        TRY(copy_in(c, {part_in(c->ccBlocked.p, blocked, nt)}));
     }
     launch_components(m->T.p, (uint32_t)nt, m->nv, blocked ? c->ccBlocked.p : nullptr, c->ccList.p, c->ccListAlt.p,
                       c->hist.p, c->ccValence.p, c->ccMate.p, c->ccParent.p, c->ccLabels.p, c->stream);
     TRY(check_launch("components"));
     uint32_t *repeated = c->pinned + kComponentsPinned;
     HIP_TRY(hipMemcpyAsync(repeated, c->ccValence.p + m->nv + 1, sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipMemcpyAsync(labels, c->ccLabels.p, sizeof(uint32_t) * nt, hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
+    TRY(copy_out(c, {{c->ccLabels.p, labels, sizeof(uint32_t) * nt}}));
     if (*repeated)
         return fail(SBG_ERR_INVALID, "repeated half-edge: two unblocked triangles share a directed edge");
     return SBG_OK;
@@ -905,23 +783,14 @@ int sbg_half_edges(sbg_context c, const uint32_t *tris, size_t ntris, const uint
     TRY(c->heQueries.ensure(nqueries));
     TRY(c->heQueryOwner.ensure(nqueries));
     TRY(c->heRepeat.ensure(1));
-    if (ntris)
-        HIP_TRY(hipMemcpyAsync(c->heTris.p, tris, sizeof(uint32_t) * 3 * ntris, hipMemcpyHostToDevice, c->stream));
-    if (nqueries)
-        HIP_TRY(hipMemcpyAsync(c->heQueries.p, queries, sizeof(uint64_t) * nqueries, hipMemcpyHostToDevice,
-                               c->stream));
+    TRY(copy_in(c, {part_in(c->heTris.p, tris, sizeof(uint32_t) * 3 * ntris),
+                    part_in(c->heQueries.p, queries, sizeof(uint64_t) * nqueries)}));
     launch_half_edges(c->heTris.p, (uint32_t)ntris, c->heQueries.p, (uint32_t)nqueries, c->ccKeys.p, c->ccOwners.p,
                       c->heOpposite.p, c->heQueryOwner.p, c->heRepeat.p, c->stream);
     TRY(check_launch("half edges"));
-    if (ntris)
-        HIP_TRY(hipMemcpyAsync(opposite, c->heOpposite.p, sizeof(uint32_t) * 3 * ntris, hipMemcpyDeviceToHost,
-                               c->stream));
-    if (nqueries)
-        HIP_TRY(hipMemcpyAsync(query_owner, c->heQueryOwner.p, sizeof(uint32_t) * nqueries, hipMemcpyDeviceToHost,
-                               c->stream));
-    HIP_TRY(hipMemcpyAsync(first_repeat, c->heRepeat.p, sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    return SBG_OK;
+    return copy_out(c, {{c->heOpposite.p, opposite, sizeof(uint32_t) * 3 * ntris},
+                        {c->heQueryOwner.p, query_owner, sizeof(uint32_t) * nqueries},
+                        {c->heRepeat.p, first_repeat, sizeof(uint32_t)}});
 }
 
 int sbg_mesh_bvh(sbg_mesh m, void *nodes_out, uint32_t *root_ref, float *root_box6)
@@ -1326,12 +1195,8 @@ int sbg_pairs_results(sbg_pairs p, uint8_t *status, double *seg)
     TRY(use(p->ctx));
     if (!p->n)
         return SBG_OK;
-    if (status)
-        HIP_TRY(hipMemcpyAsync(status, p->status.p, p->n, hipMemcpyDeviceToHost, p->ctx->stream));
-    if (seg)
-        HIP_TRY(hipMemcpyAsync(seg, p->seg.p, sizeof(double) * 6 * p->n, hipMemcpyDeviceToHost, p->ctx->stream));
-    HIP_TRY(hipStreamSynchronize(p->ctx->stream));
-    return SBG_OK;
+    return copy_out(p->ctx, {{p->status.p, status, status ? p->n : 0},
+                             {p->seg.p, seg, seg ? sizeof(double) * 6 * p->n : 0}});
 }
 
 int sbg_pairs_hits(sbg_pairs p, size_t *nhits, uint32_t *ab, double *seg)
@@ -1375,8 +1240,7 @@ int sbg_pairs_hits(sbg_pairs p, size_t *nhits, uint32_t *ab, double *seg)
         }
     }
     if (seg) {
-        HIP_TRY(hipMemcpyAsync(seg, p->hitSeg.p, segBytes, hipMemcpyDeviceToHost, c->stream));
-        HIP_TRY(hipStreamSynchronize(c->stream));
+        TRY(copy_out(c, {{p->hitSeg.p, seg, segBytes}}));
     }
     return SBG_OK;
 }
@@ -1394,14 +1258,10 @@ int sbg_tri_tri_batch(sbg_context ctx, const double *a9, const double *b9, size_
     TRY(ctx->rawB.ensure(9 * n));
     TRY(ctx->rawSeg.ensure(6 * n));
     TRY(ctx->rawStatus.ensure(n));
-    HIP_TRY(hipMemcpyAsync(ctx->rawA.p, a9, sizeof(double) * 9 * n, hipMemcpyHostToDevice, ctx->stream));
-    HIP_TRY(hipMemcpyAsync(ctx->rawB.p, b9, sizeof(double) * 9 * n, hipMemcpyHostToDevice, ctx->stream));
+    TRY(copy_in(ctx, {part_in(ctx->rawA.p, a9, sizeof(double) * 9 * n), part_in(ctx->rawB.p, b9, sizeof(double) * 9 * n)}));
     launch_tritri_raw(ctx->rawA.p, ctx->rawB.p, (uint32_t)n, ctx->rawStatus.p, ctx->rawSeg.p, ctx->stream);
     TRY(check_launch("tri_tri_raw"));
-    HIP_TRY(hipMemcpyAsync(status, ctx->rawStatus.p, n, hipMemcpyDeviceToHost, ctx->stream));
-    HIP_TRY(hipMemcpyAsync(seg, ctx->rawSeg.p, sizeof(double) * 6 * n, hipMemcpyDeviceToHost, ctx->stream));
-    HIP_TRY(hipStreamSynchronize(ctx->stream));
-    return SBG_OK;
+    return copy_out(ctx, {{ctx->rawStatus.p, status, n}, {ctx->rawSeg.p, seg, sizeof(double) * 6 * n}});
 }
 
 // ---------------------------------------------------------------------------
@@ -1495,21 +1355,6 @@ static RayBufs ray_bufs(sbg_context c, int set)
         return {c->pts2, c->flags2, c->bits2, c->votes2, c->ovf2, c->rayList2, c->pinned + kRayPinned + 4,
                 c->votesHost2};
     return {c->pts, c->flags, c->bits, c->votes, c->ovf, c->rayList, c->pinned + kRayPinned, c->votesHost};
-}
-
-// Page-locked host memory (hipHostMalloc, sbg_host_alloc, or registered by the
-// caller): a device-to-host copy into it is plain DMA.  *device says whether
-// kernels reach it at the same address.
-static bool page_locked(const void *p, bool *device)
-{
-    hipPointerAttribute_t at;
-    *device = false;
-    if (hipPointerGetAttributes(&at, p) != hipSuccess) {
-        (void)hipGetLastError();  // pageable memory is not an error here
-        return false;
-    }
-    *device = at.type == hipMemoryTypeHost && at.devicePointer == p;
-    return at.type == hipMemoryTypeHost;
 }
 
 // One side of a classification: the rays of n queries into target's grid, the
@@ -1657,20 +1502,15 @@ int sbg_classify_points(sbg_mesh target, const double *pts, size_t n, uint8_t *a
     TRY(c->pts.ensure(3 * n));
     TRY(c->bits.ensure(3 * n + 4));
     TRY(c->votes.ensure(n));
-    HIP_TRY(hipMemcpyAsync(c->pts.p, pts, sizeof(double) * 3 * n, hipMemcpyHostToDevice, c->stream));
+    TRY(copy_in(c, {part_in(c->pts.p, pts, sizeof(double) * 3 * n)}));
     RayJob job = {target, ray_bufs(c, 0), c->pts.p, nullptr, nullptr, n, inside, RayJob::kNone};
     TRY(run_rays(&job, 1, false, axis_inside != nullptr, false));
-    std::vector<uint8_t> bits;
-    if (axis_inside) {
-        bits.resize(3 * n);
-        HIP_TRY(hipMemcpyAsync(bits.data(), c->bits.p, 3 * n, hipMemcpyDeviceToHost, c->stream));
-    }
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    if (axis_inside)
-        for (size_t i = 0; i < n; ++i)
-            for (int k = 0; k < 3; ++k)
-                axis_inside[3 * i + k] = bits[(size_t)k * n + i];
-    return SBG_OK;
+    if (!axis_inside)
+        return SBG_OK;
+    TRY(c->axes.ensure(3 * n));
+    launch_interleave_axes(c->bits.p, (uint32_t)n, c->axes.p, c->stream);
+    TRY(check_launch("axes"));
+    return copy_out(c, {{c->axes.p, axis_inside, 3 * n}});
 }
 
 static int check_classify_args(sbg_mesh self, sbg_mesh other, sbg_pairs p, int side)
@@ -1907,15 +1747,11 @@ int sbg_adjoint(sbg_context ctx, const double *xyz_in, size_t nin, const uint32_
     TRY(ctx->adjSrc.ensure(5 * nd + 5));
     TRY(ctx->adjFaces.ensure(3 * nf + 3));
     hipStream_t s = ctx->stream;
-    if (nin)
-        HIP_TRY(hipMemcpyAsync(ctx->adjXyz.p, xyz_in, sizeof(double) * 3 * nin, hipMemcpyHostToDevice, s));
-    if (nd)
-        HIP_TRY(hipMemcpyAsync(ctx->adjSrc.p, src, sizeof(uint32_t) * 5 * nd, hipMemcpyHostToDevice, s));
-    if (nf)
-        HIP_TRY(hipMemcpyAsync(ctx->adjFaces.p, faces, sizeof(uint32_t) * 3 * nf, hipMemcpyHostToDevice, s));
     const bool wantGrad = grad_in != nullptr;
-    if (wantGrad && grad_derived && nd)
-        HIP_TRY(hipMemcpyAsync(ctx->adjGradD.p, grad_derived, sizeof(double) * 3 * nd, hipMemcpyHostToDevice, s));
+    TRY(copy_in(ctx, {part_in(ctx->adjXyz.p, xyz_in, sizeof(double) * 3 * nin),
+                      part_in(ctx->adjSrc.p, src, sizeof(uint32_t) * 5 * nd),
+                      part_in(ctx->adjFaces.p, faces, sizeof(uint32_t) * 3 * nf),
+                      part_in(ctx->adjGradD.p, grad_derived, wantGrad && grad_derived ? sizeof(double) * 3 * nd : 0)}));
     launch_fill_u32(reinterpret_cast<uint32_t *>(ctx->adjVol.p), 0u, 2, s);
     if (wantGrad)
         launch_fill_u32(reinterpret_cast<uint32_t *>(ctx->adjGall.p), 0u, 6 * nall, s);
@@ -1923,15 +1759,9 @@ int sbg_adjoint(sbg_context ctx, const double *xyz_in, size_t nin, const uint32_
                    vol_weight, (wantGrad && grad_derived) ? ctx->adjGradD.p : nullptr, ctx->adjAll.p, ctx->adjVol.p,
                    wantGrad ? ctx->adjGall.p : nullptr, s);
     TRY(check_launch("adjoint"));
-    if (derived_xyz && nd)
-        HIP_TRY(hipMemcpyAsync(derived_xyz, ctx->adjAll.p + 3 * nin, sizeof(double) * 3 * nd, hipMemcpyDeviceToHost,
-                               s));
-    if (volume)
-        HIP_TRY(hipMemcpyAsync(volume, ctx->adjVol.p, sizeof(double), hipMemcpyDeviceToHost, s));
-    if (wantGrad && nin)
-        HIP_TRY(hipMemcpyAsync(grad_in, ctx->adjGall.p, sizeof(double) * 3 * nin, hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
-    return SBG_OK;
+    return copy_out(ctx, {{ctx->adjAll.p + 3 * nin, derived_xyz, derived_xyz ? sizeof(double) * 3 * nd : 0},
+                          {ctx->adjVol.p, volume, volume ? sizeof(double) : 0},
+                          {ctx->adjGall.p, grad_in, wantGrad ? sizeof(double) * 3 * nin : 0}});
 }
 
 int sbg_calibrate_copy(sbg_context ctx, size_t bytes, int iters, double *avg_ms)

@@ -59,6 +59,7 @@ struct sbg_batch_s {
     DevBuf<uint8_t> status;
     DevBuf<double> seg;
     DevBuf<uint32_t> gdWork;
+    DevBuf<uint32_t> hitCount, abOut;  // sbg_batch_counts, sbg_batch_candidates
     DevBuf<uint8_t> flags, bits, votes;
     DevBuf<double> pts;
     DevBuf<uint32_t> rayList;
@@ -316,7 +317,7 @@ int sbg_batch_create(sbg_context ctx, const double *xyz, const uint32_t *tris, c
         (rc = b->ids.ensure(nt)) || (rc = b->work.ensure(nt + 1)) ||
         (rc = b->treeScratch.ensure(tree_scratch_floats((uint32_t)nt))) ||
         (rc = b->meshRoot.ensure(nmeshes)) || (rc = b->nodes.ensure(nt > 1 ? nt - 1 : 1)) ||
-        (rc = b->words.ensure(kWords)) || (rc = b->flags.ensure(nt + 4)) || (rc = b->bits.ensure(3 * nt + 4)) ||
+        (rc = b->words.ensure(kWords)) || (rc = b->hitCount.ensure(1)) || (rc = b->flags.ensure(nt + 4)) || (rc = b->bits.ensure(3 * nt + 4)) ||
         (rc = b->votes.ensure(nt)) || (rc = b->pts.ensure(4 * nt)) || (rc = b->rayList.ensure(ray_list_u32(nt))))
         return bail(rc);
     if (hipHostMalloc((void **)&b->host, sizeof(uint32_t) * kWords, hipHostMallocDefault) != hipSuccess) {
@@ -345,7 +346,7 @@ int sbg_batch_set_vertices(sbg_batch b, const double *xyz)
     if (!b || (b->nv && !xyz))
         return fail(SBG_ERR_INVALID, "null argument");
     TRY(use(b->ctx));
-    HIP_TRY(hipMemcpyAsync(b->V.p, xyz, sizeof(double) * 3 * b->nv, hipMemcpyHostToDevice, b->ctx->stream));
+    TRY(copy_in(b->ctx, {part_in(b->V.p, xyz, sizeof(double) * 3 * b->nv)}));
     HIP_TRY(hipStreamSynchronize(b->ctx->stream));
     b->ran = false;
     return SBG_OK;
@@ -556,12 +557,12 @@ int sbg_batch_counts(sbg_batch b, size_t *candidates, size_t *hits)
     if (candidates)
         *candidates = b->nCand;
     if (hits) {
-        std::vector<uint8_t> st(b->nCand);
-        if (b->nCand)
-            HIP_TRY(hipMemcpy(st.data(), b->status.p, b->nCand, hipMemcpyDeviceToHost));
-        size_t h = 0;
-        for (uint8_t v : st)
-            h += v == 1;
+        uint32_t h = 0;
+        if (b->nCand) {
+            launch_count_hits(b->status.p, b->nCand, b->hitCount.p, b->ctx->stream);
+            TRY(check_launch("hit count"));
+            TRY(copy_out(b->ctx, {{b->hitCount.p, &h, sizeof(h)}}));
+        }
         *hits = h;
     }
     return SBG_OK;
@@ -577,26 +578,16 @@ int sbg_batch_candidates(sbg_batch b, uint32_t *ab, uint8_t *status, double *seg
     const size_t n = b->nCand;
     if (!n)
         return SBG_OK;
-    if (ab) {
-        std::vector<uint64_t> p(n);
-        HIP_TRY(hipMemcpy(p.data(), b->pairsInAlt ? b->pairsAlt.p : b->pairs.p, sizeof(uint64_t) * n,
-                          hipMemcpyDeviceToHost));
-        for (size_t i = 0; i < n; ++i) {
-            ab[2 * i] = (uint32_t)(p[i] >> 32);
-            ab[2 * i + 1] = (uint32_t)p[i];
-        }
-    }
-    if (status)
-        HIP_TRY(hipMemcpy(status, b->status.p, n, hipMemcpyDeviceToHost));
-    if (seg) {
-        std::vector<uint8_t> st(n);
-        HIP_TRY(hipMemcpy(st.data(), b->status.p, n, hipMemcpyDeviceToHost));
-        HIP_TRY(hipMemcpy(seg, b->seg.p, sizeof(double) * 6 * n, hipMemcpyDeviceToHost));
-        for (size_t i = 0; i < n; ++i)
-            if (st[i] != 1)
-                std::memset(seg + 6 * i, 0, sizeof(double) * 6);
-    }
-    return SBG_OK;
+    // pairs as (a, b) couples, and the segments of pairs that do not intersect
+    // zeroed, on the GPU
+    if (ab)
+        TRY(b->abOut.ensure(2 * n));
+    launch_export_candidates(b->pairsInAlt ? b->pairsAlt.p : b->pairs.p, b->status.p, (uint32_t)n,
+                             ab ? b->abOut.p : nullptr, seg ? b->seg.p : nullptr, b->ctx->stream);
+    TRY(check_launch("candidate export"));
+    return copy_out(b->ctx, {{b->abOut.p, ab, ab ? sizeof(uint32_t) * 2 * n : 0},
+                             {b->status.p, status, status ? n : 0},
+                             {b->seg.p, seg, seg ? sizeof(double) * 6 * n : 0}});
 }
 
 int sbg_batch_sides(sbg_batch b, uint8_t *side)
@@ -606,8 +597,7 @@ int sbg_batch_sides(sbg_batch b, uint8_t *side)
     if (!b->ran)
         return fail(SBG_ERR_STATE, "no completed run");
     TRY(use(b->ctx));
-    HIP_TRY(hipMemcpy(side, b->votes.p, b->nt, hipMemcpyDeviceToHost));
-    return SBG_OK;
+    return copy_out(b->ctx, {{b->votes.p, side, b->nt}});
 }
 
 int sbg_batch_autotune(sbg_batch b, int precision, int reps, sbg_batch_tuning *best, double *best_ms)
@@ -698,7 +688,7 @@ int sbg_batch_destroy(sbg_batch b)
         p->release();
     DevBuf<uint32_t> *u32[] = {&b->T,    &b->meshOf,     &b->target,   &b->triBegin, &b->ids,
                                &b->work, &b->meshRoot, &b->hist,     &b->words,
-                               &b->gdWork, &b->rayList, &b->gridCells, &b->gridTemp};
+                               &b->gdWork, &b->hitCount, &b->abOut, &b->rayList, &b->gridCells, &b->gridTemp};
     for (auto *p : u32)
         p->release();
     DevBuf<uint64_t> *u64[] = {&b->keys, &b->keysAlt, &b->codes, &b->pairs, &b->pairsAlt};

@@ -5,6 +5,7 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include <initializer_list>
 #include <vector>
 
 #include "sbg_internal.h"
@@ -108,14 +109,16 @@ constexpr uint32_t kSpillInit = 2048, kSpillMax = 1u << 15;
 // intersecting pairs and segments up to this size leave through page-locked
 // staging (74,898 of them)
 constexpr size_t kHitStage = (size_t)4 << 20;
-// sbg_mesh_create's uploads: host threads that fill page-locked staging (two
-// slots each), the slot size, and the smallest share worth a thread of its own
-constexpr int kUploadThreads = 8;
-constexpr size_t kStageSlot = (size_t)2 << 20;
-constexpr size_t kUploadShare = (size_t)2 << 20;
-// the threads' copies alternate between this many streams, so the DMA of
-// one waits for no other's
-constexpr int kUploadStreams = 2;
+// transfers of host arrays (sbg_copy.hip): host threads, the page-locked staging
+// (two halves), the piece a thread takes at a time, what is worth a thread, what
+// leaves the GPU between two waits, and the arrays of one call
+constexpr int kCopyThreads = 8;
+constexpr size_t kStageHalf = (size_t)16 << 20;
+constexpr size_t kCopyPiece = (size_t)1 << 20;
+constexpr size_t kCopyShare = (size_t)1 << 20;
+constexpr size_t kOutRound = (size_t)4 << 20;
+constexpr int kCopyParts = 4;
+struct CopyPool;
 
 }  // namespace sbg
 
@@ -128,11 +131,12 @@ struct sbg_context_s {
     hipEvent_t auxReady = nullptr;    // orders the aux stream after the main one
     hipStream_t grids = nullptr;      // third stream (default priority): ray grids built at prepare time
     uint32_t *pinned = nullptr;  // host-visible counters (kPinnedWords): search, then two ray sides
-    // mesh uploads: their own streams, page-locked staging of 2 x kUploadThreads
-    // slots and the event after each slot's last copy (made on first use)
-    hipStream_t upload[kUploadStreams] = {};
+    // transfers of host arrays (made on first use): page-locked staging, the
+    // event after each half's last copy, the threads, and mesh uploads' stream
+    hipStream_t uploads = nullptr;
     PinnedBuf staging;
-    hipEvent_t stageDone[kUploadThreads][2] = {};
+    hipEvent_t stageDone[2] = {};
+    CopyPool *copyPool = nullptr;
     DevBuf<uint2> front[2];
     DevBuf<uint2> spill;              // depth-first spill regions
     uint32_t spillPerWave = kSpillInit;
@@ -150,6 +154,7 @@ struct sbg_context_s {
     // single calls and other scratch uses take set 0)
     DevBuf<double> pts, pts2;
     DevBuf<uint8_t> flags, bits, votes, flags2, bits2, votes2;
+    DevBuf<uint8_t> axes;  // sbg_classify_points' per-axis answers
     DevBuf<uint32_t> ovf, rayList, ovf2, rayList2;
     PinnedBuf votesHost, votesHost2;  // vote readbacks of the two sets
     PinnedBuf hitStage;               // sbg_pairs_hits: kHitStage bytes
@@ -223,5 +228,27 @@ struct Stage {
 
 int check_launch(const char *what);
 int ceil_log2(size_t n);
+
+// sbg_copy.hip
+struct CopyPart {
+    enum Kind { kBytes, kIndices32, kIndices64 };  // uploads: 64-bit ones are narrowed
+    void *dev;                                     // on 8 bytes
+    void *host;
+    size_t bytes;  // on the GPU
+    Kind kind = kBytes;
+};
+inline CopyPart part_in(void *dev, const void *host, size_t bytes) { return {dev, const_cast<void *>(host), bytes}; }
+// up to kCopyParts arrays; parts of 0 bytes are skipped
+int copy_in(sbg_context c, std::initializer_list<CopyPart> parts);
+int copy_out(sbg_context c, std::initializer_list<CopyPart> parts);
+void copy_free(sbg_context c);
+// a mesh's vertices and (narrowed) triangle indices; the largest index in *top
+template <typename S>
+int upload_mesh(sbg_context c, double *dv, uint32_t *dt, const double *xyz, size_t nx, const S *tris, size_t ni,
+                uint64_t *top);
+// Page-locked host memory (hipHostMalloc, sbg_host_alloc, or registered by the
+// caller): a copy to or from it is plain DMA.  *device says
+// whether kernels reach it at the same address.
+bool page_locked(const void *p, bool *device);
 
 }  // namespace sbg

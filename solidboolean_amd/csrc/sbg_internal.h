@@ -167,6 +167,9 @@ void launch_compact_hits(const uint64_t *pairs, const uint8_t *status, const dou
 void launch_hit_export(const uint64_t *hitPairs, const double *hitSeg, uint32_t n, uint32_t *ab, double *seg,
                        hipStream_t s);
 int compact_blocks(uint32_t n);
+void launch_count_hits(const uint8_t *status, uint32_t n, uint32_t *count, hipStream_t s);
+void launch_export_candidates(const uint64_t *pairs, const uint8_t *status, uint32_t n, uint32_t *ab, double *seg,
+                              hipStream_t s);
 
 // k_classify.hip
 void launch_mark_intersected(const uint64_t *pairs, const uint8_t *status, uint32_t n, const uint32_t *count,

@@ -889,3 +889,31 @@ def test_pair_sort_runs(gpu, levels):
     for _ in range(3):
         P = A.find_pairs(B)
         assert np.array_equal(P.array().astype(np.int64), ref), (levels, int(runs.max()))
+
+
+@pytest.mark.parametrize("n", [1, 7, 333, 7281, 7282, 50001, 350003])
+def test_host_arrays_through_staging(gpu, n):
+    """Host arrays from a few bytes to several times the staging move in and
+    out whole: triangle pairs (9 doubles each, twice) whose answers repeat those
+    of a short list, points' per-axis answers, and a mesh whose triangles come
+    back as their boxes, with 32- and 64-bit indices."""
+    rng = np.random.default_rng(n)
+    a, b = rng.random((61, 9)), rng.random((61, 9))
+    st, seg = gpu.tri_tri_batch(a, b)
+    pick = rng.integers(0, 61, n)
+    st2, seg2 = gpu.tri_tri_batch(a[pick], b[pick])
+    assert np.array_equal(st2, st[pick]) and np.array_equal(bits(seg2), bits(seg[pick]))
+
+    cube = mg.small_pair(1)[0]
+    M = gpu.mesh(cube.vertices, cube.triangles)
+    pts = rng.random((61, 3)) * 2 - 1
+    axes, inside = M.classify_points(pts)
+    axes2, inside2 = M.classify_points(pts[pick])
+    assert np.array_equal(axes2, axes[pick]) and np.array_equal(inside2, inside[pick])
+
+    v = rng.random((3 * n, 3))
+    t = rng.permutation(3 * n).reshape(-1, 3)
+    corner = v[t]
+    box = np.concatenate([corner.min(axis=1), corner.max(axis=1)], axis=1)
+    for kind in (np.uint32, np.int64):
+        assert np.array_equal(bits(gpu.mesh(v, t.astype(kind)).boxes()), bits(box))
