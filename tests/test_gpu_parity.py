@@ -917,3 +917,24 @@ def test_host_arrays_through_staging(gpu, n):
     box = np.concatenate([corner.min(axis=1), corner.max(axis=1)], axis=1)
     for kind in (np.uint32, np.int64):
         assert np.array_equal(bits(gpu.mesh(v, t.astype(kind)).boxes()), bits(box))
+
+
+@pytest.mark.parametrize("nt", [1, 63, 64, 65, 255, 256, 257, 321])
+def test_records_around_a_wave(gpu, nt):
+    """Normals and boxes (from the FP64 records) and the tree's leaf boxes (from the
+    FP32 ones) of meshes around a wave's and a workgroup's size, whose last wave
+    stores a part of its staged run, with a vertex buffer freed and reused between."""
+    from oracle.oracle import prepare
+
+    rng = np.random.default_rng(nt)
+    for _ in range(2):
+        v = rng.standard_normal((40, 3))
+        t = rng.integers(0, 40, (nt, 3))
+        n, box = prepare(v, t)
+        with_tree = gpu.mesh(v, t)
+        assert np.array_equal(bits(with_tree.normals()), bits(n))
+        assert np.array_equal(bits(with_tree.boxes()), bits(box[:, :6]))
+        if nt > 1:
+            nodes, root, rbox = with_tree.bvh()
+            check_bvh_tight(nodes, root, rbox, box[:, :6])
+        with_tree.close()
