@@ -286,15 +286,19 @@ __global__ __launch_bounds__(kSortBlock) void k_scatter(const K *__restrict__ ke
     }
 }
 
-// A list of (first << 32 | second) keys already sorted by their high word:
-// each run of equal high words is sorted by the low word in place, one lane
-// per run (the lane at the run's first entry), by insertion.  A run longer
-// than maxRun is left as it is and raises *flag (the caller then sorts the
-// whole list by both words).  Runs of ~0 keys (padding) are skipped.  Lanes
-// only ever move entries within their own run, so the high word another lane
-// reads at a run's border never changes under it.
-__global__ __launch_bounds__(256) void k_sort_runs(uint64_t *keys, uint32_t n, const uint32_t *__restrict__ count,
-                                                   uint32_t maxRun, uint32_t *flag)
+// A list of (first << 32 | second) keys already sorted by their high word, each run
+// of equal high words put in order of the low word: every lane counts the keys of
+// its run that come before its own and stores its key at that place of out.  A run
+// longer than maxRun goes over as it is and raises *flag (the caller then sorts
+// the whole list by both words); so do ~0 keys (padding), without the flag.
+// out is a permutation of keys whatever the runs are.
+//
+// One lane per run, sorting in place, waited for each load in turn: 22 us for the
+// candidates of two 655 k-triangle spheres, 9 now, and it was slower than
+// radix passes for a batch's longer runs (38 us now).
+__global__ __launch_bounds__(256) void k_sort_runs(const uint64_t *__restrict__ keys, uint64_t *__restrict__ out,
+                                                   uint32_t n, const uint32_t *__restrict__ count, uint32_t maxRun,
+                                                   uint32_t *flag)
 {
     n = (uint32_t)sort_len(n, count);
     const uint32_t i = blockIdx.x * 256 + threadIdx.x;
@@ -302,30 +306,51 @@ __global__ __launch_bounds__(256) void k_sort_runs(uint64_t *keys, uint32_t n, c
         return;
     const uint64_t k = keys[i];
     const uint32_t hi = (uint32_t)(k >> 32);
-    if (k == ~0ull || (i > 0 && (uint32_t)(keys[i - 1] >> 32) == hi))
-        return;
-    uint32_t j = i + 1;
-    while (j < n && (uint32_t)(keys[j] >> 32) == hi) {
-        if (++j - i > maxRun) {
-            atomicOr(flag, 1u);
-            return;
+    uint32_t back = 0, len = 1, less = 0;
+    if (k != ~0ull) {
+        // four neighbours at a time, their loads in flight together
+        bool more = true;
+        while (more && back <= maxRun) {
+            uint64_t v[4];
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j)
+                v[j] = keys[i > back + j ? i - back - j - 1 : 0];
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j) {
+                more = more && i > back && (uint32_t)(v[j] >> 32) == hi;
+                back += more;
+                less += more && v[j] < k;
+            }
+        }
+        len += back;
+        more = true;
+        for (uint32_t x = i + 1; more && len <= maxRun; x += 4) {
+            uint64_t v[4];
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j)
+                v[j] = keys[x + j < n ? x + j : n - 1];
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j) {
+                more = more && x + j < n && (uint32_t)(v[j] >> 32) == hi;
+                len += more;
+                less += more && v[j] < k;
+            }
         }
     }
-    for (uint32_t x = i + 1; x < j; ++x) {
-        const uint64_t v = keys[x];
-        uint32_t y = x;
-        for (; y > i && keys[y - 1] > v; --y)
-            keys[y] = keys[y - 1];
-        keys[y] = v;
+    if (len > maxRun) {
+        atomicOr(flag, 1u);
+        out[i] = k;
+        return;
     }
+    out[i - back + less] = k;
 }
 
-void launch_sort_runs(uint64_t *keys, size_t n, const uint32_t *count, uint32_t maxRun, uint32_t *flag,
-                      hipStream_t s)
+void launch_sort_runs(const uint64_t *keys, uint64_t *out, size_t n, const uint32_t *count, uint32_t maxRun,
+                      uint32_t *flag, hipStream_t s)
 {
     if (n)
-        hipLaunchKernelGGL(k_sort_runs, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, keys, (uint32_t)n, count,
-                           maxRun, flag);
+        hipLaunchKernelGGL(k_sort_runs, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, keys, out, (uint32_t)n,
+                           count, maxRun, flag);
 }
 
 // ---- sorts of one workgroup ---------------------------------------------------

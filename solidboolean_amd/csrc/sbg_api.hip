@@ -957,9 +957,11 @@ int sbg_find_pairs(sbg_mesh a, sbg_mesh b, sbg_pairs *out)
                 if (small_pairs(ns)) {
                     launch_small_pairs(p->pairs.p, ns, candCount, ceil_log2(na), kSortRunMax, runFlag, c->stream);
                 } else {
-                    preInAlt =
+                    const bool inAlt =
                         radix_sort_u64(p->pairs.p, p->alt.p, ns, ranges, 1, c->hist.p, c->stream, candCount) != 0;
-                    launch_sort_runs(preInAlt ? p->alt.p : p->pairs.p, ns, candCount, kSortRunMax, runFlag, c->stream);
+                    launch_sort_runs(inAlt ? p->alt.p : p->pairs.p, inAlt ? p->pairs.p : p->alt.p, ns, candCount,
+                                     kSortRunMax, runFlag, c->stream);
+                    preInAlt = !inAlt;
                 }
                 preSorted = ns;
                 rc = check_launch("pair sort");

@@ -22,6 +22,7 @@ constexpr uint32_t kBatchSpillInit = 2048, kBatchSpillMax = 1u << 15;
 // 35 depth-first claims, [36, 40) ray counters (36 ray flags), 40 grid entries
 constexpr int kCandW = kBatchMaxLevels + 1, kFlagW = kBatchMaxLevels + 2, kHeadW = kBatchMaxLevels + 3;
 constexpr int kRayFlagW = kBatchMaxLevels + 4, kGridW = kBatchMaxLevels + 8;
+constexpr int kRunW = kBatchMaxLevels + 9;
 constexpr int kWords = kBatchMaxLevels + 10;
 // the batch's ray-grid build: one workgroup per tile of 512 triangles (the
 // batch's grids are millions of triangles, and the branch beside them is the
@@ -59,6 +60,7 @@ struct sbg_batch_s {
     DevBuf<uint8_t> status;
     DevBuf<double> seg;
     DevBuf<uint32_t> gdWork;
+    bool longRuns = false;  // a first triangle had more candidates than launch_sort_runs takes
     DevBuf<uint32_t> hitCount, abOut;  // sbg_batch_counts, sbg_batch_candidates
     DevBuf<uint8_t> flags, bits, votes;
     DevBuf<double> pts;
@@ -218,9 +220,22 @@ int enqueue(sbg_batch b, int precision)
                         b->tune.dfs_waves, b->pairs.p, candCount, ccap, flagsW, s);
     TRY(check_launch("batch search"));
     // canonical (a, b) order of the candidates (their count read on the device)
-    const int pairRanges[4] = {0, b->triBits, 32, 32 + b->triBits};
-    b->pairsInAlt =
-        radix_sort_u64(b->pairs.p, b->pairsAlt.p, b->candCap, pairRanges, 2, b->hist.p, s, candCount) != 0;
+    // by the first triangle, then each first triangle's run by the second, unless
+    // an earlier run of this batch met one too long for that.  For 739 k triangles
+    // and beside the grid build, both triangles by radix passes took 6 of them,
+    // 58 us each; three and the runs take 210 us together.
+    if (b->longRuns) {
+        const int both[4] = {0, b->triBits, 32, 32 + b->triBits};
+        b->pairsInAlt =
+            radix_sort_u64(b->pairs.p, b->pairsAlt.p, b->candCap, both, 2, b->hist.p, s, candCount) != 0;
+    } else {
+        const int first[2] = {32, 32 + b->triBits};
+        const bool inAlt =
+            radix_sort_u64(b->pairs.p, b->pairsAlt.p, b->candCap, first, 1, b->hist.p, s, candCount) != 0;
+        launch_sort_runs(inAlt ? b->pairsAlt.p : b->pairs.p, inAlt ? b->pairs.p : b->pairsAlt.p, b->candCap, candCount,
+                         kSortRunMax, w + kRunW, s);
+        b->pairsInAlt = !inAlt;
+    }
     const uint64_t *sorted = b->pairsInAlt ? b->pairsAlt.p : b->pairs.p;
     launch_tritri(b->tri64.p, b->tri64.p, b->tri32.p, b->tri32.p, sorted, ccap, candCount, precision, b->status.p,
                   b->seg.p, b->gdWork.p, nullptr, s);
@@ -445,6 +460,10 @@ int sbg_batch_run(sbg_batch b, int precision)
             if (b->spillPerWave >= kBatchSpillMax)
                 return fail(SBG_ERR_OVERFLOW, "depth-first search exceeded its largest spill regions");
             b->spillPerWave = std::min(kBatchSpillMax, std::max(kBatchSpillInit, 4 * b->spillPerWave));
+            grow = true;
+        }
+        if (h[kRunW] && !b->longRuns) {
+            b->longRuns = true;
             grow = true;
         }
         if (rflags & 2u) {

@@ -265,3 +265,41 @@ def test_batch4096_matches_oracle(batch4096):
         ib[ref[ost == 1, 1]] = 1
         assert np.array_equal(sides[tb[2 * k]:tb[2 * k + 1]], OA.classify_triangles(OB, ia)), k
         assert np.array_equal(sides[tb[2 * k + 1]:tb[2 * k + 2]], OB.classify_triangles(OA, ib)), k
+
+
+@pytest.mark.parametrize("nb", [60, 64, 65, 66, 300])
+def test_batch_long_candidate_runs(gpu, nb):
+    """A triangle whose box meets nb others, up to, at and past the run length
+    that is sorted in place after a sort by the first triangle; past it the batch
+    sorts by both, in that run and in later ones, captured or not."""
+    rng = np.random.default_rng(nb)
+    big = mg.Mesh(np.array([[0, 0, 0], [9, 0, 0.3], [0, 9, 0.5], [0.5, 0.5, 4]], float),
+                  np.array([[0, 2, 1], [0, 1, 3], [1, 2, 3], [2, 0, 3]]))
+    c = 0.5 + rng.random((nb, 1, 3)) * [4, 4, 0.1]
+    many = mg.Mesh((c + 0.2 * rng.random((nb, 3, 3))).reshape(-1, 3), np.arange(3 * nb).reshape(-1, 3))
+    pairs = mg.batch_pairs(3, seed=nb, levels=(2, 3)) + [(big, many)] + mg.batch_pairs(2, seed=1, levels=(1, 2))
+    for graph in (0, 1):
+        batch = gpu.batch(pairs)
+        batch.set_tuning(use_graph=graph)
+        for _ in range(3):
+            batch.run(N.FP64)
+            ab, st, seg = batch.candidates()
+            key = ab[:, 0].astype(np.uint64) << np.uint64(32) | ab[:, 1].astype(np.uint64)
+            assert np.all(np.diff(key.astype(np.int64)) > 0)
+        compare_lists(batch, pairs, gpu, ab, st, seg)
+        batch.close()
+
+
+def compare_lists(batch, pairs, gpu, ab, st, seg):
+    """The candidates, statuses and segments of every pair against the single-pair path."""
+    tb = batch.tri_begin.astype(np.int64)
+    for k, (a, b) in enumerate(pairs):
+        A, B = gpu.mesh(a.vertices, a.triangles), gpu.mesh(b.vertices, b.triangles)
+        P = A.find_pairs(B)
+        P.tri_tri(A, B, N.FP64, stats=False)
+        rst, rseg = P.results()
+        sel = (ab[:, 0] >= tb[2 * k]) & (ab[:, 0] < tb[2 * k + 1])
+        assert np.array_equal(ab[sel].astype(np.int64) - [tb[2 * k], tb[2 * k + 1]], P.array()), k
+        assert np.array_equal(st[sel], rst), k
+        h = rst == 1
+        assert np.array_equal(bits(seg[sel][h]), bits(rseg[h])), k
