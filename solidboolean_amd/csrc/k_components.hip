@@ -70,6 +70,17 @@ __device__ __forceinline__ uint32_t he_owner(const unsigned long long *__restric
     return ~0u;
 }
 
+// raises the repeated-half-edge flag; once it stands it is only read
+__device__ __forceinline__ bool repeat_known(const uint32_t *repeated)
+{
+    return __hip_atomic_load(repeated, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u;
+}
+__device__ __forceinline__ void raise_repeat(uint32_t *repeated)
+{
+    if (!repeat_known(repeated))
+        atomicOr(repeated, 1u);
+}
+
 __device__ __forceinline__ uint32_t cc_find(uint32_t *parent, uint32_t x)
 {
     uint32_t p = __hip_atomic_load(&parent[x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -258,7 +269,7 @@ __global__ __launch_bounds__(kCcTile) void k_cc_tiles(const uint32_t *__restrict
                 const uint32_t of = s_vert[e], oto = s_vert[3 * ot + (ok == 2 ? 0 : ok + 1)];
                 if (min(of, oto) == lo && max(of, oto) == hi) {
                     if (of == from || (cur & 1u) || atomicOr(&s_edge[s], 1u) & 1u)
-                        atomicOr(repeated, 1u);
+                        raise_repeat(repeated);
                     else
                         cc_unite(s_parent, threadIdx.x, ot);
                     break;
@@ -309,50 +320,113 @@ __global__ __launch_bounds__(kCcTile) void k_cc_tiles(const uint32_t *__restrict
 constexpr int kCcAhead = 512;  // entries past its own that a workgroup holds
 constexpr int kCcHeld = kCcTile + kCcAhead;
 
+// the half-edge's ends, from << 32 | to
+__device__ __forceinline__ uint64_t half_of(const uint32_t *__restrict__ T, uint32_t e)
+{
+    return (uint64_t)T[e] << 32 | T[e % 3u == 2u ? e - 2u : e + 1u];
+}
+
+// the halves a and b of one edge
+__device__ __forceinline__ void pair_halves(uint64_t a, uint32_t ea, uint64_t b, uint32_t eb,
+                                            uint32_t *__restrict__ mate, uint32_t *repeated)
+{
+    if (a == b)
+        raise_repeat(repeated);
+    else if (ea / (3u * kCcTile) != eb / (3u * kCcTile))
+        mate[ea] = eb / 3u;
+}
+
+// A run longer than a workgroup holds, list[first, last): thousands of triangles
+// on one edge, which three half-edges prove to be repeated, or as many edges
+// of one hash.  The same pairing in an open-addressed table in global memory, a
+// slot of `table` per entry, so it takes one insertion per entry however long the
+// run is; it ends as soon as a repeat is known.  An entry of the table is an
+// edge's first half-edge e as (e + 1) << 1, and bit 0 once the opposite one has come.
+__device__ void match_long_run(const uint32_t *__restrict__ T, const uint64_t *__restrict__ list, uint64_t first,
+                               uint64_t last, unsigned long long *table, uint32_t *__restrict__ mate,
+                               uint32_t *repeated)
+{
+    const uint64_t slots = last - first;
+    for (uint64_t k = threadIdx.x; k < slots; k += kCcTile)
+        __hip_atomic_store(&table[k], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __threadfence();
+    __syncthreads();
+    for (uint64_t i = first + threadIdx.x; i < last && !repeat_known(repeated); i += kCcTile) {
+        const uint32_t e = (uint32_t)list[i];
+        const uint64_t half = half_of(T, e), back = half << 32 | half >> 32;
+        // MurmurHash3's 64-bit finalizer, whose last step leaves the top half as
+        // it is: the run's entries share edge_hash
+        uint64_t h = half < back ? half : back;
+        h ^= h >> 33;
+        h *= 0xff51afd7ed558ccdull;
+        h ^= h >> 33;
+        h *= 0xc4ceb9fe1a85ec53ull;
+        uint64_t s = (h >> 32) * slots >> 32;  // slots fit 32 bits
+        for (uint64_t probe = 0; probe < slots; ++probe) {
+            const unsigned long long cur = atomicCAS(&table[s], 0ull, (unsigned long long)(e + 1ull) << 1);
+            if (cur == 0ull)
+                break;
+            const uint32_t o = (uint32_t)((cur >> 1) - 1ull);
+            const uint64_t other = half_of(T, o);
+            if (other == half || other == back) {
+                if ((cur & 1ull) || atomicOr(&table[s], 1ull) & 1ull)
+                    raise_repeat(repeated);
+                else
+                    pair_halves(half, e, other, o, mate, repeated);
+                break;
+            }
+            s = s + 1 < slots ? s + 1 : 0;
+        }
+    }
+}
+
+// spare: as many entries as list (the sort's other buffer)
 __global__ __launch_bounds__(kCcTile) void k_cc_match(const uint32_t *__restrict__ T,
                                                       const uint64_t *__restrict__ list,
-                                                      const uint32_t *__restrict__ count, uint32_t *__restrict__ mate,
-                                                      uint32_t *repeated)
+                                                      const uint32_t *__restrict__ count, uint64_t *__restrict__ spare,
+                                                      uint32_t *__restrict__ mate, uint32_t *repeated)
 {
     __shared__ uint64_t s_half[kCcHeld];  // from << 32 | to
     __shared__ uint32_t s_hash[kCcHeld], s_e[kCcHeld];
     __shared__ uint32_t s_edge[kCcEdgeSlots];
-    __shared__ uint32_t s_end;
+    __shared__ uint32_t s_end, s_last0, s_known;
     const uint64_t n = *count, first = (uint64_t)blockIdx.x * kCcTile;
     if (first >= n)
         return;
+    if (threadIdx.x == 0)
+        s_known = repeat_known(repeated);
+    __syncthreads();
+    if (s_known)  // the call fails whatever else is found
+        return;
     const uint32_t held = (uint32_t)(n - first < (uint64_t)kCcHeld ? n - first : (uint64_t)kCcHeld);
     const uint32_t own = held < (uint32_t)kCcTile ? held : (uint32_t)kCcTile;
-    auto half_of = [&](uint64_t key, uint32_t &e) -> uint64_t {
-        e = (uint32_t)(key & 0xffffffffull);
-        return (uint64_t)T[e] << 32 | T[e % 3u == 2u ? e - 2u : e + 1u];
-    };
     auto hash_at = [&](uint64_t i) -> uint32_t { return (uint32_t)(list[i] >> kOpenShift); };
     // the hash of the run that came in from the workgroup before, which takes it
     const uint32_t before = first ? hash_at(first - 1) : ~0u;  // no hash has 32 bits
     for (uint32_t j = threadIdx.x; j < held; j += kCcTile) {
         const uint64_t key = list[first + j];
         s_hash[j] = (uint32_t)(key >> kOpenShift);
-        s_half[j] = half_of(key, s_e[j]);
+        s_e[j] = (uint32_t)key;
+        s_half[j] = half_of(T, s_e[j]);
     }
     for (int k = threadIdx.x; k < kCcEdgeSlots; k += kCcTile)
         s_edge[k] = 0;
-    if (threadIdx.x == 0)
+    if (threadIdx.x == 0) {
         s_end = held;
+        s_last0 = own - 1;
+    }
     __syncthreads();
-    // its last run ends before entry s_end
+    // its last run is the entries [s_last0, s_end), as far as held
     const uint32_t last = s_hash[own - 1];
-    for (uint32_t j = own + threadIdx.x; j < held; j += kCcTile)
-        if (s_hash[j] != last)
+    for (uint32_t j = threadIdx.x; j < held; j += kCcTile) {
+        if (j < own && s_hash[j] == last)
+            atomicMin(&s_last0, j);
+        else if (j >= own && s_hash[j] != last)
             atomicMin(&s_end, j);
+    }
     __syncthreads();
-    const uint32_t end = s_end;
-    auto pair = [&](uint64_t a, uint32_t ea, uint64_t b, uint32_t eb) {  // the halves a and b of one edge
-        if (a == b)
-            atomicOr(repeated, 1u);
-        else if (ea / (3u * kCcTile) != eb / (3u * kCcTile))
-            mate[ea] = eb / 3u;
-    };
+    const bool longRun = s_end == held && first + held < n && hash_at(first + held) == last;
+    const uint32_t end = longRun ? s_last0 : s_end;
     for (uint32_t j = threadIdx.x; j < end; j += kCcTile) {
         if (s_hash[j] == before)
             continue;
@@ -366,35 +440,26 @@ __global__ __launch_bounds__(kCcTile) void k_cc_match(const uint32_t *__restrict
             const uint32_t o = (cur >> 1) - 1;
             if (s_half[o] == half || s_half[o] == back) {
                 if ((cur & 1u) || atomicOr(&s_edge[s], 1u) & 1u)
-                    atomicOr(repeated, 1u);
+                    raise_repeat(repeated);
                 else
-                    pair(half, s_e[j], s_half[o], s_e[o]);
+                    pair_halves(half, s_e[j], s_half[o], s_e[o], mate, repeated);
                 break;
             }
             s = (s + 1) & (kCcEdgeSlots - 1);
         }
-        // a last run longer than the workgroup holds (an edge of hundreds of
-        // triangles, or as many edges of one hash): its entries past those
-        // held are compared with all of it, this one's with the ones behind
-        if (end == held && first + held < n && s_hash[j] == last)
-            for (uint64_t i = first + held; i < n && hash_at(i) == last; ++i) {
-                uint32_t o;
-                const uint64_t other = half_of(list[i], o);
-                if (other == half || other == back)
-                    pair(half, s_e[j], other, o);
-            }
     }
-    if (end == held && first + held < n && last != before)
-        for (uint64_t j = first + held + threadIdx.x; j < n && hash_at(j) == last; j += kCcTile) {
-            uint32_t t;
-            const uint64_t half = half_of(list[j], t), back = half << 32 | half >> 32;
-            for (uint64_t i = j + 1; i < n && hash_at(i) == last; ++i) {
-                uint32_t o;
-                const uint64_t other = half_of(list[i], o);
-                if (other == half || other == back)
-                    pair(half, t, other, o);
-            }
+    if (longRun && last != before) {
+        uint64_t a = first + held, b = n;  // the run's end: the first entry of another hash
+        while (a < b) {
+            const uint64_t m = a + (b - a) / 2;
+            if (hash_at(m) == last)
+                a = m + 1;
+            else
+                b = m;
         }
+        const uint64_t run = first + s_last0;
+        match_long_run(T, list, run, a, reinterpret_cast<unsigned long long *>(spare + run), mate, repeated);
+    }
 }
 
 // Unites the triangles of mated half-edges.  A tile's border meets few others
@@ -518,7 +583,7 @@ void launch_components(const uint32_t *T, uint32_t nt, size_t nv, const uint8_t 
     const int bits[2] = {kOpenShift, kOpenShift + open_bits(he)};
     const bool alt = radix_sort_u64(list, listAlt, he, bits, 1, hist, s, count) != 0;
     hipLaunchKernelGGL(k_cc_match, dim3((unsigned)((he + kCcTile - 1) / kCcTile)), dim3(kCcTile), 0, s, T,
-                       alt ? listAlt : list, count, mate, repeated);
+                       alt ? listAlt : list, count, alt ? list : listAlt, mate, repeated);
     hipLaunchKernelGGL(k_cc_unite, tiles, dim3(kCcTile), 0, s, mate, nt, parent);
     hipLaunchKernelGGL(k_cc_labels, dim3((nt + kComponentBlock - 1) / kComponentBlock), dim3(kComponentBlock), 0, s,
                        blocked, nt, parent, labels);

@@ -838,6 +838,65 @@ def test_components_repeats_across_tiles(gpu, copies):
     assert np.all(got[~blocked] == 0) and np.all(got[blocked] == 0xFFFFFFFF)
 
 
+@pytest.mark.parametrize("copies", [2, 2500, 120000])
+@pytest.mark.parametrize("shape", ["duplicate", "collapsed"])
+def test_components_many_on_one_edge(gpu, shape, copies):
+    """Up to far more triangles on one edge than a tile or a workgroup's share of
+    the listed half-edges holds (copies of one triangle, triangles collapsed to
+    a point): refused as repeated half-edges, in time linear in their number,
+    and with them blocked the mesh's own groups."""
+    import time
+
+    m = mg.torus(1.0, 0.3, 64, 40)
+    extra = np.repeat(m.triangles[7:8] if shape == "duplicate" else np.zeros((1, 3), m.triangles.dtype), copies, axis=0)
+    tris = np.concatenate([m.triangles[:3000], extra, m.triangles[3000:]])
+    G = gpu.mesh(m.vertices, tris, prepare=False)
+    begin = time.perf_counter()
+    with pytest.raises(N.SbgError, match="repeated half-edge"):
+        G.components()
+    assert time.perf_counter() - begin < 2.0  # one insertion each: some ms
+    blocked = np.zeros(len(tris), np.uint8)
+    blocked[3000:3000 + copies] = 1
+    got = G.components(blocked)
+    assert np.all(got[blocked == 0] == 0) and np.all(got[blocked == 1] == 0xFFFFFFFF)
+
+
+@pytest.mark.parametrize("share,open_every", [(1500, 0), (2600, 0), (2600, 3)])
+def test_components_edges_of_one_hash(gpu, share, open_every):
+    """More listed half-edges of one hash than a workgroup holds, none of them
+    repeated: two-triangle shells whose edge a -> b hashes to one value, the two
+    triangles of a shell in different tiles (some without the second one)."""
+    from oracle.oracle import face_groups
+
+    def top_hash(lo, hi):  # the top 8 of the 32 bits by which edges are listed (up to 16,384 half-edges)
+        h = lo * np.uint32(2654435761) ^ hi * np.uint32(2246822519)
+        h ^= h >> np.uint32(15)
+        h *= np.uint32(0x85EBCA6B)
+        h ^= h >> np.uint32(13)
+        return (h * np.uint32(0xC2B2AE35)) >> np.uint32(24)
+
+    nv = 1 << 21
+    v = np.arange(nv, dtype=np.uint32).reshape(-1, 2)
+    same = v[top_hash(v[:, 0], v[:, 1]) == 77]
+    third = v[top_hash(v[:, 0], v[:, 1]) == 78].ravel()
+    a, b, c = same[:share, 0], same[:share, 1], third[:share]
+    assert len(a) == len(c) == share
+    front, back = np.stack([a, b, c], 1), np.stack([b, a, c], 1)
+    if open_every:
+        back = back[np.arange(share) % open_every != 0]
+    tris = np.concatenate([front, back])
+    assert 3 * len(tris) <= 1 << 14
+    assert 2 * share > 1536
+    G = gpu.mesh(np.zeros((nv, 3)), tris, prepare=False)
+    want = face_groups(tris.astype(np.int64), None)
+    assert np.array_equal(G.components().astype(np.int64), want)
+    assert want.max() == share - 1 and np.count_nonzero(want < share) == len(tris)
+    # one of the shells closed twice: its half-edges are repeated
+    G = gpu.mesh(np.zeros((nv, 3)), np.concatenate([tris, tris[-1:]]), prepare=False)
+    with pytest.raises(N.SbgError, match="repeated half-edge"):
+        G.components()
+
+
 def test_half_edges_vs_dict(gpu):
     """sbg_half_edges against a dictionary half-edge map built in index order
     (the reference's unordered_map keyed (from << 32) | to, first insert
