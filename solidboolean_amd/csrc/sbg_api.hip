@@ -147,13 +147,6 @@ struct MeshUse {
     }
 };
 
-// waits for the second stream when leaving (work queued there must not
-// outlive the call, whatever path it returns by)
-struct AuxJoin {
-    sbg_context c;
-    ~AuxJoin() { (void)hipStreamSynchronize(c->aux); }
-};
-
 extern "C" {
 
 const char *sbg_last_error(void) { return g_err.c_str(); }
@@ -753,11 +746,13 @@ int sbg_components(sbg_mesh m, const uint8_t *blocked, uint32_t *labels)
         TRY(c->ccBlocked.ensure(nt));
         TRY(copy_in(c, {part_in(c->ccBlocked.p, blocked, nt)}));
     }
+    StreamJoin join(c->stream);
     launch_components(m->T.p, (uint32_t)nt, m->nv, blocked ? c->ccBlocked.p : nullptr, c->ccList.p, c->ccListAlt.p,
                       c->hist.p, c->ccValence.p, c->ccMate.p, c->ccParent.p, c->ccLabels.p, c->stream);
     TRY(check_launch("components"));
     uint32_t *repeated = c->pinned + kComponentsPinned;
     HIP_TRY(hipMemcpyAsync(repeated, c->ccValence.p + m->nv + 1, sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
+    join.release();
     TRY(copy_out(c, {{c->ccLabels.p, labels, sizeof(uint32_t) * nt}}));
     if (*repeated)
         return fail(SBG_ERR_INVALID, "repeated half-edge: two unblocked triangles share a directed edge");
@@ -785,9 +780,11 @@ int sbg_half_edges(sbg_context c, const uint32_t *tris, size_t ntris, const uint
     TRY(c->heRepeat.ensure(1));
     TRY(copy_in(c, {part_in(c->heTris.p, tris, sizeof(uint32_t) * 3 * ntris),
                     part_in(c->heQueries.p, queries, sizeof(uint64_t) * nqueries)}));
+    StreamJoin join(c->stream);
     launch_half_edges(c->heTris.p, (uint32_t)ntris, c->heQueries.p, (uint32_t)nqueries, c->ccKeys.p, c->ccOwners.p,
                       c->heOpposite.p, c->heQueryOwner.p, c->heRepeat.p, c->stream);
     TRY(check_launch("half edges"));
+    join.release();
     return copy_out(c, {{c->heOpposite.p, opposite, sizeof(uint32_t) * 3 * ntris},
                         {c->heQueryOwner.p, query_owner, sizeof(uint32_t) * nqueries},
                         {c->heRepeat.p, first_repeat, sizeof(uint32_t)}});
@@ -1261,8 +1258,10 @@ int sbg_tri_tri_batch(sbg_context ctx, const double *a9, const double *b9, size_
     TRY(ctx->rawSeg.ensure(6 * n));
     TRY(ctx->rawStatus.ensure(n));
     TRY(copy_in(ctx, {part_in(ctx->rawA.p, a9, sizeof(double) * 9 * n), part_in(ctx->rawB.p, b9, sizeof(double) * 9 * n)}));
+    StreamJoin join(ctx->stream);
     launch_tritri_raw(ctx->rawA.p, ctx->rawB.p, (uint32_t)n, ctx->rawStatus.p, ctx->rawSeg.p, ctx->stream);
     TRY(check_launch("tri_tri_raw"));
+    join.release();
     return copy_out(ctx, {{ctx->rawStatus.p, status, n}, {ctx->rawSeg.p, seg, sizeof(double) * 6 * n}});
 }
 
@@ -1459,11 +1458,13 @@ constexpr size_t kSharedQueries = 600000;
 
 // enqueue, wait, check; a side whose grid turned out too small is run again
 // with the grid at its exact size.  The queries stand on the context stream.
+// Whatever it returns, nothing that writes the votes is queued any more.
 static int run_rays(RayJob *jobs, int njobs, bool ordered, bool allAxes, bool cleared)
 {
     sbg_context c = jobs[0].target->ctx;
+    StreamJoin join(c->stream);
     if (njobs == 2 && jobs[0].n + jobs[1].n > kSharedQueries) {
-        const AuxJoin join{c};
+        const StreamJoin joinAux(c->aux);
         HIP_TRY(hipEventRecord(c->auxReady, c->stream));
         HIP_TRY(hipStreamWaitEvent(c->aux, c->auxReady, 0));
         TRY(enqueue_rays(jobs, 1, ordered, allAxes, cleared, c->stream));
@@ -1485,6 +1486,7 @@ static int run_rays(RayJob *jobs, int njobs, bool ordered, bool allAxes, bool cl
             if (still)
                 return fail(SBG_ERR_OVERFLOW, "ray grid did not fit after a resize");
         }
+    join.release();
     return SBG_OK;
 }
 
@@ -1504,7 +1506,7 @@ int sbg_classify_points(sbg_mesh target, const double *pts, size_t n, uint8_t *a
     TRY(c->pts.ensure(3 * n));
     TRY(c->bits.ensure(3 * n + 4));
     TRY(c->votes.ensure(n));
-    TRY(copy_in(c, {part_in(c->pts.p, pts, sizeof(double) * 3 * n)}));
+    TRY(copy_in(c, {part_in(c->pts.p, pts, sizeof(double) * 3 * n)}));  // run_rays waits
     RayJob job = {target, ray_bufs(c, 0), c->pts.p, nullptr, nullptr, n, inside, RayJob::kNone};
     TRY(run_rays(&job, 1, false, axis_inside != nullptr, false));
     if (!axis_inside)
@@ -1754,6 +1756,7 @@ int sbg_adjoint(sbg_context ctx, const double *xyz_in, size_t nin, const uint32_
                       part_in(ctx->adjSrc.p, src, sizeof(uint32_t) * 5 * nd),
                       part_in(ctx->adjFaces.p, faces, sizeof(uint32_t) * 3 * nf),
                       part_in(ctx->adjGradD.p, grad_derived, wantGrad && grad_derived ? sizeof(double) * 3 * nd : 0)}));
+    StreamJoin join(s);
     launch_fill_u32(reinterpret_cast<uint32_t *>(ctx->adjVol.p), 0u, 2, s);
     if (wantGrad)
         launch_fill_u32(reinterpret_cast<uint32_t *>(ctx->adjGall.p), 0u, 6 * nall, s);
@@ -1761,6 +1764,7 @@ int sbg_adjoint(sbg_context ctx, const double *xyz_in, size_t nin, const uint32_
                    vol_weight, (wantGrad && grad_derived) ? ctx->adjGradD.p : nullptr, ctx->adjAll.p, ctx->adjVol.p,
                    wantGrad ? ctx->adjGall.p : nullptr, s);
     TRY(check_launch("adjoint"));
+    join.release();
     return copy_out(ctx, {{ctx->adjAll.p + 3 * nin, derived_xyz, derived_xyz ? sizeof(double) * 3 * nd : 0},
                           {ctx->adjVol.p, volume, volume ? sizeof(double) : 0},
                           {ctx->adjGall.p, grad_in, wantGrad ? sizeof(double) * 3 * nin : 0}});

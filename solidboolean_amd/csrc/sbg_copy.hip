@@ -357,21 +357,20 @@ static int plan_parts(sbg_context c, std::initializer_list<CopyPart> parts, bool
     return SBG_OK;
 }
 
-// Work queued on the context stream after the call sees the data; the caller's
-// call waits for the context stream before it returns.
+// Work queued on the context stream after the call sees the data.
 int copy_in(sbg_context c, std::initializer_list<CopyPart> parts)
 {
     CopyPlan plan;
+    StreamJoin join(c->stream);
     TRY(plan_parts(c, parts, true, plan));
-    if (!plan.total)
-        return SBG_OK;
-    TRY(copy_setup(c, std::min(plan.total, 2 * kStageHalf)));
-    std::atomic<uint64_t> top{0};
-    const hipError_t e = queue_in(c, plan, c->stream, top);
-    if (e != hipSuccess) {
-        (void)hipStreamSynchronize(c->stream);
-        return fail(SBG_ERR_HIP, "copy to the GPU failed: %s", hipGetErrorString(e));
+    if (plan.total) {
+        TRY(copy_setup(c, std::min(plan.total, 2 * kStageHalf)));
+        std::atomic<uint64_t> top{0};
+        const hipError_t e = queue_in(c, plan, c->stream, top);
+        if (e != hipSuccess)
+            return fail(SBG_ERR_HIP, "copy to the GPU failed: %s", hipGetErrorString(e));
     }
+    join.release();
     return SBG_OK;
 }
 
@@ -380,8 +379,10 @@ int copy_in(sbg_context c, std::initializer_list<CopyPart> parts)
 int copy_out(sbg_context c, std::initializer_list<CopyPart> parts)
 {
     CopyPlan plan;
+    StreamJoin join(c->stream);
     TRY(plan_parts(c, parts, false, plan));
     if (!plan.total) {
+        join.release();
         HIP_TRY(hipStreamSynchronize(c->stream));
         return SBG_OK;
     }
@@ -412,6 +413,7 @@ int copy_out(sbg_context c, std::initializer_list<CopyPart> parts)
         });
     }
     const hipError_t es = hipStreamSynchronize(c->stream);
+    join.release();
     if (e != hipSuccess || (e = es) != hipSuccess)
         return fail(SBG_ERR_HIP, "copy from the GPU failed: %s", hipGetErrorString(e));
     return SBG_OK;

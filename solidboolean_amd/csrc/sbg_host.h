@@ -199,6 +199,22 @@ int use(sbg_context ctx);
 void context_release(sbg_context ctx);
 void context_free(sbg_context ctx);
 
+// Waits for a stream when a call leaves, whatever path it returns by: for work
+// queued there that reads or writes the caller's arrays, or the staging that
+// the next call fills.  release(): the call waits by itself from here on.
+struct StreamJoin {
+    hipStream_t s;
+    explicit StreamJoin(hipStream_t stream) : s(stream) {}
+    StreamJoin(const StreamJoin &) = delete;
+    StreamJoin &operator=(const StreamJoin &) = delete;
+    ~StreamJoin()
+    {
+        if (s)
+            (void)hipStreamSynchronize(s);
+    }
+    void release() { s = nullptr; }
+};
+
 // HIP-event bracket of one stage (no-op unless timing is enabled)
 struct Stage {
     sbg_context c;
@@ -238,7 +254,9 @@ struct CopyPart {
     Kind kind = kBytes;
 };
 inline CopyPart part_in(void *dev, const void *host, size_t bytes) { return {dev, const_cast<void *>(host), bytes}; }
-// up to kCopyParts arrays; parts of 0 bytes are skipped
+// Up to kCopyParts arrays; parts of 0 bytes are skipped.  copy_in leaves its
+// copies queued on the context stream when it succeeds (the caller holds a
+// StreamJoin until it waits); a failed copy_in, and copy_out always, have waited.
 int copy_in(sbg_context c, std::initializer_list<CopyPart> parts);
 int copy_out(sbg_context c, std::initializer_list<CopyPart> parts);
 void copy_free(sbg_context c);
