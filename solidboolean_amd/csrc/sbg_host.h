@@ -109,6 +109,8 @@ constexpr uint32_t kSpillInit = 2048, kSpillMax = 1u << 15;
 // intersecting pairs and segments up to this size leave through page-locked
 // staging (74,898 of them)
 constexpr size_t kHitStage = (size_t)4 << 20;
+// pair lists whose hit counts share one page-locked block
+constexpr size_t kHitSlots = 1024;
 // transfers of host arrays (sbg_copy.hip): host threads, the page-locked staging
 // (two halves), the piece a thread takes at a time, what is worth a thread, what
 // leaves the GPU between two waits, and the arrays of one call
@@ -158,6 +160,9 @@ struct sbg_context_s {
     DevBuf<uint32_t> ovf, rayList, ovf2, rayList2;
     PinnedBuf votesHost, votesHost2;  // vote readbacks of the two sets
     PinnedBuf hitStage;               // sbg_pairs_hits: kHitStage bytes
+    // page-locked words for the hit counts of the live pair lists, in blocks of
+    // kHitSlots, and those that no list has
+    std::vector<uint32_t *> hitBlocks, hitFree;
     DevBuf<unsigned long long> workCounts;  // sbg_bench_rays
     DevBuf<unsigned long long> ccKeys;      // sbg_half_edges: half-edge table
     DevBuf<uint32_t> ccOwners;

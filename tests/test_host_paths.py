@@ -57,6 +57,29 @@ CALLS = {
 }
 
 
+def test_pair_lists_share_page_locked_memory(fake_hip):
+    """Lists kept alive together, and made after others were dropped, take their
+    hit counts' page-locked words from blocks of the context's."""
+    run(fake_hip, """
+A, B = soup(50), soup(60)
+def lists(n):
+    out = [A.find_pairs(B) for _ in range(n)]
+    for p in out:
+        p.tri_tri(A, B, N.FP64, stats=False)
+    return out
+lists(1)
+before = fake.fake_host_allocs()
+keep = lists(1000)
+assert fake.fake_host_allocs() == before
+for p in keep[:600]:
+    p.close()
+keep += lists(600)
+assert fake.fake_host_allocs() == before
+keep += lists(1000)
+assert fake.fake_host_allocs() == before + 1
+""")
+
+
 @pytest.mark.parametrize("name", CALLS)
 def test_failed_call_leaves_nothing_queued(fake_hip, name):
     """A launch that fails after the call's arrays were queued to the GPU, or after
