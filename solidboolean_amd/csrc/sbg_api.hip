@@ -1606,12 +1606,15 @@ static int classify_sides(sbg_mesh self[2], sbg_mesh other[2], sbg_pairs p, uint
     const RayBufs sets[2] = {ray_bufs(c, 0), ray_bufs(c, 1)};
     const RayBufs *rb[2] = {&sets[0], &sets[self[0] ? 1 : 0]};
     TRY(enqueue_queries(c, self, p, rb));
-    std::vector<RayJob> jobs;
-    for (int k = 0; k < 2; ++k)
-        if (self[k])
-            jobs.push_back({other[k], *rb[k], rb[k]->pts.p, self[k]->sortedIds, rb[k]->flags.p, self[k]->nt, out[k],
-                            RayJob::kNone});
-    return run_rays(jobs.data(), (int)jobs.size(), true, false, true);
+    auto job = [&](int k) -> RayJob {
+        return {other[k], *rb[k], rb[k]->pts.p, self[k]->sortedIds, rb[k]->flags.p, self[k]->nt, out[k], RayJob::kNone};
+    };
+    if (self[0] && self[1]) {
+        RayJob jobs[2] = {job(0), job(1)};
+        return run_rays(jobs, 2, true, false, true);
+    }
+    RayJob only = job(self[0] ? 0 : 1);
+    return run_rays(&only, 1, true, false, true);
 }
 
 int sbg_classify_triangles(sbg_mesh self, sbg_mesh other, sbg_pairs p, int side, uint8_t *out)

@@ -9,6 +9,7 @@
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <new>
 #include <string>
 #include <vector>
 
@@ -41,6 +42,7 @@ int failSkip = -1;
 int hostAllocs = 0;
 const volatile uint8_t *watch = nullptr;
 std::string watched;
+bool failNew = false;
 
 void finish(Stream *s, uint64_t upTo)
 {
@@ -60,6 +62,17 @@ int index_of(const Stream *s)
 }
 
 }  // namespace
+
+// the library's C++ allocations resolve here too
+void *operator new(size_t n)
+{
+    void *p = failNew ? nullptr : malloc(n ? n : 1);
+    if (!p)
+        throw std::bad_alloc();
+    return p;
+}
+void operator delete(void *p) noexcept { free(p); }
+void operator delete(void *p, size_t) noexcept { free(p); }
 
 extern "C" {
 
@@ -87,6 +100,8 @@ void fake_drain(void)
     for (Stream *s : streams)
         s->done = s->queued;
 }
+// C++ allocations throw from now on, or no longer do
+void fake_fail_new(int on) { failNew = on != 0; }
 int fake_host_allocs(void) { return hostAllocs; }
 // from now on every wait for a stream notes the stream's number and *p
 void fake_watch(const uint8_t *p)
@@ -145,6 +160,7 @@ int hipStreamCreateWithFlags(void **s, unsigned)
 {
     Lock l(mu);
     streams.push_back(new Stream);
+    streams.back()->deps.reserve(4096);  // a wait allocates nothing
     *s = streams.back();
     return 0;
 }

@@ -80,6 +80,25 @@ assert fake.fake_host_allocs() == before + 1
 """)
 
 
+def test_classification_survives_a_failed_allocation(fake_hip):
+    """No C++ exception leaves the classification entry points when the heap is
+    exhausted: once its buffers stand, a call allocates nothing and succeeds."""
+    run(fake_hip, """
+A, B = soup(50), soup(60)
+P = A.find_pairs(B)
+P.tri_tri(A, B, N.FP64, stats=False)
+def calls(out=None):
+    out = A.classify_pair(B, P, out=out)
+    A.classify_triangles(B, P, 0)
+    B.classify_triangles(A, P, 1)
+    return out
+out = calls()
+fake.fake_fail_new(1)
+calls(out)
+fake.fake_fail_new(0)
+""")
+
+
 @pytest.mark.parametrize("name", CALLS)
 def test_failed_call_leaves_nothing_queued(fake_hip, name):
     """A launch that fails after the call's arrays were queued to the GPU, or after
