@@ -438,15 +438,13 @@ __device__ __forceinline__ uint32_t hits_of(uint4 v)
 }
 
 // blockOffsets: hits before each workgroup (null: counted here).  The last
-// workgroup writes the total to *nHits, the first copy for kernels, and to
-// *hostHits (page-locked).
+// workgroup writes the total to *hostHits (page-locked).
 __global__ __launch_bounds__(kCompactBlock) void k_hit_write(const uint64_t *__restrict__ pairs,
                                                              const uint8_t *__restrict__ status,
                                                              const double *__restrict__ seg, uint32_t n,
                                                              const uint32_t *__restrict__ blockOffsets,
                                                              uint64_t *__restrict__ hitPairs,
-                                                             double *__restrict__ hitSeg, uint32_t *nHits,
-                                                             uint32_t *hostHits)
+                                                             double *__restrict__ hitSeg, uint32_t *hostHits)
 {
     const uint32_t i = blockIdx.x * kCompactBlock + threadIdx.x;
     const bool hit = i < n && status[i] == 1;
@@ -485,7 +483,6 @@ __global__ __launch_bounds__(kCompactBlock) void k_hit_write(const uint64_t *__r
         uint32_t tot = s_before;
         for (int w = 0; w < kCompactBlock / 64; ++w)
             tot += s_wave[w];
-        *nHits = tot;
         *hostHits = tot;
     }
 }
@@ -625,8 +622,8 @@ void launch_tritri_raw(const double *a9, const double *b9, uint32_t n, uint8_t *
 void launch_exclusive_scan(uint32_t *data, size_t m, hipStream_t s);
 
 void launch_compact_hits(const uint64_t *pairs, const uint8_t *status, const double *seg, uint32_t n,
-                         uint32_t *blockCounts, uint64_t *hitPairs, double *hitSeg, uint32_t *nHits,
-                         uint32_t *hostHits, hipStream_t s)
+                         uint32_t *blockCounts, uint64_t *hitPairs, double *hitSeg, uint32_t *hostHits,
+                         hipStream_t s)
 {
     if (n == 0)
         return;
@@ -637,7 +634,7 @@ void launch_compact_hits(const uint64_t *pairs, const uint8_t *status, const dou
         launch_exclusive_scan(blockCounts, (size_t)nb, s);
     }
     hipLaunchKernelGGL(k_hit_write, dim3(nb), dim3(kCompactBlock), 0, s, pairs, status, seg, n,
-                       onePass ? nullptr : blockCounts, hitPairs, hitSeg, nHits, hostHits);
+                       onePass ? nullptr : blockCounts, hitPairs, hitSeg, hostHits);
 }
 
 }  // namespace sbg

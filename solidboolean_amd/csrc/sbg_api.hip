@@ -115,7 +115,7 @@ struct sbg_pairs_s {
     DevBuf<uint8_t> status;
     DevBuf<double> seg, hitSeg;
     DevBuf<uint64_t> hitPairs;
-    DevBuf<uint32_t> blockCounts, nHits, work;
+    DevBuf<uint32_t> blockCounts, work;
     uint32_t *hostHits = nullptr;  // the compaction's hit count, valid once its stream is done
     bool tested = false;
     // largest first / second index in the list (host-built lists are checked
@@ -326,7 +326,6 @@ static void pairs_free_buffers(sbg_pairs p)
     p->hitSeg.release();
     p->hitPairs.release();
     p->blockCounts.release();
-    p->nHits.release();
     p->work.release();
 }
 
@@ -1161,7 +1160,6 @@ static int run_tri_tri(sbg_mesh a, sbg_mesh b, sbg_pairs p, int precision, GdSta
     TRY(p->hitPairs.ensure(p->n));
     TRY(p->hitSeg.ensure(6 * p->n));
     TRY(p->blockCounts.ensure((size_t)compact_blocks(n)));
-    TRY(p->nHits.ensure(1));
     TRY(take_hit_slot(p));
     TRY(p->work.ensure(tritri_work_u32((uint32_t)p->n)));
     {
@@ -1172,10 +1170,8 @@ static int run_tri_tri(sbg_mesh a, sbg_mesh b, sbg_pairs p, int precision, GdSta
     }
     {
         Stage st(c, SBG_STAGE_COMPACT);
-        if (n == 0)  // otherwise the compaction's last block writes the count
-            launch_fill_u32(p->nHits.p, 0u, 1, c->stream);
         launch_compact_hits(p->pairs.p, p->status.p, p->seg.p, n, p->blockCounts.p, p->hitPairs.p, p->hitSeg.p,
-                            p->nHits.p, p->hostHits, c->stream);
+                            p->hostHits, c->stream);
         TRY(check_launch("compact"));
     }
     return SBG_OK;

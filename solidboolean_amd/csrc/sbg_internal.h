@@ -160,10 +160,10 @@ void launch_tritri(const double *tri64A, const double *tri64B, const float *tri3
 void launch_tritri_raw(const double *a9, const double *b9, uint32_t n, uint8_t *status, double *seg,
                        hipStream_t s);
 // compaction of hits (status == 1) into (pair, seg) lists, in pair order; their
-// number goes to *nHits and *hostHits (page-locked)
+// number goes to *hostHits (page-locked; not written for n = 0)
 void launch_compact_hits(const uint64_t *pairs, const uint8_t *status, const double *seg, uint32_t n,
-                         uint32_t *blockCounts, uint64_t *hitPairs, double *hitSeg, uint32_t *nHits,
-                         uint32_t *hostHits, hipStream_t s);
+                         uint32_t *blockCounts, uint64_t *hitPairs, double *hitSeg, uint32_t *hostHits,
+                         hipStream_t s);
 void launch_hit_export(const uint64_t *hitPairs, const double *hitSeg, uint32_t n, uint32_t *ab, double *seg,
                        hipStream_t s);
 int compact_blocks(uint32_t n);
