@@ -155,9 +155,6 @@ __global__ __launch_bounds__(kTreeTile) void k_tree_tiles(const K *__restrict__ 
             }
             if (dl < 0 && dr < 0) {  // the whole tree
                 write_root(rootBox, wl, wh);
-                const float b[6] = {wl.x, wl.y, wl.z, wh.x, wh.y, wh.z};
-                put6(tileBox, b);
-                list_piece(out, &s_npiece, ref, b);
                 break;
             }
             const int split = left ? hi : lo - 1;
@@ -215,11 +212,8 @@ __global__ __launch_bounds__(kTreeTile) void k_tree_tiles(const K *__restrict__ 
         s_start[lo] = 1;
         s_stop[hi] = 1;
     }
-    if (gridDim.x == 1) {  // one tile: no top node, the root its only piece
-        if (me == 0 && out.count)
-            out.count[0] = 1;
+    if (gridDim.x == 1)  // one tile: no top node, and a search starts from the root
         return;
-    }
     // indices no node of the tile took: slots from LDS, one global reservation
     // per tile (one per wave held the kernel to the rate of one counter: 215
     // us at 3.0 M leaves)

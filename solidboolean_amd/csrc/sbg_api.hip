@@ -931,7 +931,7 @@ int sbg_find_pairs(sbg_mesh a, sbg_mesh b, sbg_pairs *out)
             Stage st(c, SBG_STAGE_TRAVERSE);
             launch_fill_u32(cnt, 0u, kMaxLevels + 8, c->stream);
             const uint32_t tilesA = tree_tiles((uint32_t)na), tilesB = tree_tiles((uint32_t)nb);
-            // from the tiles wherever a tree has several of them
+            // from the tiles where both trees have several of them
             const bool byTiles = tilesA > 1 && tilesB > 1 && (uint64_t)tilesA * tilesB <= kTilePairsMax;
             if (byTiles)
                 launch_search_tiles(tile_set(a), tile_set(b), c->front[0].p, cnt, fcap, overflow, c->stream);

@@ -86,8 +86,8 @@ size_t tree_scratch_floats(uint32_t n);
 // pieces: filled for the pair search (launch_search_tiles)
 constexpr int kTreeTile = 1024;  // sorted leaves per tile
 // The largest subtrees inside each tile ("pieces": what the nodes crossing its
-// borders have for children there; the root for a tree of one tile): 2 float4
-// each, (lo xyz, node reference) and (hi xyz, 0), kTilePieces slots per tile.
+// borders have for children there; none are listed for a tree of one tile): 2
+// float4 each, (lo xyz, node reference) and (hi xyz, 0), kTilePieces slots per tile.
 // Nodes crossing one border lie on one path of the tree, on which the common
 // prefix of the keys grows from 8 (24-bit codes in 32 bits) to 31 and, by
 // index, from 32 to 63 bits: 55 at most, each with one piece in the tile.
