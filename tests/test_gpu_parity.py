@@ -1,10 +1,13 @@
 """GPU parity: the HIP path (through the C ABI) against the reference's golden
 vectors and the oracle.  Integer, index and FP64 results are compared bit for
 bit; the FP32-filtered mode must give exactly the FP64 results."""
+import os
+import re
+
 import numpy as np
 import pytest
 
-from conftest import FULL_CASES, golden_exists, load_golden
+from conftest import FULL_CASES, ROOT, golden_exists, load_golden
 from oracle.oracle import OracleMesh
 from solidboolean_amd import meshgen as mg
 from solidboolean_amd import native as N
@@ -692,10 +695,13 @@ def test_classify_pair_ragged_sides(gpu, na, nb):
 def test_classify_pair_split_sides(gpu):
     """A pair past the size up to which both sides share their launches, and
     one just below: votes equal to the single-side calls'."""
-    for size in (250, 270):
+    src = open(os.path.join(ROOT, "solidboolean_amd", "csrc", "sbg_api.hip")).read()
+    shared = int(re.search(r"kSharedQueries = (\d+);", src).group(1))
+    for size, above in ((270, False), (280, True)):
         a = mg.torus(1.0, 0.3, 2 * size, size)
         b = mg.transform(mg.torus(1.0, 0.25, 2 * size + 3, size), mg.random_rotation(mg.SplitMix64(size)),
                          (0.5, 0.1, 0.1))
+        assert (a.nt + b.nt > shared) == above and abs(a.nt + b.nt - shared) < shared // 10
         A, B = gpu.mesh(a.vertices, a.triangles), gpu.mesh(b.vertices, b.triangles)
         P = A.find_pairs(B)
         P.tri_tri(A, B, N.FP32_FILTERED)
