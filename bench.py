@@ -323,7 +323,7 @@ def stress_section(ctx, mg, N, steps: int) -> dict:
         a, b = make()
         A = ctx.mesh(a.vertices, a.triangles, prepare=False)
         B = ctx.mesh(b.vertices, b.triangles, prepare=False)
-        votes = (N.host_array(A.nt), N.host_array(B.nt))  # page-locked: the votes arrive by DMA
+        votes = (N.host_array(A.nt), N.host_array(B.nt))  # page-locked: a kernel writes the votes there
 
         def step():
             A.prepare()
@@ -506,7 +506,7 @@ def main():
     A = ctx.mesh(a.vertices, a.triangles, prepare=False)
     B = ctx.mesh(b.vertices, b.triangles, prepare=False)
     # the vote arrays are reused step after step, as a pipeline would
-    votes = (N.host_array(A.nt), N.host_array(B.nt))  # page-locked: the votes arrive by DMA
+    votes = (N.host_array(A.nt), N.host_array(B.nt))  # page-locked: a kernel writes the votes there
 
     def step(precision=N.FP32_FILTERED):
         A.prepare()

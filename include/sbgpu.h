@@ -57,7 +57,7 @@ typedef struct {
 enum {
     SBG_STAGE_RECORDS = 0, /* triangle records, normals, leaf boxes, Morton keys */
     SBG_STAGE_SORT,        /* Morton radix sort */
-    SBG_STAGE_BVH,         /* Karras hierarchy + refit */
+    SBG_STAGE_BVH,         /* radix tree and boxes, bottom-up in tiles, then the nodes above them */
     SBG_STAGE_TRAVERSE,    /* tree-vs-tree candidate search */
     SBG_STAGE_PAIR_SORT,   /* canonical (a, b) order of the candidates */
     SBG_STAGE_TRI_TRI,     /* Guigue-Devillers kernel */
@@ -93,9 +93,9 @@ int sbg_mesh_create(sbg_context ctx, const double *xyz, size_t nverts, const uin
 int sbg_mesh_create64(sbg_context ctx, const double *xyz, size_t nverts, const uint64_t *tris, size_t ntris,
                       sbg_mesh *out);
 /* Page-locked host memory, for result arrays: the classification entry
- * points copy their votes straight into page-locked output arrays by DMA
- * (any page-locked memory qualifies; other memory gets a staged copy).  No
- * counterpart in the reference. */
+ * points' last kernel writes the votes straight into page-locked output
+ * arrays (memory that kernels reach only at another address gets them by DMA,
+ * other memory a staged copy).  No counterpart in the reference. */
 int sbg_host_alloc(size_t bytes, void **out);
 int sbg_host_free(void *p);
 /* Device SolidMesh::prepare (src/solidmesh.cpp:42-76): FP64 normals
@@ -247,7 +247,9 @@ int sbg_calibrate_copy(sbg_context ctx, size_t bytes, int iters, double *avg_ms)
  * both meshes over a coordinate search of the knobs and leaves the fastest
  * set (it re-prepares both meshes). */
 typedef struct sbg_tuning {
-    int bfs_levels;   /* breadth-first levels before the persistent depth-first search (0..64) */
+    int bfs_levels;   /* at most this many breadth-first levels, in one workgroup, before the
+                         persistent depth-first search (0..64); fewer where a level holds more than
+                         2,048 node pairs, as the first one of two large trees does */
     int dfs_waves;    /* one-wave workgroups of the depth-first search (64..16384) */
     int grid_density; /* ray-grid cells per axis plane = triangles * grid_density / 16 (1..64) */
     int depth_first;  /* 0: breadth-first levels only, with a host check every 8 levels */

@@ -93,7 +93,7 @@ constexpr int kRayPinned = kMaxLevels + 8;      // 4 words per classification si
 constexpr int kPinnedWords = kRayPinned + 8;
 constexpr int kExpandGrid = 1024;
 constexpr int kLevelsPerSync = 8;
-// breadth-first levels before the persistent depth-first kernel takes the
+// most breadth-first levels before the persistent depth-first kernel takes the
 // frontier, its wave count, and the initial / largest spill region per wave
 constexpr int kBfsLevels = 24;
 constexpr int kDfsWaves = 512;
@@ -103,7 +103,7 @@ constexpr uint32_t kTopMax = 2048;
 // most pairs of tree tiles whose boxes are tested all against all for the
 // first frontier (larger trees start from their roots)
 constexpr uint64_t kTilePairsMax = (uint64_t)1 << 26;
-// longest run of one first triangle the quick pair sort orders by insertion
+// longest run of one first triangle that the quick pair sorts order
 constexpr uint32_t kSortRunMax = 64;
 constexpr uint32_t kSpillInit = 2048, kSpillMax = 1u << 15;
 // intersecting pairs and segments up to this size leave through page-locked

@@ -326,8 +326,8 @@ class Context:
 
 def host_array(n: int, dtype=np.uint8) -> np.ndarray:
     """A NumPy array of n elements in page-locked host memory (sbg_host_alloc),
-    freed when the array is collected.  Classification results written into
-    such arrays arrive by DMA, without the staged copy other memory gets."""
+    freed when the array is collected.  Classification kernels write their
+    votes straight into such arrays; other memory gets a staged copy."""
     L = load()
     dt = np.dtype(dtype)
     nbytes = max(int(n), 1) * dt.itemsize

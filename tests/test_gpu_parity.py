@@ -325,8 +325,8 @@ def test_nested_shells_many_hits(gpu):
 
 
 def test_votes_into_page_locked_arrays(gpu):
-    """Votes written into page-locked arrays (sbg_host_alloc) arrive by DMA
-    and equal those staged into ordinary arrays, for classify_pair (both
+    """Votes written straight into page-locked arrays (sbg_host_alloc)
+    equal those staged into ordinary arrays, for classify_pair (both
     sides, two calls in a row with the arrays reused) and classify_triangles."""
     a, b = mg.icosphere_pair(5, 2, (0.3, 0.2, -0.1), noise=1e-2, radius_b=0.9)
     A, B = gpu.mesh(a.vertices, a.triangles), gpu.mesh(b.vertices, b.triangles)
@@ -580,11 +580,11 @@ def test_host_pair_list_validation(gpu):
 
 def test_staged_uploads_both_index_widths(gpu):
     """sbg_mesh_create (uint32 indices) and sbg_mesh_create64 (the reference's
-    size_t indices, narrowed while staged) copy through page-locked staging on
-    up to four host threads, each share cycling through two slots: a mesh of
-    1,500,001 random triangles over 800,003 vertices (four shares per array,
-    ragged ends) gives the oracle's normals and boxes bit for bit from both,
-    and so does a one-triangle mesh (one share, one slot)."""
+    size_t indices, narrowed while staged) copy through page-locked staging in
+    1 MB pieces on up to eight host threads: a mesh of 1,500,001 random
+    triangles over 800,003 vertices (37 MB, more than both halves of the
+    staging, ragged ends) gives the oracle's normals and boxes bit for bit
+    from both, and so does a one-triangle mesh (one piece)."""
     from oracle.oracle import prepare
 
     rng = np.random.default_rng(11)
